@@ -243,22 +243,15 @@ extern "C"
      * change, only speed); used by the autotuner. */
     enum isaac_hip_tuning_key
     {
-        ISAAC_HIP_TUNE_MARCH_PREFETCH = 0, /* 1: fetch step i+1 before compositing step i (default 0) */
-        ISAAC_HIP_TUNE_MARCH_WAVES = 1, /* march occupancy target: 0 (compiler default), 6 or 8 waves per SIMD */
+        ISAAC_HIP_TUNE_MARCH_PREFETCH = 0, /* any value; without effect: the march requests every next step ahead */
+        ISAAC_HIP_TUNE_MARCH_WAVES = 1, /* 0, 6 or 8; without effect: the march has one register allocation */
         ISAAC_HIP_TUNE_MARCH_TILES = 2, /* march tile order: 0 one band of tile rows per XCD; 2, 4 (default), 8 or
                                           16: super-tiles of that many 16x16-pixel tiles a side, dealt
                                           round-robin to the XCDs */
-        ISAAC_HIP_TUNE_TEX_LAYOUT = 3, /* texture the combined-form march reads: 0 (default) the linear texture
-                                          (x fastest); 8: a copy in 8^3 bricks with a one-texel apron, built by
-                                          update_buffers after classification; 16: the classification also
-                                          writes the volume RGBA of every texel as four binary16 values, which
-                                          the trilinear march steps over (the iso sums of steps that can reach
-                                          the threshold, hit colours and the nearest sampler read the linear
-                                          texture).  The linear texture stays what isaac_hip_get_texture
-                                          returns; a change needs update_buffers before the next render;
-                                          next-step prefetch applies to layouts 0 and 16 */
-        ISAAC_HIP_TUNE_MARCH_THREADS = 4, /* combined-form march workgroup: 256 (default; 4 waves render one 16x16
-                                            tile) or 64 (one wave per workgroup, one 8x8 quarter of a tile) */
+        ISAAC_HIP_TUNE_TEX_LAYOUT = 3, /* 0, 8 or 16: the march reads one layout (the volume and the iso texture,
+                                          x fastest); a change needs update_buffers before the next render */
+        ISAAC_HIP_TUNE_MARCH_THREADS = 4, /* combined-form march workgroup: 64 (default; one wave per workgroup, one
+                                            8x8 quarter of a tile) or 256 (4 waves render one 16x16 tile) */
         ISAAC_HIP_TUNE_MARCH_OFFSETS = 5, /* combined-form trilinear march loads: 32 (default) a 32-bit byte offset
                                             from the texture's base where the texture spans < 4 GiB (larger ones
                                             always take 64-bit addresses); 64: a 64-bit address per lane */

@@ -301,8 +301,6 @@ extern "C"
             rc = build_frame(c, proj + 16 * size_t(f), mv + 16 * size_t(f), bg, vp, t, b->hF[f], b->hQ[f], b->hP[f]);
             if(rc)
                 return bfail(b, rc, c->err);
-            b->hF[f].waves = 0;
-            b->hF[f].prefetch = 0;
             b->hF[f].waveGroups = 4;
             b->hInvScale[f] = 1.0f / float(c->maxGsScaled);
             // the persistent march stages frame 0's transfer functions for every frame:

@@ -23,10 +23,10 @@ namespace isaac_hip
     // its natural one (none for a scalar source, one `length` for a vector source),
     // evaluated inline in the interpreter's operation order instead of interpreted
     constexpr int kSigNatural = 1000;
-    constexpr int kTexBrick = 8; // side of a texture brick (texture layout 8)
-    constexpr int kTexHalf = 16; // texture layout 16: the march steps over a binary16 copy of the volume RGBA
-    constexpr int kTexBrickRow = kTexBrick + 1, kTexBrickSlice = kTexBrickRow * kTexBrickRow;
-    constexpr int kTexBrickTexels = kTexBrickSlice * kTexBrickRow; // 729
+    // The march tests iso alphas only in iso cells that the classification marked: cells of 8^3
+    // base texels.  (4^3 cells would double the steps of the walk through them, 16^3 ones would
+    // double the steps tested in front of every surface.)
+    constexpr int kIsoCellShift = 3;
 
     enum Op : int32_t
     {
@@ -70,8 +70,11 @@ namespace isaac_hip
         int32_t nLut; // LUTs staged in LDS (0 = read from global)
         uint32_t divX_mul, divX_shift, divXY_mul, divXY_shift;
         const float4* luts; // nsrc * T
-        uint2* tex; // per voxel: combined volume RGBA8 (.x), combined iso RGBA8 (.y)
-        uint2* texH; // or nullptr: per voxel the volume RGBA8 as four binary16 values (see half_texel)
+        uint32_t* vol; // combined volume RGBA8 per voxel
+        uint32_t* iso; // combined iso RGBA8 per voxel, or nullptr where no source has an iso threshold
+        uint8_t* isoCells; // cells a step may read an iso alpha byte >= 128 in get the value isoEpoch
+        int32_t ncx, ncy, ncz;
+        uint8_t isoEpoch;
         int64_t nvox;
         ClassifySource src[kMaxSources];
     };
@@ -95,22 +98,16 @@ namespace isaac_hip
         float scale[3];
         float step;
         int32_t linear;
-        int32_t prefetch; // fetch the next step's taps before compositing the current one
-        int32_t waves; // march occupancy target: 0 compiler default, 6 or 8 waves per SIMD
         int32_t tileOrder; // march tile order: 0 one band of tile rows per XCD, S: SxS-tile super-tiles dealt to the XCDs
         int32_t waveGroups; // combined-form march workgroups: 1 one wave each, else 4 waves (one 16x16 tile)
         // textures
         int32_t X, Y, Z;
-        const uint2* tex; // interleaved combined textures, x fastest
-        // or nullptr: the volume RGBA of the same texels as binary16 values, the alpha's sign
-        // set where the iso alpha byte is >= 128 (half_texel); the trilinear march steps over it
-        const uint2* texH;
-        // the same texels in 8^3 bricks with a one-texel apron on the + side (9^3 texels per
-        // brick, x fastest inside, bricks x fastest; apron and partial bricks hold the
-        // clamped texel), or nullptr: every trilinear sample reads one brick
-        const uint2* texB;
-        uint32_t nbx, nbxy; // bricks per row and per slice of the brick layout
-        int32_t texOff32; // the layout the march reads spans < 4 GiB: its loads take 32-bit byte offsets
+        const uint32_t* vol; // combined volume RGBA8, x fastest
+        const uint32_t* iso; // combined iso RGBA8, same layout
+        const uint8_t* isoCells; // iso cells; those marked isoEpoch may hold an iso alpha byte >= 128
+        int32_t ncx, ncy;
+        uint32_t isoEpoch;
+        int32_t texOff32; // a texture spans < 4 GiB and a slice < 2^24 texels: 32-bit byte offsets
         int32_t isoEnabled;
         int32_t volumeEnabled;
         float minSize;
@@ -288,19 +285,6 @@ namespace isaac_hip
     {
         const float x = __builtin_amdgcn_fmed3f(v, 0.0f, 1.0f) * 255.0f;
         return (uint32_t) (x + 0x1.fffffep-2f);
-    }
-
-    // The march texel of texture layout 16: the volume RGBA8 bytes as binary16 values
-    // (every integer 0..255 is exact there), so a trilinear sum takes each one straight into
-    // an fma with mixed operand formats, and the sign of the alpha set where the iso alpha
-    // byte is >= 128 (the only steps where the iso alpha can reach 0.5; the march reads
-    // the alpha through its magnitude).  .x = (r, g), .y = (b, a) with the first in the low half.
-    __device__ inline uint2 half_texel(uint32_t vol, uint32_t iso)
-    {
-        auto h = [](uint32_t b) { return uint32_t(__half_as_ushort(__float2half_rn(float(b)))); };
-        const uint32_t flag = (iso >> 31) << 15;
-        return make_uint2(h(vol & 0xffu) | (h((vol >> 8) & 0xffu) << 16),
-                          h((vol >> 16) & 0xffu) | ((h(vol >> 24) | flag) << 16));
     }
 
     // transfer-function index of x = value * T: roundf(x), NaN -> 0, clamped to

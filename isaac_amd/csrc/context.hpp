@@ -90,11 +90,19 @@ struct isaac_hip_ctx
     int64_t gsScaled[3], lsScaled[3], maxGsScaled;
     int32_t posScaled[3];
     // device buffers
-    uint2* tex = nullptr; // per voxel: combined volume RGBA8, combined iso RGBA8
+    // combined textures, one word per voxel (x fastest) and one word of padding each; texVol is the
+    // allocation that holds both and the iso cells
+    uint32_t* texVol = nullptr; // volume RGBA8
+    uint32_t* texIso = nullptr; // iso RGBA8
     size_t texVox = 0;
-    uint2* texBricks = nullptr; // the same texels in 8^3 bricks with a +1 apron (texture layout 8)
-    uint2* texH = nullptr; // the volume RGBA as binary16 per texel (texture layout 16), texVox + 1 texels
-    size_t texBrickCount = 0;
+    bool isoWritten = false; // texIso holds the last classification's iso texels (else that had no iso source)
+    // iso cells (kIsoCellShift): marked with isoEpoch by the last classification; isoEpoch is the
+    // classification's number, 1..255 in turn, so only its wrap clears the marks
+    uint8_t* isoCells = nullptr;
+    size_t isoCellCount = 0;
+    uint8_t isoEpoch = 0;
+    // both texels of a voxel side by side, kept up to date once a caller asked for it
+    uint2* texBoth = nullptr;
     uint32_t* color = nullptr;
     float* depth = nullptr;
     float* normal = nullptr;
@@ -103,13 +111,11 @@ struct isaac_hip_ctx
     unsigned long long* counters = nullptr;
     bool counting = false;
     bool classified = false;
-    int tunePrefetch = 0;
-    int tuneWaves = 0;
     int tuneTiles = 4; // super-tiles of 4x4 tiles (measured fastest at 1080p)
-    int tuneTexLayout = 0; // march texture: 0 linear (x fastest), 8 bricks of 8^3 texels, 16 linear binary16 copy
-    int tuneMarchThreads = 256; // combined-form march workgroup: 256 (4 waves, one tile) or 64 (one wave)
+    int tuneTexLayout = 0; // accepted values 0, 8 and 16; the march reads one layout
+    int tuneMarchThreads = 64; // combined-form march workgroup: 256 (4 waves, one tile) or 64 (one wave)
     int tuneMarchOffsets = 32; // combined-form march loads: 32-bit byte offsets where the texture allows, or 64-bit addresses
-    int builtTexLayout = -1; // layout whose texels the last combined-form update_buffers wrote
+    int builtTexLayout = -1; // tuneTexLayout at the last combined-form update_buffers
     int form = ISAAC_HIP_FORM_COMBINED;
     int brickDtype = ISAAC_HIP_F32;
     int builtForm = -1; // form prepared by the last update_buffers

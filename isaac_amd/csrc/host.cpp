@@ -324,20 +324,51 @@ namespace
         dst = v;
     }
 
+    int iso_cells(const isaac_hip_ctx* c, int axis)
+    {
+        return int((c->local[axis] + (1 << kIsoCellShift) - 1) >> kIsoCellShift);
+    }
+
+    // a new number for the marks of the iso cells, none of which carries it yet
+    int next_iso_epoch(isaac_hip_ctx* c)
+    {
+        if(c->isoEpoch == 255)
+        {
+            HIPCHK(c, launch_fill_u32(reinterpret_cast<uint32_t*>(c->isoCells), 0u, (c->isoCellCount + 3) / 4, c->stream));
+            c->isoEpoch = 0;
+        }
+        c->isoEpoch++;
+        return 0;
+    }
+
     int alloc_textures(isaac_hip_ctx* c)
     {
         const size_t nvox = size_t(c->local[0]) * size_t(c->local[1]) * size_t(c->local[2]);
-        if(c->tex)
-            (void) hipFree(c->tex);
-        c->tex = nullptr;
-        if(c->texH)
-            (void) hipFree(c->texH);
-        c->texH = nullptr;
-        // one texel of padding: the march reads texels x and x+1 with one 16-byte load,
-        // also at the last texel (whose x+1 it then ignores)
+        for(void* b : {(void*) c->texVol, (void*) c->texBoth})
+            if(b)
+                (void) hipFree(b);
+        const bool wanted = c->texBoth != nullptr;
+        c->texVol = c->texIso = nullptr;
+        c->texBoth = nullptr;
+        c->isoCells = nullptr;
         c->generation++;
-        HIPCHK(c, hipMalloc(&c->tex, (nvox + 1) * 8));
-        HIPCHK(c, hipMemsetAsync(c->tex, 0, (nvox + 1) * 8, c->stream));
+        // one allocation for both textures and the iso cells, each on a 256-byte boundary.  One
+        // texel of padding: the march reads texels x and x+1 with one 8-byte load, also at the
+        // last texel (whose x+1 it then ignores)
+        const size_t texBytes = ((nvox + 1) * 4 + 255) / 256 * 256;
+        c->isoCellCount = size_t(iso_cells(c, 0)) * size_t(iso_cells(c, 1)) * size_t(iso_cells(c, 2));
+        const size_t bytes = 2 * texBytes + (c->isoCellCount + 3) / 4 * 4;
+        HIPCHK(c, hipMalloc(&c->texVol, bytes));
+        HIPCHK(c, hipMemsetAsync(c->texVol, 0, bytes, c->stream));
+        c->texIso = c->texVol + texBytes / 4;
+        c->isoCells = reinterpret_cast<uint8_t*>(c->texVol + 2 * (texBytes / 4));
+        c->isoEpoch = 0;
+        c->isoWritten = true;
+        if(wanted)
+        {
+            HIPCHK(c, hipMalloc(&c->texBoth, nvox * sizeof(uint2)));
+            HIPCHK(c, hipMemsetAsync(c->texBoth, 0, nvox * sizeof(uint2), c->stream));
+        }
         c->texVox = nvox;
         c->classified = false;
         return 0;
@@ -581,27 +612,20 @@ namespace isaac_hip
             }
         F.step = c->step;
         F.linear = c->interpolation ? 1 : 0;
-        F.prefetch = c->tunePrefetch;
-        F.waves = c->tuneWaves;
         F.tileOrder = c->tuneTiles;
         F.waveGroups = (c->form == ISAAC_HIP_FORM_COMBINED && c->tuneMarchThreads == 64) ? 1 : 4;
         F.X = int32_t(c->local[0]);
         F.Y = int32_t(c->local[1]);
         F.Z = int32_t(c->local[2]);
-        F.tex = c->tex;
-        if(c->builtTexLayout == kTexHalf && c->texH)
-            F.texH = c->texH;
-        if(c->builtTexLayout == kTexBrick && c->texBricks)
+        F.vol = c->texVol;
+        F.iso = c->texIso;
+        F.isoCells = c->isoCells;
+        F.ncx = iso_cells(c, 0);
+        F.ncy = iso_cells(c, 1);
+        F.isoEpoch = c->isoEpoch;
         {
-            F.texB = c->texBricks;
-            F.nbx = uint32_t((c->local[0] + kTexBrick - 1) / kTexBrick);
-            F.nbxy = F.nbx * uint32_t((c->local[1] + kTexBrick - 1) / kTexBrick);
-        }
-        {
-            // bytes of the layout the march reads, its padding texel included
-            const uint64_t texels = F.texB ? uint64_t(c->texBrickCount) * kTexBrickTexels
-                                           : uint64_t(c->local[0]) * c->local[1] * c->local[2];
-            F.texOff32 = (c->tuneMarchOffsets == 32 && (texels + 1) * sizeof(uint2) <= 0xffffffffull) ? 1 : 0;
+            const uint64_t slice = uint64_t(c->local[0]) * uint64_t(c->local[1]), texels = slice * uint64_t(c->local[2]) + 1;
+            F.texOff32 = (c->tuneMarchOffsets == 32 && texels * 4 <= 0xffffffffull && slice < (1ull << 24)) ? 1 : 0;
         }
         const int nvf = c->nv + c->nf;
         F.isoEnabled = 0;
@@ -954,7 +978,7 @@ extern "C"
         for(auto& p : c->parts)
             free_part(p);
         aonet_destroy(c);
-        void* bufs[] = {c->lutDev,   c->tex,        c->texBricks, c->texH,     c->color,    c->depth,
+        void* bufs[] = {c->lutDev,   c->texVol,     c->texBoth,   c->color,    c->depth,
                         c->normal,   c->ao,         c->volColor,  c->counters, c->outFloat,
                         c->mmPartials, c->mmResult, c->noise,     c->noiseTmp};
         for(void* b : bufs)
@@ -1445,17 +1469,19 @@ extern "C"
         make_fastdiv(uint32_t(P.X), P.divX_mul, P.divX_shift);
         make_fastdiv(uint32_t(P.X * P.Y), P.divXY_mul, P.divXY_shift);
         P.luts = c->lutDev;
-        P.tex = c->tex;
-        if(c->tuneTexLayout == kTexHalf)
-        {
-            if(!c->texH)
-            {
-                // one padding texel, as for the combined texture
-                HIPCHK(c, hipMalloc(&c->texH, (c->texVox + 1) * sizeof(uint2)));
-                HIPCHK(c, hipMemsetAsync(c->texH + c->texVox, 0, sizeof(uint2), c->stream));
-            }
-            P.texH = c->texH;
-        }
+        P.vol = c->texVol;
+        // without an iso source every iso texel is 0 and no iso cell is marked: the texture is not written
+        c->isoWritten = false;
+        for(int s = 0; s < nvf; s++)
+            c->isoWritten = c->isoWritten || c->iso[s] > 0.0f;
+        P.iso = c->isoWritten ? c->texIso : nullptr;
+        if(int rc = next_iso_epoch(c))
+            return rc;
+        P.isoCells = c->isoCells;
+        P.isoEpoch = c->isoEpoch;
+        P.ncx = iso_cells(c, 0);
+        P.ncy = iso_cells(c, 1);
+        P.ncz = iso_cells(c, 2);
         const int maxLds = int((64 * 1024) / (size_t(T) * sizeof(float4)));
         P.nLut = std::min(nvf, std::max(0, maxLds));
         for(int s = 0; s < nvf; s++)
@@ -1498,23 +1524,8 @@ extern "C"
             S.adv = (s >= c->nv && S.active) ? v.adv[v.advCur] : nullptr;
         }
         HIPCHK(c, launch_classify(P, c->stream));
-        if(c->tuneTexLayout == kTexBrick)
-        {
-            const size_t nb = size_t((c->local[0] + kTexBrick - 1) / kTexBrick) * size_t((c->local[1] + kTexBrick - 1) / kTexBrick)
-                * size_t((c->local[2] + kTexBrick - 1) / kTexBrick);
-            if(nb != c->texBrickCount)
-            {
-                if(c->texBricks)
-                    HIPCHK(c, hipFree(c->texBricks));
-                c->texBricks = nullptr;
-                c->texBrickCount = 0;
-                // one padding texel: the last brick's last row is read 16 bytes at a time too
-                HIPCHK(c, hipMalloc(&c->texBricks, (nb * kTexBrickTexels + 1) * sizeof(uint2)));
-                HIPCHK(c, hipMemsetAsync(c->texBricks + nb * kTexBrickTexels, 0, sizeof(uint2), c->stream));
-                c->texBrickCount = nb;
-            }
-            HIPCHK(c, launch_tex_bricks(c->tex, c->texBricks, int(c->local[0]), int(c->local[1]), int(c->local[2]), c->stream));
-        }
+        if(c->texBoth)
+            HIPCHK(c, launch_interleave(c->texVol, P.iso, c->texBoth, P.nvox, c->stream));
         // the particle records after the classification, so the host enqueues their short
         // launches while the classification runs
         HIPCHK(c, mark(c, 2));
@@ -1546,6 +1557,18 @@ extern "C"
             return fail(c, ISAAC_HIP_ERR_STATE, "render form changed; call isaac_hip_update_buffers");
         if(c->form == ISAAC_HIP_FORM_COMBINED && c->builtTexLayout != c->tuneTexLayout)
             return fail(c, ISAAC_HIP_ERR_STATE, "texture layout changed; call isaac_hip_update_buffers");
+        if(c->form == ISAAC_HIP_FORM_COMBINED && !c->isoWritten)
+        {
+            // a threshold set after a classification without one: its iso texels are 0
+            bool on = false;
+            for(int s = 0; s < c->nv + c->nf; s++)
+                on = on || c->iso[s] > 0.0f;
+            if(on)
+            {
+                HIPCHK(c, launch_fill_u32(c->texIso, 0u, c->texVox, c->stream));
+                c->isoWritten = true;
+            }
+        }
         const int W = c->cfg.framebuffer_size[0], H = c->cfg.framebuffer_size[1];
         FrameTargets tg{W, H, c->color, c->depth, c->normal, c->ao, c->volColor, c->floatOut ? c->outFloat : nullptr, c->counters};
         FrameParams F;
@@ -1684,13 +1707,11 @@ extern "C"
             return ISAAC_HIP_ERR_ARG;
         switch(key)
         {
-        case ISAAC_HIP_TUNE_MARCH_PREFETCH:
-            c->tunePrefetch = value != 0;
+        case ISAAC_HIP_TUNE_MARCH_PREFETCH: // (the march requests every next step ahead)
             return 0;
         case ISAAC_HIP_TUNE_MARCH_WAVES:
             if(value != 0 && value != 6 && value != 8)
                 return fail(c, ISAAC_HIP_ERR_ARG, "march waves: 0, 6 or 8");
-            c->tuneWaves = value;
             return 0;
         case ISAAC_HIP_TUNE_MARCH_TILES:
             if(value != 0 && value != 2 && value != 4 && value != 8 && value != 16)
@@ -1716,8 +1737,8 @@ extern "C"
             c->tuneMarchOffsets = value;
             return 0;
         case ISAAC_HIP_TUNE_TEX_LAYOUT:
-            if(value != 0 && value != kTexBrick && value != kTexHalf)
-                return fail(c, ISAAC_HIP_ERR_ARG, "texture layout: 0 (linear), 8 (8^3 bricks) or 16 (binary16 copy)");
+            if(value != 0 && value != 8 && value != 16)
+                return fail(c, ISAAC_HIP_ERR_ARG, "texture layout: 0, 8 or 16");
             c->tuneTexLayout = value;
             return 0;
         default:
@@ -1821,10 +1842,20 @@ extern "C"
     {
         if(!c)
             return ISAAC_HIP_ERR_ARG;
-        if(texels)
-            *texels = c->tex;
         if(texel_bytes)
             *texel_bytes = 8;
+        if(!texels)
+            return 0;
+        // built by the first request, and by every update after it
+        isaac_hip_ctx* m = const_cast<isaac_hip_ctx*>(c);
+        if(!m->texBoth)
+        {
+            HIPCHK(m, hipSetDevice(m->device));
+            HIPCHK(m, hipMalloc(&m->texBoth, m->texVox * sizeof(uint2)));
+            HIPCHK(m, launch_interleave(m->texVol, m->isoWritten ? m->texIso : nullptr, m->texBoth, int64_t(m->texVox), m->stream));
+            HIPCHK(m, hipStreamSynchronize(m->stream));
+        }
+        *texels = m->texBoth;
         return 0;
     }
 

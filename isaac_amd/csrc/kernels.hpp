@@ -20,7 +20,8 @@ namespace isaac_hip
     // the fused march (clear, particles, iso + volume), the SSAO pass and shading
     // + volume blend; the host records its per-kernel events between them
     hipError_t launch_march(const FrameParams& F, const ParticleParams& PP, bool counting, hipStream_t s);
-    hipError_t launch_tex_bricks(const uint2* tex, uint2* out, int X, int Y, int Z, hipStream_t s);
+    // vol and iso (nullptr: zeros) side by side, n voxels
+    hipError_t launch_interleave(const uint32_t* vol, const uint32_t* iso, uint2* out, int64_t n, hipStream_t s);
     // shade: the occlusion kernel also shades its pixels (only where ssao_shades(F))
     hipError_t launch_ssao(const FrameParams& F, hipStream_t s, bool shade = false);
     bool ssao_shades(const FrameParams& F);

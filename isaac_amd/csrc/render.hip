@@ -1,10 +1,6 @@
-// gfx950 kernels of the per-rank render path.
+// gfx950 kernels of the per-rank render path (the combined form's march: march.hip).
 //
 //   classify_kernel        MergeToCombinedTextureKernel  lib/isaac/isaac_common_kernel.hpp:553-615,690-758
-//   march_kernel           ClearBufferKernel + ParticleRenderKernel + CombinedIsoRenderKernel +
-//                          the march of CombinedVolumeRenderKernel, fused per pixel
-//                          lib/isaac/isaac_common_kernel.hpp:195-217, lib/isaac/isaac_particle_kernel.hpp:117-260,
-//                          lib/isaac/isaac_iso_kernel.hpp:25-128, lib/isaac/isaac_volume_kernel.hpp:23-82
 //   ssao_tiled_kernel      SSAOKernel (live 7x7 part)     lib/isaac/isaac_ssao_kernel.hpp:161-182
 //                          (with the shading of its pixels fused in render modes 0, 1, 3)
 //   shade_kernel           ShadingKernel + the volume pass's final blend
@@ -18,7 +14,7 @@
 // tile (16x16 pixels per workgroup), so the 64 rays of a wave sample
 // neighbouring voxels; the march deals its tiles to the 8 XCDs (each with its
 // own L2) in super-tiles or bands (march_tile), and can run one-wave workgroups.
-#include "kernels.hpp"
+#include "render_device.hpp"
 
 namespace isaac_hip
 {
@@ -140,6 +136,22 @@ namespace isaac_hip
         return q(r) | (q(g) << 8) | (q(b) << 16) | (q(a) << 24);
     }
 
+    // Marks the iso cells whose steps may read one of the voxels x0..x1 of row (y, z), which
+    // holds an iso alpha byte >= 128 (ClassifyParams::isoCells).  Cell c serves the base texels
+    // 8c..8c+7 with their + neighbours, and one voxel more on each side for the rounding of the
+    // march's cell exits: voxels 8c-1..8c+9.  Every writer stores the same value, so plain
+    // stores do; the value is the update's number, so nothing is cleared between updates.
+    __device__ inline void mark_iso_cells(const ClassifyParams& P, int x0, int x1, int y, int z)
+    {
+        const int cx0 = max(0, (x0 - 2) >> kIsoCellShift), cx1 = min(P.ncx - 1, (x1 + 1) >> kIsoCellShift);
+        const int cy0 = max(0, (y - 2) >> kIsoCellShift), cy1 = min(P.ncy - 1, (y + 1) >> kIsoCellShift);
+        const int cz0 = max(0, (z - 2) >> kIsoCellShift), cz1 = min(P.ncz - 1, (z + 1) >> kIsoCellShift);
+        for(int cz = cz0; cz <= cz1; cz++)
+            for(int cy = cy0; cy <= cy1; cy++)
+                for(int cx = cx0; cx <= cx1; cx++)
+                    P.isoCells[(size_t(cz) * size_t(P.ncy) + size_t(cy)) * size_t(P.ncx) + size_t(cx)] = P.isoEpoch;
+    }
+
     // One workgroup stages up to nLut transfer functions (T float4 each) in LDS
     // and then walks voxels with a grid-stride loop (x fastest, coalesced
     // source reads and texel writes).
@@ -211,11 +223,13 @@ namespace isaac_hip
             }
             const uint32_t vol = dither_b4(P.ditherMode, x, y, z, vr, vg, vb, va);
             const uint32_t q0 = unorm8(ir), q1 = unorm8(ig), q2 = unorm8(ib), q3 = unorm8(ia);
-            // one 8-byte texel per voxel: combined volume RGBA8, combined iso RGBA8
-            const uint32_t iso = q0 | (q1 << 8) | (q2 << 16) | (q3 << 24);
-            P.tex[idx] = make_uint2(vol, iso);
-            if(P.texH)
-                P.texH[idx] = half_texel(vol, iso);
+            P.vol[idx] = vol;
+            if(P.iso)
+            {
+                P.iso[idx] = q0 | (q1 << 8) | (q2 << 16) | (q3 << 24);
+                if(q3 >= 128u)
+                    mark_iso_cells(P, x, x, y, z);
+            }
         }
     }
 
@@ -243,912 +257,6 @@ namespace isaac_hip
             float c0 = e[0], c1 = dim > 1 ? e[1] : 0.f, c2 = dim > 2 ? e[2] : 0.f, c3 = dim > 3 ? e[3] : 0.f;
             dst[i] = apply_chain(chain, c0, c1, c2, c3, dim);
         }
-    }
-
-    // ------------------------------------------------------------------ rays
-    struct Ray
-    {
-        F3 dir, start;
-        float startDepth, endDepth;
-        bool isClipped;
-        F3 clipN;
-    };
-
-    // pixelToRay (lib/isaac/isaac_common_kernel.hpp:51-92); glm mat4*vec4 = (m0*x+m1*y)+(m2*z+m3*w)
-    __device__ inline Ray pixel_to_ray(const FrameParams& F, int px, int py)
-    {
-        const float vx = float(px) / F.fbW * 2.0f - 1.0f;
-        const float vy = float(py) / F.fbH * 2.0f - 1.0f;
-        float s[4], e[4];
-#pragma unroll
-        for(int r = 0; r < 4; r++)
-        {
-            const float a0 = F.inv[0 * 4 + r] * vx;
-            const float a1 = F.inv[1 * 4 + r] * vy;
-            const float s0 = a0 + a1;
-            const float bs = F.inv[2 * 4 + r] * -1.0f;
-            const float be = F.inv[2 * 4 + r] * 1.0f;
-            const float a3 = F.inv[3 * 4 + r] * 1.0f;
-            s[r] = s0 + (bs + a3);
-            e[r] = s0 + (be + a3);
-        }
-        Ray ray;
-        F3 st = f3(s[0] / s[3], s[1] / s[3], s[2] / s[3]);
-        F3 en = f3(e[0] / e[3], e[1] / e[3], e[2] / e[3]);
-        st = muls(st, F.maxSize);
-        en = muls(en, F.maxSize);
-        ray.dir = normalize3(sub(en, st));
-        ray.start = st;
-        ray.isClipped = false;
-        ray.clipN = f3(0.f, 0.f, 0.f);
-        ray.startDepth = 0.f;
-        ray.endDepth = 0.f;
-        return ray;
-    }
-
-    // clipRay (lib/isaac/isaac_common_kernel.hpp:94-193)
-    __device__ inline bool clip_ray(const FrameParams& F, Ray& ray)
-    {
-        ray.start = add(ray.start, f3(F.off[0], F.off[1], F.off[2]));
-        float bmin[3], bmax[3];
-        const float st[3] = {ray.start.x, ray.start.y, ray.start.z};
-        const float dr[3] = {ray.dir.x, ray.dir.y, ray.dir.z};
-#pragma unroll
-        for(int i = 0; i < 3; i++)
-        {
-            bmin[i] = (F.bbMin[i] - st[i]) / dr[i];
-            bmax[i] = (F.bbMax[i] - st[i]) / dr[i];
-            if(bmax[i] < bmin[i])
-            {
-                float t = bmax[i];
-                bmax[i] = bmin[i];
-                bmin[i] = t;
-            }
-        }
-        ray.startDepth = gmax(bmin[0], gmax(bmin[1], bmin[2]));
-        ray.endDepth = gmin(bmax[0], gmin(bmax[1], bmax[2]));
-        float cn[3] = {0.f, 0.f, 0.f};
-#pragma unroll
-        for(int i = 0; i < 3; i++)
-        {
-            const float sgn = gsign(dr[i]);
-            const bool lowOuter = F.outerLow[i] && (sgn + 1.0f) != 0.0f;
-            const bool highOuter = F.outerHigh[i] && (sgn - 1.0f) != 0.0f;
-            if(bmin[i] == ray.startDepth && (lowOuter || highOuter))
-            {
-                ray.isClipped = true;
-                cn[i] = sgn;
-            }
-        }
-        ray.clipN = f3(cn[0], cn[1], cn[2]);
-        for(int i = 0; i < F.nclip; i++)
-        {
-            const F3 n = f3(F.cnorm[i][0], F.cnorm[i][1], F.cnorm[i][2]);
-            const F3 p = f3(F.cpos[i][0], F.cpos[i][1], F.cpos[i][2]);
-            const float d = dot3(ray.dir, n);
-            const float depth = (dot3(p, n) - dot3(ray.start, n)) / d;
-            if(d > 0.0f)
-            {
-                if(ray.endDepth < depth)
-                    return false;
-                if(ray.startDepth <= depth)
-                {
-                    ray.clipN = n;
-                    ray.isClipped = true;
-                    ray.startDepth = depth;
-                }
-            }
-            else
-            {
-                if(ray.startDepth > depth)
-                    return false;
-                if(ray.endDepth > depth)
-                    ray.endDepth = depth;
-            }
-        }
-        ray.startDepth = gmax(ray.startDepth, kZNear);
-        if(ray.startDepth > ray.endDepth || isinf(ray.startDepth) || isinf(ray.endDepth))
-            return false;
-        return true;
-    }
-
-    // ------------------------------------------------------------------ texture sampling
-    // x / 255 in binary32 as x*r plus one fma residual correction, r = RN(1/255).
-    // For every float x in [0, 256] this equals the IEEE quotient bit for bit
-    // (tests/test_div255.py checks all 1,132,462,081 inputs); trilinear results
-    // of RGBA8 texels always lie in [0, 255].  Three instructions instead of the
-    // correctly rounded division sequence.
-    __device__ inline float div255(float x)
-    {
-        const float r = 1.0f / 255.0f;
-        const float q0 = x * r;
-        const float e = __builtin_fmaf(-q0, 255.0f, x);
-        return __builtin_fmaf(e, r, q0);
-    }
-
-    // The 8 trilinear taps of one sample position (or the single NEAREST tap),
-    // each an 8-byte texel: .x combined volume RGBA8, .y combined iso RGBA8.
-    // Tap k holds voxel (x0 + (k>>2), y0 + ((k>>1)&1), z0 + (k&1)), clamped.
-    struct Taps
-    {
-        uint2 t[8];
-        float fx, fy, fz;
-    };
-
-    // two adjacent texels (8-byte aligned; one 16-byte load)
-    struct TexPair
-    {
-        uint2 a, b;
-    };
-
-    // index of texel (x, y, z) in the brick layout (FrameParams::texB)
-    __device__ inline uint32_t brick_texel(const FrameParams& F, uint32_t x, uint32_t y, uint32_t z)
-    {
-        const uint32_t b = (z >> 3) * F.nbxy + (y >> 3) * F.nbx + (x >> 3);
-        return b * uint32_t(kTexBrickTexels) + (z & 7u) * uint32_t(kTexBrickSlice) + (y & 7u) * uint32_t(kTexBrickRow)
-            + (x & 7u);
-    }
-
-    // Sampler<LINEAR|NEAREST, CLAMP> addressing (lib/isaac/isaac_texture.hpp:182-259).  Every
-    // coordinate is clamped into the texture, so a fetch at any position is in bounds.
-    // BRICK reads the brick layout (texels x and x + 1 of a row stay adjacent there:
-    // x & 7 = 7 is followed by the apron texel).
-    template<bool LINEAR, bool BRICK>
-    __device__ inline void fetch_taps(const FrameParams& F, float px, float py, float pz, Taps& T)
-    {
-        const uint2* __restrict__ tex = BRICK ? F.texB : F.tex;
-        const int X = F.X, Y = F.Y, Z = F.Z;
-        auto index = [&](uint32_t x, uint32_t y, uint32_t z)
-        { return BRICK ? brick_texel(F, x, y, z) : x + uint32_t(X) * (y + uint32_t(Y) * z); };
-        if(!LINEAR)
-        {
-            const uint32_t x = iclamp(int(px), 0, X - 1), y = iclamp(int(py), 0, Y - 1), z = iclamp(int(pz), 0, Z - 1);
-            T.t[0] = tex[index(x, y, z)];
-            T.fx = T.fy = T.fz = 0.0f;
-            return;
-        }
-        const float cx = px - 0.5f, cy = py - 0.5f, cz = pz - 0.5f;
-        const float flx = floorf(cx), fly = floorf(cy), flz = floorf(cz);
-        T.fx = cx - flx;
-        T.fy = cy - fly;
-        T.fz = cz - flz;
-        const int bx = int(flx), by = int(fly), bz = int(flz);
-        const uint32_t x0 = iclamp(bx, 0, X - 1), x1 = iclamp(bx + 1, 0, X - 1);
-        const uint32_t y0 = iclamp(by, 0, Y - 1), y1 = iclamp(by + 1, 0, Y - 1);
-        const uint32_t z0 = iclamp(bz, 0, Z - 1), z1 = iclamp(bz + 1, 0, Z - 1);
-        // texels x0 and x0+1 are adjacent: one 16-byte load per (y, z) row; at the
-        // x edge (x1 == x0) the second texel (the next row's first, the padding
-        // texel after the last, or an apron texel) is replaced by the first
-        const TexPair p00 = *reinterpret_cast<const TexPair*>(tex + index(x0, y0, z0));
-        const TexPair p01 = *reinterpret_cast<const TexPair*>(tex + index(x0, y0, z1));
-        const TexPair p10 = *reinterpret_cast<const TexPair*>(tex + index(x0, y1, z0));
-        const TexPair p11 = *reinterpret_cast<const TexPair*>(tex + index(x0, y1, z1));
-        const bool dup = x1 == x0;
-        T.t[0] = p00.a;
-        T.t[1] = p01.a;
-        T.t[2] = p10.a;
-        T.t[3] = p11.a;
-        T.t[4] = dup ? p00.a : p00.b;
-        T.t[5] = dup ? p01.a : p01.b;
-        T.t[6] = dup ? p10.a : p10.b;
-        T.t[7] = dup ? p11.a : p11.b;
-    }
-
-    // one normalised channel: trilinear of the bytes (z innermost, x outermost,
-    // lib/isaac/isaac_helper.hpp:124-144), then / 255
-    template<bool LINEAR, bool ISO>
-    __device__ inline float channel(const Taps& T, int sh)
-    {
-        auto d = [&](int k) { return float(((ISO ? T.t[k].y : T.t[k].x) >> sh) & 0xffu); };
-        if(!LINEAR)
-            return div255(d(0));
-        const float oz = 1.0f - T.fz, oy = 1.0f - T.fy, ox = 1.0f - T.fx;
-        const float a0 = d(0) * oz + d(1) * T.fz, a1 = d(2) * oz + d(3) * T.fz;
-        const float A = a0 * oy + a1 * T.fy;
-        const float b0 = d(4) * oz + d(5) * T.fz, b1 = d(6) * oz + d(7) * T.fz;
-        const float B = b0 * oy + b1 * T.fy;
-        return div255(A * ox + B * T.fx);
-    }
-
-    // bitwise OR of the taps' volume (.x) or iso (.y) texels
-    template<bool LINEAR, bool ISO>
-    __device__ inline uint32_t taps_or(const Taps& T)
-    {
-        uint32_t o = ISO ? T.t[0].y : T.t[0].x;
-        if(LINEAR)
-        {
-#pragma unroll
-            for(int k = 1; k < 8; k++)
-                o |= ISO ? T.t[k].y : T.t[k].x;
-        }
-        return o;
-    }
-
-    template<bool LINEAR, bool BRICK>
-    __device__ inline float iso_alpha_at(const FrameParams& F, float px, float py, float pz)
-    {
-        Taps T;
-        fetch_taps<LINEAR, BRICK>(F, px, py, pz, T);
-        return channel<LINEAR, true>(T, 24);
-    }
-
-    // ------------------------------------------------------------------ march sampling
-    // The march's per-step samples weigh the eight texels once per position: each
-    // channel is sum_k byte_k * w_k (one multiply and seven fmas) with the corner
-    // weights w_k = wx * wy * wz, instead of seven lerps per channel, and at the x
-    // edge (both x taps on texel x0, CLAMP) the first texel takes weight 1 instead of
-    // the texels being swapped.  In exact arithmetic this is the reference's trilinear
-    // (lib/isaac/isaac_helper.hpp:124-144); in binary32 the result differs from its
-    // nested lerps by rounding only.  Texel indices are 32-bit; rows y+1 and z+1
-    // are the row of y and z plus a stride or plus 0 at a clamped edge.
-    struct Corners
-    {
-        uint2 t[8]; // k = 4 x + 2 y + z (x outermost, as the reference's lerps nest)
-        float w[8];
-    };
-
-    // the corners of the sample at c: for LINEAR the position minus 0.5 (the texel
-    // centres' offset), for NEAREST the position itself; BRICK reads the brick layout
-    // OFF32: the texture spans < 4 GiB, so the loads take a 32-bit byte offset from the
-    // texture's (uniform) base address instead of a 64-bit address per lane.  HALF reads
-    // the binary16 copy of the linear layout (same texel indices) instead.
-    template<bool LINEAR, bool BRICK, bool OFF32 = false, bool HALF = false>
-    __device__ inline void fetch_corners(const FrameParams& F, uint32_t XY, float cx, float cy, float cz, Corners& C)
-    {
-        static_assert(!(HALF && BRICK), "the binary16 copy has the linear layout");
-        const uint2* __restrict__ tex = HALF ? F.texH : (BRICK ? F.texB : F.tex);
-        const int X = F.X, Y = F.Y, Z = F.Z;
-        if(!LINEAR)
-        {
-            const uint32_t x = iclamp(int(cx), 0, X - 1), y = iclamp(int(cy), 0, Y - 1), z = iclamp(int(cz), 0, Z - 1);
-            C.t[0] = tex[BRICK ? brick_texel(F, x, y, z) : x + uint32_t(X) * y + XY * z];
-            return;
-        }
-        const float flx = floorf(cx), fly = floorf(cy), flz = floorf(cz);
-        const int bx = int(flx), by = int(fly), bz = int(flz);
-        // taps x0 and x0 + 1 come from one 16-byte load; where both are x0 (bx < 0 or
-        // bx >= X - 1) the second gets weight 0
-        const bool xin = uint32_t(bx) < uint32_t(X - 1);
-        const float fx = xin ? cx - flx : 0.0f, fy = cy - fly, fz = cz - flz;
-        const uint32_t x0 = iclamp(bx, 0, X - 1), y0 = iclamp(by, 0, Y - 1), z0 = iclamp(bz, 0, Z - 1);
-        // rows y + 1 and z + 1: the next row / slice, or the same one at a clamped edge
-        // (in the brick layout the next row of y & 7 = 7 is the apron row)
-        const uint32_t dy = uint32_t(by) < uint32_t(Y - 1) ? (BRICK ? uint32_t(kTexBrickRow) : uint32_t(X)) : 0u;
-        const uint32_t dz = uint32_t(bz) < uint32_t(Z - 1) ? (BRICK ? uint32_t(kTexBrickSlice) : XY) : 0u;
-        const uint32_t i00 = BRICK ? brick_texel(F, x0, y0, z0) : x0 + __umul24(y0, uint32_t(X)) + z0 * XY;
-        uint4 p00, p01, p10, p11;
-        if constexpr(OFF32)
-        {
-            const char* base = reinterpret_cast<const char*>(tex);
-            const uint32_t o00 = i00 << 3, o01 = o00 + (dz << 3), o10 = o00 + (dy << 3), o11 = o10 + (dz << 3);
-            p00 = *reinterpret_cast<const uint4*>(base + o00);
-            p01 = *reinterpret_cast<const uint4*>(base + o01);
-            p10 = *reinterpret_cast<const uint4*>(base + o10);
-            p11 = *reinterpret_cast<const uint4*>(base + o11);
-        }
-        else
-        {
-            const uint32_t i01 = i00 + dz, i10 = i00 + dy, i11 = i10 + dz;
-            p00 = *reinterpret_cast<const uint4*>(tex + i00);
-            p01 = *reinterpret_cast<const uint4*>(tex + i01);
-            p10 = *reinterpret_cast<const uint4*>(tex + i10);
-            p11 = *reinterpret_cast<const uint4*>(tex + i11);
-        }
-        C.t[0] = make_uint2(p00.x, p00.y);
-        C.t[1] = make_uint2(p01.x, p01.y);
-        C.t[2] = make_uint2(p10.x, p10.y);
-        C.t[3] = make_uint2(p11.x, p11.y);
-        C.t[4] = make_uint2(p00.z, p00.w);
-        C.t[5] = make_uint2(p01.z, p01.w);
-        C.t[6] = make_uint2(p10.z, p10.w);
-        C.t[7] = make_uint2(p11.z, p11.w);
-        const float ox = 1.0f - fx, oy = 1.0f - fy, oz = 1.0f - fz;
-        const float w00 = oy * oz, w01 = oy * fz, w10 = fy * oz, w11 = fy * fz;
-        C.w[0] = ox * w00;
-        C.w[1] = ox * w01;
-        C.w[2] = ox * w10;
-        C.w[3] = ox * w11;
-        C.w[4] = fx * w00;
-        C.w[5] = fx * w01;
-        C.w[6] = fx * w10;
-        C.w[7] = fx * w11;
-    }
-
-    // one channel in byte units (0..255): the volume (.x) or iso (.y) texel's byte at `sh`
-    template<bool LINEAR, bool ISO>
-    __device__ inline float corner_sum(const Corners& C, int sh)
-    {
-        auto d = [&](int k) { return float(((ISO ? C.t[k].y : C.t[k].x) >> sh) & 0xffu); };
-        if(!LINEAR)
-            return d(0);
-        float v = d(0) * C.w[0];
-#pragma unroll
-        for(int k = 1; k < 8; k++)
-            v = __builtin_fmaf(d(k), C.w[k], v);
-        return v;
-    }
-
-    // channel ch (0..3: r, g, b, a) of the volume RGBA from corners of the binary16 copy,
-    // in byte units: the same sum as corner_sum<true, false>(C, 8 * ch) (each binary16 value
-    // is its byte exactly; the first product goes through an fma with +0, which returns the
-    // product itself as both factors are >= +0); the alpha is read through its magnitude
-    template<int CH>
-    __device__ inline float half_sum(const Corners& C)
-    {
-        auto d = [&](int k)
-        {
-            const uint32_t u = CH < 2 ? C.t[k].x : C.t[k].y;
-            const float v = float(__ushort_as_half((unsigned short) ((CH & 1) ? (u >> 16) : (u & 0xffffu))));
-            return CH == 3 ? fabsf(v) : v;
-        };
-        float v = __builtin_fmaf(d(0), C.w[0], 0.0f);
-#pragma unroll
-        for(int k = 1; k < 8; k++)
-            v = __builtin_fmaf(d(k), C.w[k], v);
-        return v;
-    }
-
-    template<bool LINEAR, bool ISO>
-    __device__ inline uint32_t corners_or(const Corners& C)
-    {
-        uint32_t o = ISO ? C.t[0].y : C.t[0].x;
-        if(LINEAR)
-        {
-#pragma unroll
-            for(int k = 1; k < 8; k++)
-                o |= ISO ? C.t[k].y : C.t[k].x;
-        }
-        return o;
-    }
-
-    struct F4
-    {
-        float x, y, z, w;
-    };
-
-    // ------------------------------------------------------------------ pixel tiling
-    // workgroup -> 16x16 tile, XCD-banded; returns false for threads outside the viewport
-    // pixel of this thread in 16x16 tile `b` of the viewport (row-major tiles)
-    // pixel of this lane in 16x16 tile b, whose 8x8 quarter `wave` (0..3) its wave renders
-    __device__ inline bool tile_pixel_at(const FrameParams& F, uint32_t b, uint32_t wave, int& px, int& py)
-    {
-        const uint32_t tx = b % uint32_t(F.tilesX), ty = b / uint32_t(F.tilesX);
-        const uint32_t lane = threadIdx.x & 63u;
-        px = F.vx0 + int(tx * 16u + (wave & 1u) * 8u + (lane & 7u));
-        py = F.vy0 + int(ty * 16u + (wave >> 1) * 8u + (lane >> 3));
-        return b < uint32_t(F.tilesX) * uint32_t(F.tilesY) && px < F.vx1 && py < F.vy1;
-    }
-
-    __device__ inline bool tile_pixel_at(const FrameParams& F, uint32_t b, int& px, int& py)
-    {
-        return tile_pixel_at(F, b, threadIdx.x >> 6, px, py);
-    }
-
-    // The march's workgroups: one 16x16 tile of 4 waves each, or (F.waveGroups == 1)
-    // one wave each: workgroup b is then quarter (b / 8) % 4 of the tile of logical
-    // workgroup (b / 32) * 8 + b % 8, and runs on the XCD b % 8 of that logical
-    // workgroup, so the dealing of tiles to the XCDs is unchanged while the
-    // dispatcher fills any SIMD with a free wave slot.
-    __device__ inline uint32_t march_block(const FrameParams& F)
-    {
-        return F.waveGroups == 1 ? ((blockIdx.x >> 5) << 3) | (blockIdx.x & 7u) : blockIdx.x;
-    }
-    __device__ inline uint32_t march_wave(const FrameParams& F)
-    {
-        return F.waveGroups == 1 ? (blockIdx.x >> 3) & 3u : threadIdx.x >> 6;
-    }
-
-    __device__ inline uint32_t xcd_tile(const FrameParams& F, uint32_t b)
-    {
-        const uint32_t nb = uint32_t(F.tilesX) * uint32_t(F.tilesY);
-        const uint32_t full = nb & ~7u;
-        if(b < full)
-            b = (b & 7u) * (full >> 3) + (b >> 3);
-        return b;
-    }
-
-    // Super-tiles of SxS tiles (S = F.tileOrder: 2, 4, 8 or 16; 4 is 64x64 pixels)
-    // dealt round-robin to the XCDs: workgroup b runs on XCD b % 8 and takes tile
-    // (b / 8) % S^2 of that XCD's super-tile number (b / 8) / S^2.  Every XCD gets
-    // super-tiles from all over the frame (balanced when the work is concentrated,
-    // e.g. a volume in the middle of the frame) while the rays of one super-tile
-    // share its L2.  Grid: march_grid workgroups; padding workgroups map to no tile.
-    __device__ inline uint32_t supertile_tile(const FrameParams& F, uint32_t b)
-    {
-        const uint32_t S = uint32_t(F.tileOrder), sh = uint32_t(__ffs(int(S)) - 1);
-        const uint32_t tX = uint32_t(F.tilesX), tY = uint32_t(F.tilesY);
-        const uint32_t sx = (tX + S - 1u) >> sh, sy = (tY + S - 1u) >> sh;
-        const uint32_t i = b >> 3;
-        const uint32_t s = (b & 7u) + 8u * (i >> (2u * sh)), w = i & (S * S - 1u);
-        if(s >= sx * sy)
-            return 0xffffffffu;
-        const uint32_t tx = ((s % sx) << sh) + (w & (S - 1u)), ty = ((s / sx) << sh) + (w >> sh);
-        if(tx >= tX || ty >= tY)
-            return 0xffffffffu;
-        return ty * tX + tx;
-    }
-
-    __device__ inline uint32_t march_tile(const FrameParams& F)
-    {
-        const uint32_t b = march_block(F);
-        return F.tileOrder != 0 ? supertile_tile(F, b) : xcd_tile(F, b);
-    }
-
-    __device__ inline bool tile_pixel(const FrameParams& F, int& px, int& py)
-    {
-        return tile_pixel_at(F, xcd_tile(F, blockIdx.x), px, py);
-    }
-
-    __device__ inline void block_count_add(unsigned long long* dst, unsigned long long v)
-    {
-        __shared__ unsigned long long red[4];
-        // wave reduction through DPP-free shuffles
-        for(int off = 32; off > 0; off >>= 1)
-            v += __shfl_down(v, off, 64);
-        if((threadIdx.x & 63) == 0)
-            red[threadIdx.x >> 6] = v;
-        __syncthreads();
-        if(threadIdx.x == 0)
-        {
-            unsigned long long s = 0;
-            for(uint32_t w = 0; w < (blockDim.x >> 6); w++)
-                s += red[w];
-            if(s)
-                atomicAdd(dst, s);
-        }
-        __syncthreads();
-    }
-
-    // ------------------------------------------------------------------ particles
-    // ParticleRenderKernel (lib/isaac/isaac_particle_kernel.hpp:117-260): 3D-DDA over
-    // the particle cell grid from the clipped ray start; the first cell holding a
-    // visible sphere hit ends the walk (hit point of the nearest sphere in it).
-    template<bool COUNT>
-    __device__ inline void particle_dda(
-        const ParticleParams& PP,
-        const Ray& ray,
-        uint32_t& color,
-        float& depth,
-        F3& normal,
-        unsigned long long& nCells,
-        unsigned long long& nTests)
-    {
-        const F3 ps = f3(PP.pscale[0], PP.pscale[1], PP.pscale[2]);
-        const int ds[3] = {int(gsign(ray.dir.x)), int(gsign(ray.dir.y)), int(gsign(ray.dir.z))};
-        const F3 cur = add(ray.start, muls(ray.dir, ray.startDepth));
-        const F3 cdiv = divv(cur, ps);
-        uint32_t cell[3];
-        cell[0] = uint32_t(iclamp(int(cdiv.x), 0, PP.grid[0] - 1));
-        cell[1] = uint32_t(iclamp(int(cdiv.y), 0, PP.grid[1] - 1));
-        cell[2] = uint32_t(iclamp(int(cdiv.z), 0, PP.grid[2] - 1));
-        const float rayLength = ray.endDepth - ray.startDepth;
-        float tested = 0.0f;
-        const float curA[3] = {cur.x, cur.y, cur.z};
-        const float dA[3] = {ray.dir.x, ray.dir.y, ray.dir.z};
-        const float psA[3] = {ps.x, ps.y, ps.z};
-        float t[3], dt[3];
-#pragma unroll
-        for(int i = 0; i < 3; i++)
-        {
-            t[i] = ((float(cell[i]) + float(ds[i] > 0 ? ds[i] : 0)) * psA[i] - curA[i]) / dA[i];
-            dt[i] = psA[i] / dA[i] * float(ds[i]);
-            if(dA[i] == 0.0f)
-                t[i] = FLT_MAX;
-        }
-        bool hit = false;
-        float pdepth = FLT_MAX;
-        float4 pcol = make_float4(0.f, 0.f, 0.f, 0.f);
-        F3 pn = f3(0.f, 0.f, 0.f);
-        const uint32_t gx = uint32_t(PP.grid[0]), gy = uint32_t(PP.grid[1]), gz = uint32_t(PP.grid[2]);
-        auto inside = [&](const uint32_t (&c)[3]) { return c[0] < gx && c[1] < gy && c[2] < gz; };
-        auto cell_id = [&](const uint32_t (&c)[3]) { return int(c[0] + gx * (c[1] + gy * c[2])); };
-        // record ranges of the current cell, requested one cell ahead: the walk's next
-        // cell depends on the ray only, so the range of cell i + 1 is in flight while
-        // the spheres of cell i are tested
-        int2 kr[4] = {};
-        if(inside(cell))
-        {
-            const int cid = cell_id(cell);
-#pragma unroll
-            for(int s = 0; s < 4; s++)
-                if(s < PP.nsrc)
-                    kr[s] = PP.src[s].vrange[cid];
-        }
-        while(inside(cell) && !hit && tested <= rayLength)
-        {
-            if(COUNT)
-                nCells++;
-            // the walk's next cell (ties between axes go towards z)
-            uint32_t next[3] = {cell[0], cell[1], cell[2]};
-            float nextTested;
-            const bool ax0 = t[0] < t[1] && t[0] < t[2];
-            const bool ax1 = !ax0 && t[1] < t[0] && t[1] < t[2];
-            if(ax0)
-            {
-                next[0] += uint32_t(ds[0]);
-                nextTested = t[0];
-            }
-            else if(ax1)
-            {
-                next[1] += uint32_t(ds[1]);
-                nextTested = t[1];
-            }
-            else
-            {
-                next[2] += uint32_t(ds[2]);
-                nextTested = t[2];
-            }
-            int2 krn[4] = {};
-            if(inside(next))
-            {
-                const int nid = cell_id(next);
-#pragma unroll
-                for(int s = 0; s < 4; s++)
-                    if(s < PP.nsrc)
-                        krn[s] = PP.src[s].vrange[nid];
-            }
-            const F3 cf = f3(float(cell[0]), float(cell[1]), float(cell[2]));
-#pragma unroll
-            for(int s = 0; s < 4; s++)
-            {
-                if(s >= PP.nsrc)
-                    break;
-                const ParticleSourceDev& S = PP.src[s];
-                for(int k = kr[s].x; k < kr[s].y; k++)
-                {
-                    if(COUNT)
-                        nTests++;
-                    const float4 rec = S.recs[k];
-                    const F3 ppos = mul(add(f3(rec.x, rec.y, rec.z), cf), ps);
-                    const F3 L = sub(ppos, cur);
-                    const float radius = (S.radius ? S.radius[k] : S.constRadius) * S.weight;
-                    const float r2 = radius * radius;
-                    const float tca = dot3(L, ray.dir);
-                    const float d2 = dot3(L, L) - tca * tca;
-                    if(d2 <= r2)
-                    {
-                        const float thc = sqrtf(r2 - d2);
-                        const float t0 = tca - thc;
-                        const float t1 = tca + thc;
-                        if(t1 >= 0.0f && t0 < pdepth)
-                        {
-                            const float4 val = S.lut[__float_as_int(rec.w)];
-                            if(val.w >= 0.5f)
-                            {
-                                pcol = val;
-                                pdepth = t0;
-                                hit = true;
-                                pn = sub(add(cur, muls(ray.dir, t0)), ppos);
-                                if(t0 < 0.0f && ray.isClipped)
-                                    pn = f3(-ray.clipN.x, -ray.clipN.y, -ray.clipN.z);
-                            }
-                        }
-                    }
-                }
-            }
-            cell[0] = next[0];
-            cell[1] = next[1];
-            cell[2] = next[2];
-            tested = nextTested;
-            if(ax0)
-                t[0] = t[0] + dt[0];
-            else if(ax1)
-                t[1] = t[1] + dt[1];
-            else
-                t[2] = t[2] + dt[2];
-#pragma unroll
-            for(int s = 0; s < 4; s++)
-                kr[s] = krn[s];
-        }
-        if(hit)
-        {
-            normal = normalize3(pn);
-            color = to_byte4(pcol.x, pcol.y, pcol.z, 1.0f);
-            depth = pdepth + ray.startDepth;
-        }
-    }
-
-    // ------------------------------------------------------------------ fused march
-    // One pass per pixel: clear, particle DDA, then ONE traversal of the ray that
-    // serves both the iso march (CombinedIsoRenderKernel) and the volume march
-    // (CombinedVolumeRenderKernel).  Both reference kernels sample the same
-    // positions startU + stepVec*i from the same startSteps; the volume stops at
-    // floor(min(clipEnd, depth)/step) where depth is the particle/iso depth, so
-    // the iso decision at step i is made before the volume consumes step i.  The
-    // premultiplied volume colour goes to volColor and is blended over the shaded
-    // solid colour by shade_kernel after SSAO, which keeps the reference's pass
-    // order (particles, iso, SSAO, shading, volume) for every pixel.
-    // The taps of step i+1 are fetched before step i is composited (clamped
-    // addresses, so a fetch past the last step stays in bounds).
-    template<bool LINEAR, bool COUNT, bool PREFETCH, bool BRICK, bool OFF32 = false, bool HALF = false>
-    __device__ __attribute__((always_inline)) inline void march_body(const FrameParams& F, const ParticleParams& PP)
-    {
-        int px, py;
-        const bool valid = tile_pixel_at(F, march_tile(F), march_wave(F), px, py);
-        unsigned long long nCells = 0, nTests = 0, nIso = 0, nIsoHits = 0, nIsoRays = 0, nPartRays = 0;
-        unsigned long long nVol = 0, nVolRays = 0, nSteps = 0;
-        if(valid)
-        {
-            const size_t p = size_t(py) * size_t(F.W) + size_t(px);
-            uint32_t color = F.bgClear;
-            F3 normal = f3(0.f, 0.f, 0.f);
-            float depth = FLT_MAX;
-            float4 vcol = make_float4(0.f, 0.f, 0.f, -1.f);
-            Ray ray = pixel_to_ray(F, px, py);
-            const bool inside = clip_ray(F, ray);
-            // ---- particles
-            if(inside && PP.nsrc > 0)
-            {
-                nPartRays++;
-                particle_dda<COUNT>(PP, ray, color, depth, normal, nCells, nTests);
-            }
-            // ---- iso + volume, one traversal
-            const int mode = F.renderMode;
-            // ShadingKernel zeroes the depth in these modes, so the volume pass never blends there
-            const bool depthZeroed = mode == 2 || (mode >= 4 && mode <= 8);
-            if(inside)
-            {
-                const float endAfterParticles = gmin(ray.endDepth, depth);
-                bool isoOn = F.isoEnabled && endAfterParticles > ray.startDepth;
-                bool volBlend = F.volumeEnabled && !depthZeroed && endAfterParticles > ray.startDepth;
-                if(isoOn || volBlend)
-                {
-                    const F3 sc = f3(F.scale[0], F.scale[1], F.scale[2]);
-                    const float stepU = F.step * (len3(ray.dir) / len3(divv(ray.dir, sc)));
-                    const float factor = stepU / F.minSize * 2.0f * F.totalWeightAll;
-                    const int startSteps = int(ceilf(ray.startDepth / stepU));
-                    const int endIso = int(floorf(endAfterParticles / stepU));
-                    int endVol = endIso;
-                    const F3 stepVec = divv(muls(ray.dir, stepU), sc);
-                    const F3 startU = divv(ray.start, sc);
-                    if(isoOn)
-                        nIsoRays++;
-                    float cr = 0.f, cg = 0.f, cb = 0.f, ca = 0.f;
-                    // The traversal state is kept in plain numbers rather than flags, so
-                    // the loop carries no lane masks: the iso test runs while i <= isoEnd and
-                    // the volume while i <= volEnd (either set below the first step to switch
-                    // it off); hitStep is the step of the iso hit (-1: none); oldValue is the
-                    // previous step's iso sum, -1 where it was not formed; blendW is the
-                    // volume colour's w marker (0: the volume pass blends, -1: it does not).
-                    const int off = -0x7fffffff;
-                    int isoEnd = isoOn ? endIso : off;
-                    int volEnd = volBlend ? endVol : off;
-                    int hitStep = -1;
-                    float oldValue = 0.0f;
-                    float blendW = volBlend ? 0.0f : -1.0f;
-                    int i = startSteps;
-                    int last = isoOn ? endIso : endVol;
-                    if(i <= last)
-                    {
-                        // volume samples in byte units times factor / 255
-                        const float vscale = factor * (1.0f / 255.0f);
-                        const uint32_t XY = uint32_t(F.X) * uint32_t(F.Y);
-                        // sample i at startC + stepVec * i (one fma per axis), shifted by the
-                        // texel centres' -0.5 for the trilinear sampler
-                        const float sh = LINEAR ? 0.5f : 0.0f;
-                        const F3 startC = f3(startU.x - sh, startU.y - sh, startU.z - sh);
-                        // the step's corners (from the binary16 copy for HALF) and, for the iso
-                        // sums of HALF, the combined texture's corners at the same position
-                        auto at = [&](int k, Corners& C)
-                        {
-                            const float fk = float(k);
-                            fetch_corners<LINEAR, BRICK, OFF32, HALF>(F, XY, __builtin_fmaf(stepVec.x, fk, startC.x),
-                                                                      __builtin_fmaf(stepVec.y, fk, startC.y),
-                                                                      __builtin_fmaf(stepVec.z, fk, startC.z), C);
-                        };
-                        auto atIso = [&](int k, Corners& C)
-                        {
-                            const float fk = float(k);
-                            fetch_corners<LINEAR, BRICK, OFF32, false>(F, XY, __builtin_fmaf(stepVec.x, fk, startC.x),
-                                                                       __builtin_fmaf(stepVec.y, fk, startC.y),
-                                                                       __builtin_fmaf(stepVec.z, fk, startC.z), C);
-                        };
-                        // one step: the iso test and the volume sample of the corners c of step i
-                        auto process = [&](const Corners& cur) __attribute__((always_inline))
-                        {
-                            if(COUNT)
-                                nSteps++;
-                            if(i <= isoEnd)
-                            {
-                                // the iso alpha in byte units; alpha >= 0.5 is a sum >= 127.5, which
-                                // needs an alpha byte >= 128 (the corner weights sum to 1 up to a few
-                                // ulps, so eight bytes <= 127 stay below 127.1).  Without such a byte
-                                // the sum is not formed: it is exactly 0 when all alpha bytes are 0,
-                                // else it is formed again from the step's corners if the next step hits
-                                // (HALF: the flag is the sign of the binary16 alpha, and the sum
-                                // comes from the combined texture's corners of this step)
-                                const uint32_t alphas = corners_or<LINEAR, true>(cur);
-                                const bool high = (alphas >> 31) != 0u;
-                                float sum = 0.0f;
-                                if(HALF)
-                                {
-                                    if(high)
-                                    {
-                                        Corners ic;
-                                        atIso(i, ic);
-                                        sum = corner_sum<LINEAR, true>(ic, 24);
-                                    }
-                                }
-                                else if(high)
-                                    sum = corner_sum<LINEAR, true>(cur, 24);
-                                if(COUNT)
-                                    nIso++;
-                                float tmpSum = oldValue;
-                                oldValue = (high || (!HALF && (alphas >> 24) == 0u)) ? sum : -1.0f;
-                                if(sum >= 127.5f)
-                                {
-                                    if(tmpSum < 0.0f)
-                                    {
-                                        Corners pc;
-                                        atIso(i - 1, pc);
-                                        tmpSum = corner_sum<LINEAR, true>(pc, 24);
-                                    }
-                                    const bool first = ray.isClipped && i == startSteps;
-                                    const float tt = float(i) * stepU;
-                                    const float value = div255(sum), tmp = div255(tmpSum);
-                                    float d;
-                                    if(first)
-                                        d = ray.startDepth;
-                                    else
-                                        d = tt + stepU * (0.5f - tmp) / (value - tmp);
-                                    // colour and gradient at the hit are sampled after the loop
-                                    hitStep = i;
-                                    depth = d;
-                                    if(COUNT)
-                                        nIsoHits++;
-                                    isoEnd = off;
-                                    // the volume pass ends at min(clip end, iso depth)
-                                    const float ve = gmin(ray.endDepth, d);
-                                    if(!(ve > ray.startDepth))
-                                    {
-                                        volEnd = off;
-                                        blendW = -1.0f;
-                                    }
-                                    else if(volEnd != off)
-                                        volEnd = int(floorf(ve / stepU));
-                                }
-                            }
-                            // (eight zero volume texels give the sample (0,0,0,0), which leaves
-                            // the accumulated colour unchanged, so no test for them: the branch
-                            // cost more than the arithmetic it skipped)
-                            if(i <= volEnd)
-                            {
-                                if(COUNT)
-                                    nVol++;
-                                const float vr = HALF ? half_sum<0>(cur) : corner_sum<LINEAR, false>(cur, 0);
-                                const float vg = HALF ? half_sum<1>(cur) : corner_sum<LINEAR, false>(cur, 8);
-                                const float vb = HALF ? half_sum<2>(cur) : corner_sum<LINEAR, false>(cur, 16);
-                                const float va = HALF ? half_sum<3>(cur) : corner_sum<LINEAR, false>(cur, 24);
-                                const float w = (1.0f - ca) * vscale;
-                                cr = cr + w * vr;
-                                cg = cg + w * vg;
-                                cb = cb + w * vb;
-                                ca = ca + w * va;
-                                if(ca > 0.99f)
-                                    volEnd = off;
-                            }
-                        };
-                        Corners cur;
-                        at(i, cur);
-                        if constexpr(PREFETCH)
-                        {
-                            // two buffers in turn: the next step's corners are requested before
-                            // this step's are composited, with no copy between the buffers (a hit
-                            // can extend the volume pass by one step past the range requested)
-                            Corners nxt;
-                            for(;;)
-                            {
-                                bool ahead = i + 1 <= last;
-                                if(ahead)
-                                    at(i + 1, nxt);
-                                process(cur);
-                                last = isoEnd > volEnd ? isoEnd : volEnd;
-                                if(i + 1 > last)
-                                    break;
-                                i++;
-                                if(!ahead)
-                                    at(i, nxt);
-                                ahead = i + 1 <= last;
-                                if(ahead)
-                                    at(i + 1, cur);
-                                process(nxt);
-                                last = isoEnd > volEnd ? isoEnd : volEnd;
-                                if(i + 1 > last)
-                                    break;
-                                i++;
-                                if(!ahead)
-                                    at(i, cur);
-                            }
-                        }
-                        else
-                        {
-                            for(;;)
-                            {
-                                process(cur);
-                                last = isoEnd > volEnd ? isoEnd : volEnd;
-                                if(i + 1 > last)
-                                    break;
-                                i++;
-                                at(i, cur);
-                            }
-                        }
-                    }
-                    const bool isoHit = hitStep >= 0;
-                    const bool isoFirst = isoHit && ray.isClipped && hitStep == startSteps;
-                    if(isoHit)
-                    {
-                        // hit colour and central-difference gradient of the iso alpha
-                        // (lib/isaac/isaac_iso_kernel.hpp:97-119)
-                        const F3 pu = divv(add(ray.start, muls(ray.dir, depth)), sc);
-                        Taps h;
-                        fetch_taps<LINEAR, BRICK>(F, pu.x, pu.y, pu.z, h);
-                        const float hr = channel<LINEAR, true>(h, 0), hg = channel<LINEAR, true>(h, 8);
-                        const float hb = channel<LINEAR, true>(h, 16);
-                        F3 g;
-                        g.x = iso_alpha_at<LINEAR, BRICK>(F, pu.x + 1.0f, pu.y, pu.z) - iso_alpha_at<LINEAR, BRICK>(F, pu.x - 1.0f, pu.y, pu.z);
-                        g.y = iso_alpha_at<LINEAR, BRICK>(F, pu.x, pu.y + 1.0f, pu.z) - iso_alpha_at<LINEAR, BRICK>(F, pu.x, pu.y - 1.0f, pu.z);
-                        g.z = iso_alpha_at<LINEAR, BRICK>(F, pu.x, pu.y, pu.z + 1.0f) - iso_alpha_at<LINEAR, BRICK>(F, pu.x, pu.y, pu.z - 1.0f);
-                        float gl = len3(g);
-                        if(isoFirst || gl == 0.0f)
-                        {
-                            g = ray.clipN;
-                            gl = 1.0f;
-                        }
-                        normal = f3(-g.x / gl, -g.y / gl, -g.z / gl);
-                        color = to_byte4(hr, hg, hb, 1.0f);
-                    }
-                    if(blendW >= 0.0f)
-                    {
-                        nVolRays++;
-                        vcol = make_float4(cr, cg, cb, ca);
-                    }
-                }
-            }
-            F.color[p] = color;
-            F.depth[p] = depth;
-            F.normal[3 * p + 0] = normal.x;
-            F.normal[3 * p + 1] = normal.y;
-            F.normal[3 * p + 2] = normal.z;
-            F.volColor[p] = vcol;
-            if(!F.aoEnabled)
-                F.ao[p] = 0.0f;
-        }
-        if(COUNT)
-        {
-            block_count_add(F.counters + 0, nVol);
-            block_count_add(F.counters + 1, nIso);
-            block_count_add(F.counters + 2, nIsoHits);
-            block_count_add(F.counters + 3, nCells);
-            block_count_add(F.counters + 4, nTests);
-            block_count_add(F.counters + 5, nVolRays);
-            block_count_add(F.counters + 6, nIsoRays);
-            block_count_add(F.counters + 7, nPartRays);
-            block_count_add(F.counters + 8, nSteps);
-            // the wave runs the traversal loop as long as its longest lane
-            int wm = int(nSteps);
-            for(int off = 32; off > 0; off >>= 1)
-                wm = max(wm, __shfl_xor(wm, off, 64));
-            block_count_add(F.counters + 9, (threadIdx.x & 63u) == 0 ? (unsigned long long) wm : 0ull);
-        }
-    }
-
-    // The march at the compiler's register allocation, and at occupancy targets of
-    // 6 and 8 waves per SIMD (at most 80 / 64 VGPRs); the launcher picks one by the
-    // tuning key ISAAC_HIP_TUNE_MARCH_WAVES.
-    template<bool LINEAR, bool COUNT, bool PREFETCH, bool BRICK, bool OFF32 = false, bool HALF = false>
-    __global__ __launch_bounds__(256) void march_kernel(const FrameParams F, const ParticleParams PP)
-    {
-        march_body<LINEAR, COUNT, PREFETCH, BRICK, OFF32, HALF>(F, PP);
-    }
-    template<bool LINEAR, bool BRICK, bool OFF32, bool HALF = false>
-    __global__ __launch_bounds__(256, 6) void march_kernel_w6(const FrameParams F, const ParticleParams PP)
-    {
-        march_body<LINEAR, false, false, BRICK, OFF32, HALF>(F, PP);
-    }
-    template<bool LINEAR, bool BRICK, bool OFF32, bool HALF = false>
-    __global__ __launch_bounds__(256, 8) void march_kernel_w8(const FrameParams F, const ParticleParams PP)
-    {
-        march_body<LINEAR, false, false, BRICK, OFF32, HALF>(F, PP);
     }
 
     // ------------------------------------------------------------------ SSAO
@@ -2223,17 +1331,6 @@ namespace isaac_hip
 
     static_assert(sizeof(FrameParams) + sizeof(PostParams) + sizeof(ParticleParams) <= 4096, "kernel argument block");
 
-    // workgroups of a march launch: one per tile, or the padded super-tile grid
-    unsigned march_grid(const FrameParams& F)
-    {
-        const unsigned nb = unsigned(F.tilesX) * unsigned(F.tilesY);
-        const unsigned S = unsigned(F.tileOrder);
-        if(S == 0 || nb == 0)
-            return nb;
-        const unsigned ns = ((unsigned(F.tilesX) + S - 1u) / S) * ((unsigned(F.tilesY) + S - 1u) / S);
-        return (ns + 7u) / 8u * 8u * S * S;
-    }
-
     // a source's chain is its natural one: no operations for a scalar source, one
     // `length` (then nothing) for a vector source
     bool natural_chain(const ChainDesc& c, int dim)
@@ -2417,7 +1514,7 @@ namespace isaac_hip
         }
     }
 
-    // classification of one fetched quad, its 4 texels stored with two 16-byte stores
+    // classification of one fetched quad, its 4 texels stored with one 16-byte store per texture
     template<int SIG>
     __device__ __attribute__((always_inline)) inline void cls_emit(
         const ClassifyParams& P, const float4* lds_lut, const float (&f)[sig_count(SIG)][16], int x, int y, int z, int64_t q)
@@ -2425,7 +1522,7 @@ namespace isaac_hip
         constexpr int N = sig_count(SIG);
         const int T = P.T;
         const uint32_t u = uint32_t(q) << 2;
-        uint32_t texel[8];
+        uint32_t vol[4], iso[4];
 #pragma unroll
         for(int k = 0; k < 4; k++)
         {
@@ -2476,34 +1573,16 @@ namespace isaac_hip
             {
                 vr = vg = vb = va = 0.0f;
             }
-            texel[2 * k] = dither_b4(P.ditherMode, x + k, y, z, vr, vg, vb, va);
+            vol[k] = dither_b4(P.ditherMode, x + k, y, z, vr, vg, vb, va);
             const uint32_t q0 = unorm8(ir), q1 = unorm8(ig), q2 = unorm8(ib), q3 = unorm8(ia);
-            texel[2 * k + 1] = q0 | (q1 << 8) | (q2 << 16) | (q3 << 24);
+            iso[k] = q0 | (q1 << 8) | (q2 << 16) | (q3 << 24);
         }
-        uint4* o = reinterpret_cast<uint4*>(P.tex + u);
-        if(P.texH)
+        *reinterpret_cast<uint4*>(P.vol + u) = make_uint4(vol[0], vol[1], vol[2], vol[3]);
+        if(P.iso)
         {
-            // the march steps over the binary16 copy and reads the combined texture only at
-            // steps that can hit the iso-surface: its stores are non-temporal, so they do not
-            // displace the copy from the caches
-            typedef uint32_t v4u __attribute__((ext_vector_type(4)));
-            __builtin_nontemporal_store(v4u{texel[0], texel[1], texel[2], texel[3]}, reinterpret_cast<v4u*>(o));
-            __builtin_nontemporal_store(v4u{texel[4], texel[5], texel[6], texel[7]}, reinterpret_cast<v4u*>(o) + 1);
-        }
-        else
-        {
-            o[0] = make_uint4(texel[0], texel[1], texel[2], texel[3]);
-            o[1] = make_uint4(texel[4], texel[5], texel[6], texel[7]);
-        }
-        if(P.texH)
-        {
-            uint2 h[4];
-#pragma unroll
-            for(int k = 0; k < 4; k++)
-                h[k] = half_texel(texel[2 * k], texel[2 * k + 1]);
-            uint4* oh = reinterpret_cast<uint4*>(P.texH + u);
-            oh[0] = make_uint4(h[0].x, h[0].y, h[1].x, h[1].y);
-            oh[1] = make_uint4(h[2].x, h[2].y, h[3].x, h[3].y);
+            *reinterpret_cast<uint4*>(P.iso + u) = make_uint4(iso[0], iso[1], iso[2], iso[3]);
+            if(((iso[0] | iso[1] | iso[2] | iso[3]) >> 31) != 0u)
+                mark_iso_cells(P, x, x + 3, y, z);
         }
     }
 
@@ -2513,7 +1592,7 @@ namespace isaac_hip
     // thread classifies 4 consecutive voxels of a row per iteration (every source's
     // values in 16-byte loads; requesting the next quad's values before classifying the
     // current one held 32 more VGPRs, 90 against 71, and was 11 % slower than the
-    // occupancy that frees) and stores the 4 texels with two 16-byte stores.  Same
+    // occupancy that frees) and stores the 4 texels with one 16-byte store per texture.  Same
     // arithmetic, in the same order, as classify_kernel.  Workgroups of 512 threads:
     // eight waves share one LDS copy of the transfer functions, which halves the
     // staging reads against 256-thread workgroups and lets 8 waves per SIMD be
@@ -2545,7 +1624,7 @@ namespace isaac_hip
     // Pc receives the active sources in slot order
     int classify_signature(const ClassifyParams& P, ClassifyParams& Pc)
     {
-        if(P.X % 4 != 0 || (reinterpret_cast<uintptr_t>(P.tex) & 15u) != 0)
+        if(P.X % 4 != 0 || ((reinterpret_cast<uintptr_t>(P.vol) | reinterpret_cast<uintptr_t>(P.iso)) & 15u) != 0)
             return 0;
         Pc = P;
         int n = 0, sig = 0, w = 1;
@@ -2844,134 +1923,21 @@ namespace isaac_hip
         return hipGetLastError();
     }
 
-    // the trilinear march over the binary16 copy (texture layout 16), at every schedule
-    template<bool OFF32>
-    void launch_march_half(const FrameParams& F, const ParticleParams& PP, bool counting, bool prefetch, dim3 grid, dim3 block,
-                           hipStream_t s)
+    // The combined texture with both texels of a voxel side by side, for readers of the
+    // textures (the march reads the two separately); iso == nullptr: iso texels of 0.
+    __global__ __launch_bounds__(256) void interleave_kernel(const uint32_t* __restrict__ vol, const uint32_t* __restrict__ iso,
+                                                             uint2* __restrict__ out, int64_t n)
     {
-        if(counting)
-            hipLaunchKernelGGL((march_kernel<true, true, false, false, OFF32, true>), grid, block, 0, s, F, PP);
-        else if(prefetch)
-            hipLaunchKernelGGL((march_kernel<true, false, true, false, OFF32, true>), grid, block, 0, s, F, PP);
-        else if(F.waves == 6)
-            hipLaunchKernelGGL((march_kernel_w6<true, false, OFF32, true>), grid, block, 0, s, F, PP);
-        else if(F.waves == 8)
-            hipLaunchKernelGGL((march_kernel_w8<true, false, OFF32, true>), grid, block, 0, s, F, PP);
-        else
-            hipLaunchKernelGGL((march_kernel<true, false, false, false, OFF32, true>), grid, block, 0, s, F, PP);
+        for(int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += int64_t(gridDim.x) * blockDim.x)
+            out[i] = make_uint2(vol[i], iso ? iso[i] : 0u);
     }
 
-    template<bool BRICK>
-    hipError_t launch_march_layout(const FrameParams& F, const ParticleParams& PP, bool counting, hipStream_t s)
+    hipError_t launch_interleave(const uint32_t* vol, const uint32_t* iso, uint2* out, int64_t n, hipStream_t s)
     {
-        const unsigned nb = march_grid(F);
-        if(nb == 0)
+        if(n <= 0)
             return hipSuccess;
-        // one-wave workgroups: 4 per logical workgroup, the logical grid rounded to 8
-        const dim3 grid(F.waveGroups == 1 ? (nb + 7u) / 8u * 32u : nb), block(F.waveGroups == 1 ? 64 : 256);
-        // next-step prefetch is compiled for the linear layout only
-        const bool prefetch = F.prefetch && !BRICK;
-        if constexpr(!BRICK)
-        {
-            if(F.texH && F.linear)
-            {
-                if(F.texOff32)
-                    launch_march_half<true>(F, PP, counting, prefetch, grid, block, s);
-                else
-                    launch_march_half<false>(F, PP, counting, prefetch, grid, block, s);
-                return hipGetLastError();
-            }
-        }
-        if(!counting && !prefetch && (F.waves == 6 || F.waves == 8))
-        {
-            if(F.waves == 6)
-            {
-                if(F.linear && F.texOff32)
-                    hipLaunchKernelGGL((march_kernel_w6<true, BRICK, true>), grid, block, 0, s, F, PP);
-                else if(F.linear)
-                    hipLaunchKernelGGL((march_kernel_w6<true, BRICK, false>), grid, block, 0, s, F, PP);
-                else
-                    hipLaunchKernelGGL((march_kernel_w6<false, BRICK, false>), grid, block, 0, s, F, PP);
-            }
-            else
-            {
-                if(F.linear && F.texOff32)
-                    hipLaunchKernelGGL((march_kernel_w8<true, BRICK, true>), grid, block, 0, s, F, PP);
-                else if(F.linear)
-                    hipLaunchKernelGGL((march_kernel_w8<true, BRICK, false>), grid, block, 0, s, F, PP);
-                else
-                    hipLaunchKernelGGL((march_kernel_w8<false, BRICK, false>), grid, block, 0, s, F, PP);
-            }
-            return hipGetLastError();
-        }
-        const int v = (F.linear ? 4 : 0) | (counting ? 2 : 0) | (prefetch ? 1 : 0);
-        switch(v)
-        {
-        case 0: hipLaunchKernelGGL((march_kernel<false, false, false, BRICK>), grid, block, 0, s, F, PP); break;
-        case 2: hipLaunchKernelGGL((march_kernel<false, true, false, BRICK>), grid, block, 0, s, F, PP); break;
-        case 4:
-            if(F.texOff32)
-                hipLaunchKernelGGL((march_kernel<true, false, false, BRICK, true>), grid, block, 0, s, F, PP);
-            else
-                hipLaunchKernelGGL((march_kernel<true, false, false, BRICK, false>), grid, block, 0, s, F, PP);
-            break;
-        case 6: hipLaunchKernelGGL((march_kernel<true, true, false, BRICK>), grid, block, 0, s, F, PP); break;
-        default:
-            if constexpr(!BRICK)
-            {
-                if(v == 1)
-                    hipLaunchKernelGGL((march_kernel<false, false, true, false>), grid, block, 0, s, F, PP);
-                else if(v == 3)
-                    hipLaunchKernelGGL((march_kernel<false, true, true, false>), grid, block, 0, s, F, PP);
-                else if(v == 5 && F.texOff32)
-                    hipLaunchKernelGGL((march_kernel<true, false, true, false, true>), grid, block, 0, s, F, PP);
-                else if(v == 5)
-                    hipLaunchKernelGGL((march_kernel<true, false, true, false>), grid, block, 0, s, F, PP);
-                else
-                    hipLaunchKernelGGL((march_kernel<true, true, true, false>), grid, block, 0, s, F, PP);
-            }
-            break;
-        }
-        return hipGetLastError();
-    }
-
-    hipError_t launch_march(const FrameParams& F, const ParticleParams& PP, bool counting, hipStream_t s)
-    {
-        return F.texB ? launch_march_layout<true>(F, PP, counting, s) : launch_march_layout<false>(F, PP, counting, s);
-    }
-
-    // Linear texture -> brick layout (FrameParams::texB): one workgroup per brick, the
-    // 729 texels of brick b (apron and parts beyond the volume take the clamped texel)
-    // written in order.
-    __global__ __launch_bounds__(256) void tex_brick_kernel(
-        const uint2* __restrict__ tex,
-        uint2* __restrict__ out,
-        int X,
-        int Y,
-        int Z,
-        uint32_t nbx,
-        uint32_t nby)
-    {
-        const uint32_t b = blockIdx.x;
-        const uint32_t bx = b % nbx, by = (b / nbx) % nby, bz = b / (nbx * nby);
-        for(uint32_t t = threadIdx.x; t < uint32_t(kTexBrickTexels); t += 256u)
-        {
-            const uint32_t lz = t / uint32_t(kTexBrickSlice), ly = (t / uint32_t(kTexBrickRow)) % uint32_t(kTexBrickRow);
-            const uint32_t lx = t % uint32_t(kTexBrickRow);
-            const uint32_t x = min(bx * uint32_t(kTexBrick) + lx, uint32_t(X - 1));
-            const uint32_t y = min(by * uint32_t(kTexBrick) + ly, uint32_t(Y - 1));
-            const uint32_t z = min(bz * uint32_t(kTexBrick) + lz, uint32_t(Z - 1));
-            out[size_t(b) * kTexBrickTexels + t] = tex[x + size_t(X) * (y + size_t(Y) * z)];
-        }
-    }
-
-    hipError_t launch_tex_bricks(const uint2* tex, uint2* out, int X, int Y, int Z, hipStream_t s)
-    {
-        const uint32_t nbx = uint32_t(X + kTexBrick - 1) / kTexBrick, nby = uint32_t(Y + kTexBrick - 1) / kTexBrick;
-        const uint32_t nbz = uint32_t(Z + kTexBrick - 1) / kTexBrick;
-        if(nbx * nby * nbz == 0)
-            return hipSuccess;
-        hipLaunchKernelGGL(tex_brick_kernel, dim3(nbx * nby * nbz), dim3(256), 0, s, tex, out, X, Y, Z, nbx, nby);
+        const int64_t blocks = std::min<int64_t>((n + 255) / 256, 4096);
+        hipLaunchKernelGGL(interleave_kernel, dim3(unsigned(blocks)), dim3(256), 0, s, vol, iso, out, n);
         return hipGetLastError();
     }
 

@@ -1,0 +1,95 @@
+"""The combined form's march against its counting variant, which tests the iso alpha
+and clamps the texels at every step: volumes about the sizes of a texel, of an iso
+cell (8 texels) and of several, where the interior steps and the marked cells begin
+and end, and the states an iso texture can be in between updates."""
+import dataclasses
+
+import numpy as np
+import pytest
+
+from isaac_amd import scenes
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", autouse=True)
+def gpu():
+    torch = pytest.importorskip("torch")
+    if not torch.cuda.is_available():
+        pytest.skip("needs a GPU")
+
+
+def _spec(size, linear=True, iso=0.4, step=0.5, pose=scenes.DEFAULT_POSE):
+    X, Y, Z = size
+    rng = np.random.default_rng(X * 10007 + Y * 101 + Z)
+    dens = (0.7 * scenes.gaussian_mixture((Z, Y, X), 5, 6, (0.08 * max(size), 0.3 * max(size)))
+            + 0.2 * rng.uniform(0.0, 1.0, (Z, Y, X))).astype(np.float32)
+    vol = scenes.VolumeSourceSpec("density", dens, "idem", list(scenes.DENSITY_TF), 2.0, iso)
+    return scenes.SceneSpec("march", tuple(size), tuple(size), (1, 1, 1), framebuffer=(150, 117), volumes=[vol], step=step,
+                            interpolation=linear, camera=pose, clipping=[((0.1, 0.0, 0.0), (1.0, 0.2, 0.0))])
+
+
+def _counting_equal(vis):
+    img = vis.draw()
+    g = [a.copy() for a in vis.gbuffer()]
+    vis.set_counting(True)
+    ref = vis.draw()
+    gr = [a.copy() for a in vis.gbuffer()]
+    vis.set_counting(False)
+    assert np.array_equal(img, ref)
+    for a, b in zip(g, gr):
+        assert np.array_equal(a, b)
+    return img
+
+
+@pytest.mark.parametrize("linear", [True, False])
+@pytest.mark.parametrize("size", [(1, 1, 1), (2, 1, 3), (7, 8, 9), (16, 17, 15), (40, 8, 23), (8, 64, 8), (65, 33, 49)])
+def test_march_equals_counting_march(size, linear):
+    from isaac_amd import visualization as V
+
+    for step, pose in ((0.5, scenes.FILL_POSE), (0.13, scenes.Camera(distance=-1.2)), (3.0, scenes.DEFAULT_POSE)):
+        vis = V.from_scene(_spec(size, linear, step=step, pose=pose))
+        for iso in (0.4, 0.05, 0.0):
+            vis.iso_threshold = [iso]
+            vis.update_buffers()
+            _counting_equal(vis)
+        vis.close()
+
+
+def test_iso_threshold_changed_between_updates():
+    """A threshold set after a classification without one finds no surface until the next
+    update, as the iso texels are 0 then; the texels a caller asked for follow every update."""
+    from isaac_amd import visualization as V
+
+    vis = V.from_scene(_spec((24, 20, 16), iso=0.0))
+    vis.update_buffers()
+    plain = _counting_equal(vis)
+    vol, iso = vis.combined_textures()
+    assert not iso.any() and vol.any()
+    vis.iso_threshold = [0.3]
+    assert np.array_equal(_counting_equal(vis), plain)
+    vis.update_buffers()
+    assert not np.array_equal(_counting_equal(vis), plain)
+    vol2, iso2 = vis.combined_textures()
+    assert iso2.any() and np.array_equal(vol, vol2)
+    vis.iso_threshold = [0.0]
+    vis.update_buffers()
+    assert np.array_equal(_counting_equal(vis), plain)
+    assert not vis.combined_textures()[1].any()
+    vis.close()
+
+
+def test_iso_cell_marks_do_not_outlive_their_update():
+    """300 updates (the marks' numbers wrap at 255), a surface in every 70th."""
+    from isaac_amd import visualization as V
+
+    vis = V.from_scene(dataclasses.replace(_spec((24, 20, 16)), clipping=[]))
+    vis.update_buffers()
+    with_iso = vis.draw()
+    for k in range(300):
+        vis.iso_threshold = [0.4 if k % 70 == 69 else 0.0]
+        vis.update_buffers()
+        if k % 70 == 69:
+            assert np.array_equal(_counting_equal(vis), with_iso)
+    assert not np.array_equal(_counting_equal(vis), with_iso)
+    vis.close()
