@@ -1,14 +1,7 @@
 // Learned occlusion pass: U-Net kernels on gfx950 (forward, backward, Adam).
 //
-// Convolutions are implicit GEMMs on the matrix cores: the forward layers on
-// v_mfma_f32_16x16x32_f16 (below, "forward convolution"), backward data and the
-// weight gradient on v_mfma_f32_16x16x16_f16.  For one 16x16x16 step, lane l of
-// the wave supplies
-//   A (16 x 16, rows = output channels):  row l % 16, k = 4*(l / 16) .. +3
-//   B (16 x 16, cols = pixels):           col l % 16, k = 4*(l / 16) .. +3
-// and receives D rows 4*(l / 16) .. +3 of column l % 16.  With k = tap*Cin + ci
-// and Cin a multiple of 4, the four k of a lane are four consecutive channels of
-// one tap: one 8-byte load each for A (weights) and B (input patch in LDS).
+// Convolutions are implicit GEMMs on the matrix cores (v_mfma_f32_16x16x32_f16, below);
+// the weight gradients are in aonet_grad.hip.
 #include "aonet.hpp"
 
 #include <cfloat>
@@ -18,158 +11,8 @@ namespace isaac_hip
     typedef _Float16 h4 __attribute__((ext_vector_type(4)));
     typedef float f4 __attribute__((ext_vector_type(4)));
 
-    __device__ inline f4 mfma16(h4 a, h4 b, f4 c)
-    {
-        return __builtin_amdgcn_mfma_f32_16x16x16f16(a, b, c, 0, 0, 0);
-    }
-
     // ------------------------------------------------------------------ convolution
-    // stage rows y0-1 .. y0+rows of the 66-pixel-wide window at x0-1 (zero outside
-    // the image) into LDS as [row][66][cin]; channels < ca come upsampled from `up`
-    __device__ inline void stage_patch(
-        _Float16* patch,
-        const _Float16* __restrict__ x,
-        const _Float16* __restrict__ up,
-        int ca,
-        int cin,
-        int n,
-        int h,
-        int w,
-        int y0,
-        int x0,
-        int rows)
-    {
-        const int cs = cin - ca;
-        const int units = rows * 66 * cin / 4;
-        for(int u = threadIdx.x; u < units; u += blockDim.x)
-        {
-            const int e = u * 4;
-            const int pix = e / cin, c = e - pix * cin;
-            const int r = pix / 66, col = pix - r * 66;
-            const int yy = y0 + r - 1, xx = x0 + col - 1;
-            h4 v = {0, 0, 0, 0};
-            if(yy >= 0 && yy < h && xx >= 0 && xx < w)
-            {
-                if(c < ca)
-                    v = *reinterpret_cast<const h4*>(up + ((size_t(n) * (h / 2) + yy / 2) * (w / 2) + xx / 2) * ca + c);
-                else
-                    v = *reinterpret_cast<const h4*>(x + ((size_t(n) * h + yy) * w + xx) * cs + (c - ca));
-            }
-            *reinterpret_cast<h4*>(patch + e) = v;
-        }
-    }
-
-    // Backward data: dx (FP32, +=) = conv(dz, flipped transposed weights).
-    // Workgroup = ROWS image rows x 64 pixels; four waves split the 64-pixel row
-    // segment into 16-pixel columns, and each wave computes its column in all ROWS
-    // rows for all output channels, so every weight fragment it loads feeds ROWS
-    // MFMAs.  The (ROWS + 2) x 66 x cin input patch is staged in LDS once.
-    template<int COUT, int ROWS>
-    __global__ __launch_bounds__(256) void conv3x3_bwd_kernel(const ConvArgs a)
-    {
-        extern __shared__ _Float16 patch[];
-        const int x0 = blockIdx.x * 64, y0 = blockIdx.y * ROWS, n = blockIdx.z;
-        const int cin = a.cin;
-        stage_patch(patch, a.x, a.up, a.ca, cin, n, a.h, a.w_, y0, x0, ROWS + 2);
-        __syncthreads();
-        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-        const int pl = wave * 16 + (lane & 15);
-        const int kq = 4 * (lane >> 4);
-        f4 acc[ROWS][COUT / 16];
-#pragma unroll
-        for(int r = 0; r < ROWS; r++)
-#pragma unroll
-            for(int cb = 0; cb < COUT / 16; cb++)
-                acc[r][cb] = f4{0.f, 0.f, 0.f, 0.f};
-        const _Float16* wrow = a.w + size_t(lane & 15) * a.kp;
-        for(int kc = 0; kc < a.kp; kc += 16)
-        {
-            const int kk = kc + kq;
-            const int tap = kk / cin, ci = kk - tap * cin;
-            h4 w[COUT / 16];
-#pragma unroll
-            for(int cb = 0; cb < COUT / 16; cb++)
-                w[cb] = *reinterpret_cast<const h4*>(wrow + size_t(cb * 16) * a.kp + kk);
-            const bool valid = tap < 9;
-            const int ky = valid ? tap / 3 : 0, kx = valid ? tap - ky * 3 : 0;
-#pragma unroll
-            for(int r = 0; r < ROWS; r++)
-            {
-                h4 b = {0, 0, 0, 0};
-                if(valid)
-                    b = *reinterpret_cast<const h4*>(patch + ((r + ky) * 66 + pl + kx) * cin + ci);
-#pragma unroll
-                for(int cb = 0; cb < COUT / 16; cb++)
-                    acc[r][cb] = mfma16(w[cb], b, acc[r][cb]);
-            }
-        }
-        const int x = x0 + pl;
-        if(x >= a.w_)
-            return;
-#pragma unroll
-        for(int r = 0; r < ROWS; r++)
-        {
-            const int y = y0 + r;
-            if(y >= a.h)
-                break;
-            const size_t p = (size_t(n) * a.h + y) * a.w_ + x;
-#pragma unroll
-            for(int cb = 0; cb < COUT / 16; cb++)
-            {
-                const int co = cb * 16 + 4 * (lane >> 4);
-                float4* dst = reinterpret_cast<float4*>(reinterpret_cast<float*>(a.y) + p * COUT + co);
-                float4 d = *dst;
-                d.x += acc[r][cb][0];
-                d.y += acc[r][cb][1];
-                d.z += acc[r][cb][2];
-                d.w += acc[r][cb][3];
-                *dst = d;
-            }
-        }
-    }
-
-    template<int COUT, int ROWS>
-    hipError_t conv_bwd_launch(const ConvArgs& a, hipStream_t s)
-    {
-        const dim3 grid(unsigned((a.w_ + 63) / 64), unsigned((a.h + ROWS - 1) / ROWS), unsigned(a.n));
-        const size_t lds = size_t((ROWS + 2) * 66) * a.cin * sizeof(_Float16);
-        hipLaunchKernelGGL((conv3x3_bwd_kernel<COUT, ROWS>), grid, dim3(256), lds, s, a);
-        return hipGetLastError();
-    }
-
-    template<int COUT>
-    hipError_t conv_bwd_rows(const ConvArgs& a, size_t max_lds, hipStream_t s)
-    {
-        // four rows per workgroup when the patch fits and the grid still covers the
-        // chip several times over; else one
-        const size_t lds4 = size_t(6 * 66) * a.cin * sizeof(_Float16);
-        const int64_t groups4 = int64_t((a.w_ + 63) / 64) * ((a.h + 3) / 4) * a.n;
-        if(lds4 <= max_lds && groups4 >= 1024)
-            return conv_bwd_launch<COUT, 4>(a, s);
-        return conv_bwd_launch<COUT, 1>(a, s);
-    }
-
-    hipError_t launch_conv3x3_bwd(const ConvArgs& a, int cout, size_t max_lds, hipStream_t s)
-    {
-        if(a.cin % 4 != 0 || a.ca % 4 != 0 || a.ca > a.cin || (a.ca > 0 && !a.up) || a.kp % 16 != 0 || a.kp < 9 * a.cin
-           || size_t(3 * 66) * a.cin * 2 > max_lds || (a.up && (a.h % 2 || a.w_ % 2)))
-            return hipErrorInvalidValue;
-        if(a.n == 0 || a.h == 0 || a.w_ == 0)
-            return hipSuccess;
-        switch(cout)
-        {
-        case 16: return conv_bwd_rows<16>(a, max_lds, s);
-        case 32: return conv_bwd_rows<32>(a, max_lds, s);
-        case 48: return conv_bwd_rows<48>(a, max_lds, s);
-        case 64: return conv_bwd_rows<64>(a, max_lds, s);
-        case 96: return conv_bwd_rows<96>(a, max_lds, s);
-        case 128: return conv_bwd_rows<128>(a, max_lds, s);
-        default: return hipErrorInvalidValue;
-        }
-    }
-
-    // ------------------------------------------------------------------ forward convolution
-    // Forward layers run on v_mfma_f32_16x16x32_f16 (gfx950): lane l supplies
+    // Forward layers (and, with GRAD, their backward data) run on v_mfma_f32_16x16x32_f16 (gfx950): lane l supplies
     //   A row l % 16 (output channel), k = 8*(l / 16) .. +7
     //   B col l % 16 (pixel),          k = 8*(l / 16) .. +7
     // and receives D rows 4*(l / 16) .. +3 of column l % 16.  Cin is a multiple of 8,
@@ -298,7 +141,9 @@ namespace isaac_hip
     // x ROWS rows, so each weight fragment feeds NPC * ROWS MFMAs.  Weights come from
     // LDS (loaded once per workgroup) or, when they do not fit, from global memory
     // PD chunks ahead of the MFMAs.
-    template<int CIN, int COUT, int CA, int ROWS>
+    // GRAD: y is FP32 without bias and ReLU, and workgroups with blockIdx.y = s compute the
+    // 16-channel blocks s * COUT .. of a.couts output channels.
+    template<int CIN, int COUT, int CA, int ROWS, bool GRAD = false>
     __global__ __launch_bounds__(256) void conv_fwd_kernel(const ConvArgs a, int tilesX, int tilesY, int numTiles)
     {
         using L = FwdLds<CIN, COUT>;
@@ -325,6 +170,7 @@ namespace isaac_hip
         };
         PatchStager<CIN, CA, ROWS + 2> st;
         st.init();
+        const _Float16* wsrc = GRAD ? a.w + size_t(blockIdx.y) * COUT * KP : a.w;
         int t = int(blockIdx.x), n, y0, x0;
         coords(t, n, y0, x0);
         if constexpr(WLDS)
@@ -337,7 +183,7 @@ namespace isaac_hip
             {
                 const int u = int(threadIdx.x) + it * 256;
                 if(WU % 256 == 0 || u < WU)
-                    wv[it] = *reinterpret_cast<const h8*>(a.w + size_t(u) * 8);
+                    wv[it] = *reinterpret_cast<const h8*>(wsrc + size_t(u) * 8);
             }
             st.load(a.x, a.up, n, a.h, a.w_, y0, x0);
 #pragma unroll
@@ -353,13 +199,13 @@ namespace isaac_hip
         }
         else
             st.load(a.x, a.up, n, a.h, a.w_, y0, x0);
-        const _Float16* wrow = a.w + size_t(cb * 16 + (lane & 15)) * KP + 8 * g;
+        const _Float16* wrow = wsrc + size_t(cb * 16 + (lane & 15)) * KP + 8 * g;
         _Float16* y = reinterpret_cast<_Float16*>(a.y);
         const int co = cb * 16 + 4 * g;
         float bias[4];
 #pragma unroll
         for(int e = 0; e < 4; e++)
-            bias[e] = a.bias[co + e];
+            bias[e] = GRAD ? 0.0f : a.bias[co + e];
         for(; t < numTiles; t += int(gridDim.x))
         {
             st.store(patch);
@@ -427,6 +273,13 @@ namespace isaac_hip
                     const int yy = cy0 + r;
                     const bool in = xin && yy < a.h;
                     const size_t p = (size_t(cn) * a.h + yy) * a.w_ + x;
+                    if constexpr(GRAD)
+                    {
+                        if(in)
+                            *reinterpret_cast<f4*>(reinterpret_cast<float*>(a.y) + p * (size_t(gridDim.y) * COUT)
+                                                   + size_t(blockIdx.y) * COUT + co) = acc[r][q];
+                        continue;
+                    }
                     h4 o;
 #pragma unroll
                     for(int e = 0; e < 4; e++)
@@ -503,8 +356,8 @@ namespace isaac_hip
         return cus[dev];
     }
 
-    template<int CIN, int COUT, int CA, int ROWS>
-    hipError_t conv_fwd_launch(const ConvArgs& a, hipStream_t s)
+    template<int CIN, int COUT, int CA, int ROWS, bool GRAD>
+    hipError_t conv_fwd_launch(const ConvArgs& a, int slices, hipStream_t s)
     {
         const int tilesX = (a.w_ + 63) / 64, tilesY = (a.h + ROWS - 1) / ROWS;
         const int64_t numTiles = int64_t(tilesX) * tilesY * a.n;
@@ -515,13 +368,13 @@ namespace isaac_hip
         if(perCu == 0)
         {
             int v = 0;
-            if(hipOccupancyMaxActiveBlocksPerMultiprocessor(&v, conv_fwd_kernel<CIN, COUT, CA, ROWS>, 256, lds) != hipSuccess || v <= 0)
+            if(hipOccupancyMaxActiveBlocksPerMultiprocessor(&v, conv_fwd_kernel<CIN, COUT, CA, ROWS, GRAD>, 256, lds) != hipSuccess || v <= 0)
                 v = 1;
             perCu = v;
         }
-        const int64_t grid = std::min<int64_t>(numTiles, int64_t(device_cus()) * perCu);
-        hipLaunchKernelGGL((conv_fwd_kernel<CIN, COUT, CA, ROWS>), dim3(unsigned(grid)), dim3(256), lds, s, a, tilesX, tilesY,
-                           int(numTiles));
+        const int64_t grid = std::min<int64_t>(numTiles, (int64_t(device_cus()) * perCu + slices - 1) / slices);
+        hipLaunchKernelGGL((conv_fwd_kernel<CIN, COUT, CA, ROWS, GRAD>), dim3(unsigned(grid), unsigned(slices)), dim3(256), lds, s,
+                           a, tilesX, tilesY, int(numTiles));
         return hipGetLastError();
     }
 
@@ -529,8 +382,8 @@ namespace isaac_hip
     // workgroups per CU and whose tiles cover every CU twice; else the most that fit
     // with a tile per CU; else the fewest that fit (a fused pool needs an even count).
     // A wave keeps at most 8 accumulator tiles (rows x its 16-pixel columns).
-    template<int CIN, int COUT, int CA>
-    hipError_t conv_fwd_rows(const ConvArgs& a, size_t max_lds, hipStream_t s)
+    template<int CIN, int COUT, int CA, bool GRAD = false>
+    hipError_t conv_fwd_rows(const ConvArgs& a, size_t max_lds, hipStream_t s, int slices = 1)
     {
         using L = FwdLds<CIN, COUT>;
         constexpr int NPC = COUT / 16 < 4 ? COUT / 16 : 4;
@@ -549,16 +402,16 @@ namespace isaac_hip
             const int64_t minTiles = pass == 0 ? 2 * cus : (pass == 1 ? cus : 0);
             if constexpr(fits(8))
                 if(pass < 2 && ok(8, lim, minTiles))
-                    return conv_fwd_launch<CIN, COUT, CA, 8>(a, s);
+                    return conv_fwd_launch<CIN, COUT, CA, 8, GRAD>(a, slices, s);
             if constexpr(fits(4))
                 if(pass < 2 && ok(4, lim, minTiles))
-                    return conv_fwd_launch<CIN, COUT, CA, 4>(a, s);
+                    return conv_fwd_launch<CIN, COUT, CA, 4, GRAD>(a, slices, s);
             if constexpr(fits(2))
                 if(ok(2, lim, minTiles) && (pass < 2 || !ok(1, lim, 0)))
-                    return conv_fwd_launch<CIN, COUT, CA, 2>(a, s);
+                    return conv_fwd_launch<CIN, COUT, CA, 2, GRAD>(a, slices, s);
             if constexpr(fits(1))
                 if(ok(1, lim, minTiles))
-                    return conv_fwd_launch<CIN, COUT, CA, 1>(a, s);
+                    return conv_fwd_launch<CIN, COUT, CA, 1, GRAD>(a, slices, s);
         }
         return hipErrorInvalidValue;
     }
@@ -592,252 +445,43 @@ namespace isaac_hip
         return hipErrorInvalidValue;
     }
 
-    // ------------------------------------------------------------------ weight gradient
-    // GEMM dW (cout x kp) = dZ^T (cout x P) . col(X) (P x kp) over the pixels P.
-    // Workgroup (tile group g, pixel split q): waves own up to 4 16x16 tiles of dW each
-    // (tile t = (cb, kb), t = g*16 + wave*4 + j) and accumulate over the 64-pixel row
-    // segments [q*segs, (q+1)*segs); one FP32 atomic per tile element at the end.
-    __global__ __launch_bounds__(256) void conv_dw_kernel(
-        const _Float16* __restrict__ x,
-        const _Float16* __restrict__ up,
-        int ca,
-        const _Float16* __restrict__ dz,
-        float* __restrict__ dw,
-        int n,
-        int h,
-        int w,
-        int cin,
-        int cout,
-        int kdim,
-        int segsPerBlock)
+    hipError_t launch_conv_bwd(const ConvArgs& a, int cout, size_t max_lds, hipStream_t s)
     {
-        extern __shared__ _Float16 lds[];
-        _Float16* patch = lds; // [3][66][cin]
-        _Float16* dzt = lds + 3 * 66 * cin; // [64][cout]
-        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-        const int ncb = cout / 16, nkb = (kdim + 15) / 16, ntiles = ncb * nkb;
-        const int segW = (w + 63) / 64;
-        const int64_t nseg = int64_t(n) * h * segW;
-        int tcb[4], tkb[4];
-        bool own[4];
-        for(int j = 0; j < 4; j++)
-        {
-            const int t = blockIdx.x * 16 + wave * 4 + j;
-            own[j] = t < ntiles;
-            tcb[j] = own[j] ? t / nkb : 0;
-            tkb[j] = own[j] ? t - tcb[j] * nkb : 0;
-        }
-        f4 acc[4];
-        for(int j = 0; j < 4; j++)
-            acc[j] = f4{0.f, 0.f, 0.f, 0.f};
-        const int64_t s0 = int64_t(blockIdx.y) * segsPerBlock;
-        const int64_t s1 = s0 + segsPerBlock < nseg ? s0 + segsPerBlock : nseg;
-        for(int64_t sg = s0; sg < s1; sg++)
-        {
-            const int xs = int(sg % segW) * 64;
-            const int64_t row = sg / segW;
-            const int y = int(row % h), img = int(row / h);
-            __syncthreads();
-            stage_patch(patch, x, up, ca, cin, img, h, w, y, xs, 3);
-            const int dunits = 64 * cout / 4;
-            for(int u = threadIdx.x; u < dunits; u += 256)
-            {
-                const int e = u * 4;
-                const int pix = e / cout, c = e - pix * cout;
-                h4 v = {0, 0, 0, 0};
-                if(xs + pix < w)
-                    v = *reinterpret_cast<const h4*>(dz + ((size_t(img) * h + y) * w + xs + pix) * cout + c);
-                *reinterpret_cast<h4*>(dzt + e) = v;
-            }
-            __syncthreads();
-            for(int sub = 0; sub < 4; sub++)
-            {
-                const int pb = sub * 16 + 4 * (lane >> 4);
-                for(int j = 0; j < 4; j++)
-                {
-                    if(!own[j])
-                        continue;
-                    const int co = tcb[j] * 16 + (lane & 15);
-                    h4 av;
-                    for(int e = 0; e < 4; e++)
-                        av[e] = dzt[(pb + e) * cout + co];
-                    const int k = tkb[j] * 16 + (lane & 15);
-                    const int tap = k / cin, ci = k - tap * cin;
-                    h4 bv = {0, 0, 0, 0};
-                    if(tap < 9)
-                    {
-                        const int ky = tap / 3, kx = tap - ky * 3;
-                        for(int e = 0; e < 4; e++)
-                            bv[e] = patch[(ky * 66 + pb + e + kx) * cin + ci];
-                    }
-                    acc[j] = mfma16(av, bv, acc[j]);
-                }
-            }
-        }
-        for(int j = 0; j < 4; j++)
-        {
-            if(!own[j])
-                continue;
-            const int k = tkb[j] * 16 + (lane & 15);
-            if(k >= kdim)
-                continue;
-            for(int r = 0; r < 4; r++)
-            {
-                const int co = tcb[j] * 16 + 4 * (lane >> 4) + r;
-                if(acc[j][r] != 0.0f)
-                    atomicAdd(dw + size_t(co) * kdim + k, acc[j][r]);
-            }
-        }
-    }
-
-    hipError_t launch_conv3x3_dw(
-        const _Float16* x,
-        const _Float16* up,
-        int ca,
-        const _Float16* dz,
-        float* dw,
-        int n,
-        int h,
-        int w,
-        int cin,
-        int cout,
-        hipStream_t s)
-    {
-        if(cin % 4 != 0 || cout % 16 != 0 || ca % 4 != 0 || ca > cin || (ca > 0 && !up) || (up && (h % 2 || w % 2)))
+        if(a.up || a.pool || a.head || a.ca != 0)
             return hipErrorInvalidValue;
-        const int kdim = 9 * cin;
-        const int64_t nseg = int64_t(n) * h * ((w + 63) / 64);
-        if(nseg == 0)
+        if(a.n == 0 || a.h == 0 || a.w_ == 0)
             return hipSuccess;
-        const int ntiles = (cout / 16) * ((kdim + 15) / 16);
-        const int groups = (ntiles + 15) / 16;
-        // about 2048 pixels per workgroup, at least 256 workgroups in total when possible
-        int64_t segs = 32;
-        while(segs > 1 && groups * ((nseg + segs - 1) / segs) < 256)
-            segs /= 2;
-        const dim3 grid(unsigned(groups), unsigned((nseg + segs - 1) / segs));
-        const size_t lds = (size_t(3 * 66) * cin + size_t(64) * cout) * sizeof(_Float16);
-        if(lds > 64 * 1024)
-            return hipErrorInvalidValue;
-        hipLaunchKernelGGL(conv_dw_kernel, grid, dim3(256), lds, s, x, up, ca, dz, dw, n, h, w, cin, cout, kdim, int(segs));
-        return hipGetLastError();
+        if(a.cin == 16 && (cout == 16 || cout == 48))
+            return conv_fwd_rows<16, 16, 0, true>(a, max_lds, s, cout / 16);
+        if(a.cin == 32 && cout == 16)
+            return conv_fwd_rows<32, 16, 0, true>(a, max_lds, s);
+        if(a.cin == 32 && (cout == 32 || cout == 96))
+            return conv_fwd_rows<32, 32, 0, true>(a, max_lds, s, cout / 32);
+        if(a.cin == 64 && cout == 32)
+            return conv_fwd_rows<64, 32, 0, true>(a, max_lds, s);
+        if(a.cin == 64 && (cout == 64 || cout == 128))
+            return conv_fwd_rows<64, 64, 0, true>(a, max_lds, s, cout / 64);
+        return hipErrorInvalidValue;
     }
 
-    // ------------------------------------------------------------------ elementwise / reshaping
-    __global__ __launch_bounds__(256) void bias_grad_kernel(const _Float16* __restrict__ dz, float* db, int64_t npx, int c)
-    {
-        // thread t: channel t % c, pixel lane t / c; grid-stride over pixels
-        const int lanesPerBlock = 256 / c;
-        const int ch = threadIdx.x % c, pl = threadIdx.x / c;
-        float sum = 0.0f;
-        if(pl < lanesPerBlock)
-            for(int64_t p = int64_t(blockIdx.x) * lanesPerBlock + pl; p < npx; p += int64_t(gridDim.x) * lanesPerBlock)
-                sum += float(dz[p * c + ch]);
-        __shared__ float red[256];
-        red[threadIdx.x] = pl < lanesPerBlock ? sum : 0.0f;
-        __syncthreads();
-        if(threadIdx.x < c)
-        {
-            float t = 0.0f;
-            for(int i = 0; i < lanesPerBlock; i++)
-                t += red[i * c + threadIdx.x];
-            atomicAdd(db + threadIdx.x, t);
-        }
-    }
-
-    hipError_t launch_bias_grad(const _Float16* dz, float* db, int64_t npx, int c, hipStream_t s)
-    {
-        if(c > 256 || 256 % c != 0)
-            return hipErrorInvalidValue;
-        if(npx == 0)
-            return hipSuccess;
-        const int lanes = 256 / c;
-        int64_t blocks = (npx + lanes * 64 - 1) / (lanes * 64);
-        if(blocks > 1024)
-            blocks = 1024;
-        hipLaunchKernelGGL(bias_grad_kernel, dim3(unsigned(blocks)), dim3(256), 0, s, dz, db, npx, c);
-        return hipGetLastError();
-    }
-
-    __global__ __launch_bounds__(256) void relu_bwd_kernel(const float* dy, const _Float16* y, _Float16* dz, int64_t count)
-    {
-        for(int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < count; i += int64_t(gridDim.x) * blockDim.x)
-            dz[i] = _Float16(float(y[i]) > 0.0f ? dy[i] : 0.0f);
-    }
-
+    // ------------------------------------------------------------------ elementwise
     static unsigned grid_for(int64_t count)
     {
         int64_t b = (count + 255) / 256;
         return unsigned(b > 8192 ? 8192 : (b < 1 ? 1 : b));
     }
 
-    hipError_t launch_relu_bwd(const float* dy, const _Float16* y, _Float16* dz, int64_t count, hipStream_t s)
+    __global__ __launch_bounds__(256) void to_half_kernel(const float* __restrict__ f, _Float16* __restrict__ x, int64_t count)
+    {
+        for(int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < count; i += int64_t(gridDim.x) * blockDim.x)
+            x[i] = _Float16(f[i]);
+    }
+
+    hipError_t launch_to_half(const float* f, _Float16* x, int64_t count, hipStream_t s)
     {
         if(count == 0)
             return hipSuccess;
-        hipLaunchKernelGGL(relu_bwd_kernel, dim3(grid_for(count)), dim3(256), 0, s, dy, y, dz, count);
-        return hipGetLastError();
-    }
-
-    // dx (n, h, w, c) += dy(n, h/2, w/2, c) / 4; one thread per dx element
-    __global__ __launch_bounds__(256) void pool2_bwd_kernel(const float* dy, float* dx, int n, int h, int w, int c)
-    {
-        const int64_t count = int64_t(n) * h * w * c;
-        for(int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < count; i += int64_t(gridDim.x) * blockDim.x)
-        {
-            const int ch = int(i % c);
-            const int64_t q = i / c;
-            const int xx = int(q % w), yy = int((q / w) % h);
-            const int64_t img = q / (int64_t(w) * h);
-            dx[i] += 0.25f * dy[((img * (h / 2) + yy / 2) * (w / 2) + xx / 2) * c + ch];
-        }
-    }
-
-    hipError_t launch_pool2_bwd(const float* dy, float* dx, int n, int h, int w, int c, hipStream_t s)
-    {
-        const int64_t count = int64_t(n) * h * w * c;
-        if(count == 0)
-            return hipSuccess;
-        hipLaunchKernelGGL(pool2_bwd_kernel, dim3(grid_for(count)), dim3(256), 0, s, dy, dx, n, h, w, c);
-        return hipGetLastError();
-    }
-
-    // da (n, h/2, w/2, ca) += sum of the 4 upsampled positions; dskip (n, h, w, cs) += dy[.., ca:]
-    __global__ __launch_bounds__(256) void upcat_bwd_a_kernel(const float* dy, float* da, int n, int h, int w, int ca, int cs)
-    {
-        const int ct = ca + cs, ho = h / 2, wo = w / 2;
-        const int64_t count = int64_t(n) * ho * wo * ca;
-        for(int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < count; i += int64_t(gridDim.x) * blockDim.x)
-        {
-            const int ch = int(i % ca);
-            const int64_t q = i / ca;
-            const int xo = int(q % wo), yo = int((q / wo) % ho);
-            const int64_t img = q / (int64_t(wo) * ho);
-            const float* b = dy + ((img * h + 2 * yo) * w + 2 * xo) * ct + ch;
-            da[i] += (b[0] + b[ct]) + (b[size_t(w) * ct] + b[size_t(w) * ct + ct]);
-        }
-    }
-
-    __global__ __launch_bounds__(256) void upcat_bwd_skip_kernel(const float* dy, float* dskip, int n, int h, int w, int ca, int cs)
-    {
-        const int ct = ca + cs;
-        const int64_t count = int64_t(n) * h * w * cs;
-        for(int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < count; i += int64_t(gridDim.x) * blockDim.x)
-        {
-            const int ch = int(i % cs);
-            const int64_t q = i / cs;
-            dskip[i] += dy[q * ct + ca + ch];
-        }
-    }
-
-    hipError_t launch_upcat_bwd(const float* dy, float* da, float* dskip, int n, int h, int w, int ca, int cs, hipStream_t s)
-    {
-        const int64_t ca_count = int64_t(n) * (h / 2) * (w / 2) * ca;
-        const int64_t cs_count = int64_t(n) * h * w * cs;
-        if(ca_count)
-            hipLaunchKernelGGL(upcat_bwd_a_kernel, dim3(grid_for(ca_count)), dim3(256), 0, s, dy, da, n, h, w, ca, cs);
-        if(cs_count)
-            hipLaunchKernelGGL(upcat_bwd_skip_kernel, dim3(grid_for(cs_count)), dim3(256), 0, s, dy, dskip, n, h, w, ca, cs);
+        hipLaunchKernelGGL(to_half_kernel, dim3(grid_for(count)), dim3(256), 0, s, f, x, count);
         return hipGetLastError();
     }
 
@@ -1022,33 +666,41 @@ namespace isaac_hip
         return hipGetLastError();
     }
 
-    __global__ __launch_bounds__(256) void pack_weights_kernel(const float* master, _Float16* wf, _Float16* wb, int cin, int cout, int kp)
+    // all layers in one launch (blockIdx.y): eleven launches took ten times as long
+    struct PackArgs
     {
-        const int K = 9 * cin;
-        const int64_t nf = int64_t(cout) * kp;
-        const int64_t nb = int64_t(cin) * 9 * cout;
-        for(int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < nf + nb; i += int64_t(gridDim.x) * blockDim.x)
+        PackLayer L[kGradMaxLayers];
+    };
+
+    __global__ __launch_bounds__(256) void pack_weights_kernel(const PackArgs a)
+    {
+        const PackLayer& L = a.L[blockIdx.y];
+        const int K = 9 * L.cin, KB = 9 * L.cout;
+        const int nf = L.cout * L.kp, nb = L.cin * L.kpb;
+        for(int i = int(blockIdx.x * blockDim.x + threadIdx.x); i < nf + nb; i += int(gridDim.x * blockDim.x))
         {
             if(i < nf)
             {
-                const int co = int(i / kp), k = int(i - int64_t(co) * kp);
-                wf[i] = _Float16(k < K ? master[int64_t(co) * K + k] : 0.0f);
+                const int co = i / L.kp, k = i - co * L.kp;
+                L.wf[i] = _Float16(k < K ? L.master[co * K + k] : 0.0f);
             }
             else
             {
-                const int64_t j = i - nf; // [ci][t][co]
-                const int co = int(j % cout);
-                const int t = int((j / cout) % 9);
-                const int ci = int(j / (int64_t(cout) * 9));
-                wb[j] = _Float16(master[(int64_t(co) * 9 + (8 - t)) * cin + ci]);
+                const int j = i - nf, ci = j / L.kpb, k = j - ci * L.kpb; // [ci][t][co]
+                const int t = k / L.cout, co = k - t * L.cout;
+                L.wb[j] = _Float16(k < KB ? L.master[(co * 9 + (8 - t)) * L.cin + ci] : 0.0f);
             }
         }
     }
 
-    hipError_t launch_pack_weights(const float* master, _Float16* wf, _Float16* wb, int cin, int cout, int kp, hipStream_t s)
+    hipError_t launch_pack_weights(const PackLayer* layers, int count, hipStream_t s)
     {
-        const int64_t count = int64_t(cout) * kp + int64_t(cin) * 9 * cout;
-        hipLaunchKernelGGL(pack_weights_kernel, dim3(grid_for(count)), dim3(256), 0, s, master, wf, wb, cin, cout, kp);
+        if(count < 1 || count > kGradMaxLayers)
+            return hipErrorInvalidValue;
+        PackArgs a{};
+        for(int l = 0; l < count; l++)
+            a.L[l] = layers[l];
+        hipLaunchKernelGGL(pack_weights_kernel, dim3(128, unsigned(count)), dim3(256), 0, s, a);
         return hipGetLastError();
     }
 } // namespace isaac_hip

@@ -1,7 +1,6 @@
 // Kernels of the learned occlusion pass: a U-Net over the G-buffer whose 3x3
 // convolutions run as implicit GEMMs on the gfx950 matrix cores
-// (v_mfma_f32_16x16x32_f16 forward, v_mfma_f32_16x16x16_f16 backward: FP16
-// operands, FP32 accumulation).
+// (v_mfma_f32_16x16x32_f16: FP16 operands, FP32 accumulation).
 //
 // Tensors are channels-last: element (n, y, x, c) at ((n*H + y)*W + x)*C + c.
 // Forward convolution weights are [Cout][Kp] FP16 with k = tap*Cin + ci (tap =
@@ -27,7 +26,7 @@ namespace isaac_hip
         int32_t ca; // channels from `up` (a multiple of 4; 0 without `up`)
         const _Float16* w; // [cout][kp]
         const float* bias; // [cout] (forward only)
-        void* y; // forward: _Float16 [n][h][w][cout] = relu(conv + bias) (nullable); backward data: float, +=
+        void* y; // forward: _Float16 [n][h][w][cout] = relu(conv + bias) (nullable); backward data: float
         int32_t n, h, w_, cin, kp; // cin a multiple of 4
         // forward only (launch_conv_fwd), all optional:
         _Float16* pool; // [n][h/2][w/2][cout]: 2x2 average of the FP16 activation (h, w even)
@@ -36,11 +35,11 @@ namespace isaac_hip
         int32_t imgW, imgH;
     };
 
-    // Backward data of a layer: y (FP32, +=) = 3x3 convolution of x with the layer's
-    // flipped, transposed weights ([cin][kp], kp = 9*cout); `cout` here is the
-    // layer's cin, in {16, 32, 48, 64, 96, 128}.  max_lds: the device's LDS bytes per
-    // workgroup (picks the rows per workgroup).
-    hipError_t launch_conv3x3_bwd(const ConvArgs& a, int cout, size_t max_lds, hipStream_t s);
+    // Backward data of a layer: y (FP32 [n][h][w][cout]) = 3x3 convolution of x (the
+    // layer's dz) with its flipped, transposed weights ([cout][kp], kp as for the forward
+    // weights of a.cin channels); `cout` here is the layer's cin and a.cin its cout:
+    // (a.cin, cout) = (16, 16) (16, 48) (32, 16) (32, 32) (32, 96) (64, 32) (64, 64) (64, 128).
+    hipError_t launch_conv_bwd(const ConvArgs& a, int cout, size_t max_lds, hipStream_t s);
 
     // Forward layer y = relu(conv(x) + bias) on v_mfma_f32_16x16x32_f16 for the
     // network's (cin, cout, ca) shapes: (8,16,0) (16,16,0) (16,32,0) (32,32,0)
@@ -49,29 +48,42 @@ namespace isaac_hip
     // head outputs equal launch_pool2 / launch_head_infer applied to the activation.
     hipError_t launch_conv_fwd(const ConvArgs& a, int cout, size_t max_lds, hipStream_t s);
 
-    // dW[co][k] += sum_p dz[p][co] * col(x)[p][k] for k < 9*cin (FP32 atomics into dw,
-    // rows of 9*cin floats: the master weight layout [cout][9][cin])
-    hipError_t launch_conv3x3_dw(
-        const _Float16* x,
-        const _Float16* up,
-        int ca,
-        const _Float16* dz,
-        float* dw,
-        int n,
-        int h,
-        int w,
-        int cin,
-        int cout,
-        hipStream_t s);
-    // db[c] += sum_p dz[p][c]
-    hipError_t launch_bias_grad(const _Float16* dz, float* db, int64_t npx, int c, hipStream_t s);
-    // dz = half(dy * (y > 0))
-    hipError_t launch_relu_bwd(const float* dy, const _Float16* y, _Float16* dz, int64_t count, hipStream_t s);
-    // backward of the 2x2 average pool (h, w even): dx += dy / 4
-    hipError_t launch_pool2_bwd(const float* dy, float* dx, int n, int h, int w, int c, hipStream_t s);
-    // backward of y = concat(nearest-upsample(a), skip): da += 2x2 sums of dy[.., :ca],
-    // dskip += dy[.., ca:]
-    hipError_t launch_upcat_bwd(const float* dy, float* da, float* dskip, int n, int h, int w, int ca, int cs, hipStream_t s);
+    // Where the gradient of a layer's output comes from
+    enum DyMode : int32_t
+    {
+        kDyPlain = 0, // g [n][h][w][gStride], channels gOff ..
+        kDyUpsampled = 1, // g [n][2h][2w][gStride], channels gOff ..: the sum of the 2x2 positions that read it
+        kDySkipAndPool = 2 // as kDyPlain, plus gPool [n][h/2][w/2][cout] / 4 (the 2x2 average pool's gradient)
+    };
+    // One layer of the weight gradient: dz = half(dy * (act > 0)) is formed and stored, and
+    // dw / db are the sums over all pixels (launch_conv_grad, then launch_grad_sum)
+    struct GradLayer
+    {
+        const _Float16* x; // the layer's input, as in ConvArgs
+        const _Float16* up;
+        int32_t ca, cin, cout; // cout 16, 32 or 64
+        const _Float16* act; // the layer's output [n][h][w][cout]
+        int32_t dyMode;
+        const float* g;
+        int32_t gStride, gOff; // multiples of 4
+        const float* gPool;
+        _Float16* dz; // out: [n][h][w][cout]
+        float* partial; // grad_shape(...).partial floats
+        float* partialBias; // grad_shape(...).splits * cout floats
+        float* dw; // out: [cout][9][cin] (the master weight layout)
+        float* db; // out: [cout]
+        int32_t n, h, w;
+    };
+    struct GradShape
+    {
+        int32_t ct, groups, splits; // 16-channel input blocks per workgroup, groups of them, pixel splits
+        size_t partial; // floats
+    };
+    constexpr int kGradMaxLayers = 11;
+    GradShape grad_shape(int cin, int cout, int n, int h, int w);
+    hipError_t launch_conv_grad(const GradLayer& L, hipStream_t s);
+    // dw and db of all layers from their partial sums
+    hipError_t launch_grad_sum(const GradLayer* layers, int count, hipStream_t s);
 
     // network input from a G-buffer window: 8 channels (depth / scale or 0, background
     // flag, normal xyz, 0, 0, 0); pixels outside the image are background.  With `ao`
@@ -121,14 +133,16 @@ namespace isaac_hip
         float c2,
         float gscale,
         hipStream_t s);
-    // FP16 forward weights [cout][kp] and flipped-transposed backward weights
-    // [cin][9*cout] (w'[ci][t][co] = w[co][8-t][ci]) from FP32 master [cout][9][cin]
-    hipError_t launch_pack_weights(
-        const float* master,
-        _Float16* wf,
-        _Float16* wb,
-        int cin,
-        int cout,
-        int kp,
-        hipStream_t s);
+    // Of every layer: FP16 forward weights [cout][kp] and flipped-transposed backward
+    // weights [cin][kpb] (w'[ci][t*cout + co] = w[co][8-t][ci]) from FP32 master
+    // [cout][9][cin], both rows padded with zeros (kp, kpb: multiples of 32)
+    struct PackLayer
+    {
+        const float* master;
+        _Float16 *wf, *wb;
+        int32_t cin, cout, kp, kpb;
+    };
+    hipError_t launch_pack_weights(const PackLayer* layers, int count, hipStream_t s);
+    // x (FP16) = f, `count` values
+    hipError_t launch_to_half(const float* f, _Float16* x, int64_t count, hipStream_t s);
 } // namespace isaac_hip

@@ -52,6 +52,9 @@ namespace isaac_hip
         float* g[kNumLayers] = {};
         float *gp0 = nullptr, *gp1 = nullptr, *gp2 = nullptr, *gc2 = nullptr, *gc1 = nullptr, *gc0 = nullptr;
         _Float16* dz = nullptr;
+        // partial sums of the weight and bias gradients, all layers
+        float* partial = nullptr;
+        size_t partialOff[kNumLayers] = {}, partialBiasOff[kNumLayers] = {};
 
         void release()
         {
@@ -97,7 +100,8 @@ namespace isaac_hip
             chk(get(origins, size_t(2) * n_));
             if(grads_)
             {
-                for(int i = 0; i < kNumLayers; i++)
+                // outputs of one reader; those read by a decoder come from gc* and gp*
+                for(int i : {0, 2, 4, 6, 10})
                     chk(get(g[i], lvl[kLevel[i]] * kLayers[i].cout));
                 chk(get(gp0, half * 16));
                 chk(get(gp1, quarter * 32));
@@ -106,6 +110,17 @@ namespace isaac_hip
                 chk(get(gc1, half * 96));
                 chk(get(gc0, full * 48));
                 chk(get(dz, full * 16));
+                // (a smaller batch splits into no more partial sums)
+                size_t off = 0;
+                for(int i = 0; i < kNumLayers; i++)
+                {
+                    const GradShape s = grad_shape(kLayers[i].cin, kLayers[i].cout, n_, h_ >> kLevel[i], w_ >> kLevel[i]);
+                    partialOff[i] = off;
+                    off += s.partial;
+                    partialBiasOff[i] = off;
+                    off += size_t(s.splits) * kLayers[i].cout;
+                }
+                chk(get(partial, off));
             }
             if(e != hipSuccess)
             {
@@ -194,7 +209,7 @@ namespace isaac_hip
             for(int i = 0; i < kNumLayers && e == hipSuccess; i++)
             {
                 chk(hipMalloc(&net->wf[i], size_t(kLayers[i].cout) * net->kp[i] * sizeof(_Float16)));
-                chk(hipMalloc(&net->wb[i], size_t(kLayers[i].cin) * 9 * kLayers[i].cout * sizeof(_Float16)));
+                chk(hipMalloc(&net->wb[i], size_t(kLayers[i].cin) * kpad(kLayers[i].cout) * sizeof(_Float16)));
             }
             if(e != hipSuccess)
             {
@@ -207,14 +222,11 @@ namespace isaac_hip
 
         hipError_t pack(AoNet* net, hipStream_t s)
         {
+            PackLayer p[kNumLayers];
             for(int i = 0; i < kNumLayers; i++)
-            {
-                hipError_t e = launch_pack_weights(net->master + net->woff[i], net->wf[i], net->wb[i], kLayers[i].cin,
-                                                   kLayers[i].cout, net->kp[i], s);
-                if(e != hipSuccess)
-                    return e;
-            }
-            return hipSuccess;
+                p[i] = PackLayer{net->master + net->woff[i], net->wf[i], net->wb[i], kLayers[i].cin, kLayers[i].cout, net->kp[i],
+                                 kpad(kLayers[i].cout)};
+            return launch_pack_weights(p, kNumLayers, s);
         }
 
         // input of a decoder layer: upsampled `up` (ca channels) followed by the skip tensor
@@ -298,42 +310,32 @@ namespace isaac_hip
             return launch_conv_fwd(a, kLayers[10].cout, net->maxLds, s);
         }
 
-        // backward of layer i given ws.g[i] (gradient wrt its ReLU output): weight and
-        // bias gradients, and (when gin != nullptr) += gradient wrt its input
-        hipError_t layer_bwd(
-            AoNet* net,
-            AoWorkspace& ws,
-            int i,
-            const _Float16* in,
-            float* gin,
-            int n,
-            int h,
-            int w,
-            hipStream_t s,
-            const _Float16* up = nullptr,
-            int ca = 0)
+        // backward of layer L.i: its dz and the partial sums of its weight and bias
+        // gradients, then (gin != nullptr) the gradient wrt its input
+        hipError_t layer_bwd(AoNet* net, AoWorkspace& ws, int i, GradLayer& L, float* gin, hipStream_t s)
         {
-            const int cin = kLayers[i].cin, cout = kLayers[i].cout;
-            const int64_t npx = int64_t(n) * h * w;
             hipError_t e;
-            AOCHK(launch_relu_bwd(ws.g[i], ws.act[i], ws.dz, npx * cout, s));
-            AOCHK(launch_conv3x3_dw(in, up, ca, ws.dz, net->grad + net->woff[i], n, h, w, cin, cout, s));
-            AOCHK(launch_bias_grad(ws.dz, net->grad + net->boff[i], npx, cout, s));
+            L.cin = kLayers[i].cin;
+            L.cout = kLayers[i].cout;
+            L.act = ws.act[i];
+            L.dz = ws.dz;
+            L.partial = ws.partial + ws.partialOff[i];
+            L.partialBias = ws.partial + ws.partialBiasOff[i];
+            L.dw = net->grad + net->woff[i];
+            L.db = net->grad + net->boff[i];
+            AOCHK(launch_conv_grad(L, s));
             if(gin)
             {
                 ConvArgs a{};
                 a.x = ws.dz;
-                a.up = nullptr;
-                a.ca = 0;
                 a.w = net->wb[i];
-                a.bias = nullptr;
                 a.y = gin;
-                a.n = n;
-                a.h = h;
-                a.w_ = w;
-                a.cin = cout;
-                a.kp = 9 * cout;
-                AOCHK(launch_conv3x3_bwd(a, cin, net->maxLds, s));
+                a.n = L.n;
+                a.h = L.h;
+                a.w_ = L.w;
+                a.cin = L.cout;
+                a.kp = kpad(L.cout);
+                AOCHK(launch_conv_bwd(a, L.cin, net->maxLds, s));
             }
             return hipSuccess;
         }
@@ -343,42 +345,46 @@ namespace isaac_hip
             return launch_fill_u32(reinterpret_cast<uint32_t*>(p), 0u, count, s);
         }
 
-        // loss and parameter gradients (into net->grad, zeroed first) of ws over n images
+        // loss and parameter gradients (into net->grad) of ws over n images; every other
+        // buffer is written before it is read
         hipError_t backward(AoNet* net, AoWorkspace& ws, int n, int h, int w, hipStream_t s)
         {
-            const size_t full = size_t(n) * h * w, half = full / 4, quarter = full / 16, eighth = full / 64;
-            const size_t lvl[4] = {full, half, quarter, eighth};
-            const int h1 = h / 2, w1 = w / 2, h2 = h / 4, w2 = w / 4, h3 = h / 8, w3 = w / 8;
+            const size_t full = size_t(n) * h * w;
             hipError_t e;
-            AOCHK(zero(net->grad, size_t(net->nparams), s));
+            AOCHK(zero(net->grad + net->headOff, kHeadIn + 1, s));
             AOCHK(zero(ws.loss, 1, s));
-            for(int i = 0; i < kNumLayers; i++)
-                AOCHK(zero(ws.g[i], lvl[kLevel[i]] * kLayers[i].cout, s));
-            AOCHK(zero(ws.gp0, half * 16, s));
-            AOCHK(zero(ws.gp1, quarter * 32, s));
-            AOCHK(zero(ws.gp2, eighth * 64, s));
-            AOCHK(zero(ws.gc2, quarter * 128, s));
-            AOCHK(zero(ws.gc1, half * 96, s));
-            AOCHK(zero(ws.gc0, full * 48, s));
             AOCHK(launch_head_train(ws.act[10], net->master + net->headOff, ws.target, ws.loss, net->grad + net->headOff,
                                     ws.g[10], ws.out, int64_t(full), s));
-            AOCHK(layer_bwd(net, ws, 10, ws.act[1], ws.gc0, n, h, w, s, ws.act[9], 32));
-            AOCHK(launch_upcat_bwd(ws.gc0, ws.g[9], ws.g[1], n, h, w, 32, 16, s));
-            AOCHK(layer_bwd(net, ws, 9, ws.act[3], ws.gc1, n, h1, w1, s, ws.act[8], 64));
-            AOCHK(launch_upcat_bwd(ws.gc1, ws.g[8], ws.g[3], n, h1, w1, 64, 32, s));
-            AOCHK(layer_bwd(net, ws, 8, ws.act[5], ws.gc2, n, h2, w2, s, ws.act[7], 64));
-            AOCHK(launch_upcat_bwd(ws.gc2, ws.g[7], ws.g[5], n, h2, w2, 64, 64, s));
-            AOCHK(layer_bwd(net, ws, 7, ws.act[6], ws.g[6], n, h3, w3, s));
-            AOCHK(layer_bwd(net, ws, 6, ws.p2, ws.gp2, n, h3, w3, s));
-            AOCHK(launch_pool2_bwd(ws.gp2, ws.g[5], n, h2, w2, 64, s));
-            AOCHK(layer_bwd(net, ws, 5, ws.act[4], ws.g[4], n, h2, w2, s));
-            AOCHK(layer_bwd(net, ws, 4, ws.p1, ws.gp1, n, h2, w2, s));
-            AOCHK(launch_pool2_bwd(ws.gp1, ws.g[3], n, h1, w1, 32, s));
-            AOCHK(layer_bwd(net, ws, 3, ws.act[2], ws.g[2], n, h1, w1, s));
-            AOCHK(layer_bwd(net, ws, 2, ws.p0, ws.gp0, n, h1, w1, s));
-            AOCHK(launch_pool2_bwd(ws.gp0, ws.g[1], n, h, w, 16, s));
-            AOCHK(layer_bwd(net, ws, 1, ws.act[0], ws.g[0], n, h, w, s));
-            AOCHK(layer_bwd(net, ws, 0, ws.x0, nullptr, n, h, w, s));
+            GradLayer L[kNumLayers];
+            auto layer = [&](int i, const _Float16* in, float* gin, const _Float16* up, int ca, int mode, const float* g, int stride,
+                             int off, const float* pool)
+            {
+                L[i] = GradLayer{};
+                L[i].x = in;
+                L[i].up = up;
+                L[i].ca = ca;
+                L[i].dyMode = mode;
+                L[i].g = g;
+                L[i].gStride = stride;
+                L[i].gOff = off;
+                L[i].gPool = pool;
+                L[i].n = n;
+                L[i].h = h >> kLevel[i];
+                L[i].w = w >> kLevel[i];
+                return layer_bwd(net, ws, i, L[i], gin, s);
+            };
+            AOCHK(layer(10, ws.act[1], ws.gc0, ws.act[9], 32, kDyPlain, ws.g[10], 16, 0, nullptr));
+            AOCHK(layer(9, ws.act[3], ws.gc1, ws.act[8], 64, kDyUpsampled, ws.gc0, 48, 0, nullptr));
+            AOCHK(layer(8, ws.act[5], ws.gc2, ws.act[7], 64, kDyUpsampled, ws.gc1, 96, 0, nullptr));
+            AOCHK(layer(7, ws.act[6], ws.g[6], nullptr, 0, kDyUpsampled, ws.gc2, 128, 0, nullptr));
+            AOCHK(layer(6, ws.p2, ws.gp2, nullptr, 0, kDyPlain, ws.g[6], 64, 0, nullptr));
+            AOCHK(layer(5, ws.act[4], ws.g[4], nullptr, 0, kDySkipAndPool, ws.gc2, 128, 64, ws.gp2));
+            AOCHK(layer(4, ws.p1, ws.gp1, nullptr, 0, kDyPlain, ws.g[4], 64, 0, nullptr));
+            AOCHK(layer(3, ws.act[2], ws.g[2], nullptr, 0, kDySkipAndPool, ws.gc1, 96, 64, ws.gp1));
+            AOCHK(layer(2, ws.p0, ws.gp0, nullptr, 0, kDyPlain, ws.g[2], 32, 0, nullptr));
+            AOCHK(layer(1, ws.act[0], ws.g[0], nullptr, 0, kDySkipAndPool, ws.gc0, 48, 32, ws.gp0));
+            AOCHK(layer(0, ws.x0, nullptr, nullptr, 0, kDyPlain, ws.g[0], 16, 0, nullptr));
+            AOCHK(launch_grad_sum(L, kNumLayers, s));
             return hipSuccess;
 #undef AOCHK
         }
@@ -386,10 +392,10 @@ namespace isaac_hip
         int upload_features(isaac_hip_ctx* c, AoWorkspace& ws, int n, int h, int w, const float* features, const float* target)
         {
             const size_t full = size_t(n) * h * w;
-            std::vector<_Float16> x(full * kFeatures);
-            for(size_t i = 0; i < x.size(); i++)
-                x[i] = _Float16(features[i]);
-            HIPCHK(c, hipMemcpyAsync(ws.x0, x.data(), x.size() * sizeof(_Float16), hipMemcpyHostToDevice, c->stream));
+            // as floats into a gradient buffer (written by no kernel before the backward pass), rounded
+            // to half there
+            HIPCHK(c, hipMemcpyAsync(ws.gc0, features, full * kFeatures * sizeof(float), hipMemcpyHostToDevice, c->stream));
+            HIPCHK(c, launch_to_half(ws.gc0, ws.x0, int64_t(full * kFeatures), c->stream));
             if(target)
                 HIPCHK(c, hipMemcpyAsync(ws.target, target, full * sizeof(float), hipMemcpyHostToDevice, c->stream));
             HIPCHK(c, hipStreamSynchronize(c->stream));
