@@ -309,7 +309,7 @@ extern "C"
      * No counterpart in the reference (one frame of one sub-volume per drawCallBack,
      * lib/isaac.hpp:2140-2543).  A batch renders frames = contexts x views, all at
      * width x height: one persistent march launch over every 16x16 tile of every
-     * frame (workgroups pop chunks of tiles from a global counter), one occlusion
+     * frame (waves pop tiles from one work queue per XCD), one occlusion
      * pass over all frames (plain SSAO, or the learned pass of context 0, evaluated
      * over several frames at a time) and one shading launch.  Each context is one
      * sub-volume in the brick form with update_buffers done, and all contexts share
@@ -334,7 +334,7 @@ extern "C"
     };
     enum isaac_hip_batch_tuning_key
     {
-        ISAAC_HIP_BATCH_TUNE_CHUNK = 0, /* tiles per pop of the work counter (default 4) */
+        ISAAC_HIP_BATCH_TUNE_CHUNK = 0, /* 8x8-pixel tiles a wave takes per pop of its work queue (default 1) */
         ISAAC_HIP_BATCH_TUNE_GROUPS_PER_CU = 1, /* persistent workgroups per compute unit (default 4) */
         ISAAC_HIP_BATCH_TUNE_AO_CHUNK = 2 /* frames per evaluation of the learned occlusion network (default 16) */
     };

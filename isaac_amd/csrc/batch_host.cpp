@@ -25,7 +25,7 @@ struct isaac_hip_batch
     isaac_hip::AoWorkspace* aoWs = nullptr; // learned occlusion activations of this batch
     int W = 0, H = 0, nviews = 0, nframes = 0;
     int tilesPerFrame = 0;
-    int chunk = 4, groupsPerCU = 4, aoChunk = 16;
+    int chunk = 1, groupsPerCU = 4, aoChunk = 16;
     int numCU = 256;
     // host copies of the per-frame parameter blocks
     std::vector<FrameParams> hF;
@@ -36,7 +36,7 @@ struct isaac_hip_batch
     FrameParams* dF = nullptr;
     PostParams* dQ = nullptr;
     ParticleParams* dP = nullptr;
-    uint32_t* dTileStart = nullptr;
+    uint32_t* dOrder = nullptr;
     uint32_t* dCounter = nullptr;
     float* dInvScale = nullptr;
     uint32_t* color = nullptr;
@@ -77,14 +77,14 @@ namespace
 
     void free_frames(isaac_hip_batch* b)
     {
-        void* bufs[] = {b->dF, b->dQ, b->dP, b->dTileStart, b->dInvScale, b->color, b->depth, b->normal, b->ao, b->volColor};
+        void* bufs[] = {b->dF, b->dQ, b->dP, b->dOrder, b->dInvScale, b->color, b->depth, b->normal, b->ao, b->volColor};
         for(void* p : bufs)
             if(p)
                 (void) hipFree(p);
         b->dF = nullptr;
         b->dQ = nullptr;
         b->dP = nullptr;
-        b->dTileStart = nullptr;
+        b->dOrder = nullptr;
         b->dInvScale = nullptr;
         b->color = nullptr;
         b->depth = nullptr;
@@ -115,7 +115,7 @@ namespace
         BCHK(b, hipMalloc(&b->dF, sizeof(FrameParams) * nframes));
         BCHK(b, hipMalloc(&b->dQ, sizeof(PostParams) * nframes));
         BCHK(b, hipMalloc(&b->dP, sizeof(ParticleParams) * nframes));
-        BCHK(b, hipMalloc(&b->dTileStart, sizeof(uint32_t) * (nframes + 1)));
+        BCHK(b, hipMalloc(&b->dOrder, sizeof(uint32_t) * nframes));
         BCHK(b, hipMalloc(&b->dInvScale, sizeof(float) * nframes));
         BCHK(b, hipMalloc(&b->color, px * 4));
         BCHK(b, hipMalloc(&b->depth, px * 4));
@@ -130,16 +130,17 @@ namespace
     // the sequence of one batched frame set: persistent march, occlusion, shading
     int enqueue(isaac_hip_batch* b)
     {
-        BCHK(b, launch_fill_u32(b->dCounter, 0u, 1, b->stream));
+        BCHK(b, launch_fill_u32(b->dCounter, 0u, kMarchQueues * kMarchQueueStride, b->stream));
         BatchParams B{};
         B.frames = b->dF;
         B.posts = b->dQ;
         B.parts = b->dP;
-        B.tileStart = b->dTileStart;
+        B.order = b->dOrder;
         B.nframes = b->nframes;
-        B.ntiles = uint32_t(b->tilesPerFrame) * uint32_t(b->nframes);
+        B.tilesX = (b->W + 15) / 16;
+        B.tilesY = (b->H + 15) / 16;
         B.chunk = b->chunk;
-        B.counter = b->dCounter;
+        B.counters = b->dCounter;
         const int grid = std::max(1, b->numCU * b->groupsPerCU);
         BCHK(b, launch_batch_march(B, b->dtype, b->linear, b->sig, b->lutLds, grid, b->stream));
         if(b->aoOn)
@@ -178,7 +179,7 @@ extern "C"
         b->ctxEv.assign(size_t(n), nullptr);
         b->gen.assign(size_t(n), 0);
         bool ok = hipSetDevice(b->device) == hipSuccess && hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking) == hipSuccess
-                  && hipMalloc(&b->dCounter, 64) == hipSuccess && hipEventCreate(&b->ev[0]) == hipSuccess
+                  && hipMalloc(&b->dCounter, sizeof(uint32_t) * kMarchQueues * kMarchQueueStride) == hipSuccess && hipEventCreate(&b->ev[0]) == hipSuccess
                   && hipEventCreate(&b->ev[1]) == hipSuccess;
         for(int i = 0; ok && i < n; i++)
             ok = hipEventCreateWithFlags(&b->ctxEv[i], hipEventDisableTiming) == hipSuccess;
@@ -315,13 +316,21 @@ extern "C"
                 return bfail(b, ISAAC_HIP_ERR_ARG,
                              "context " + std::to_string(f / nviews) + ": bound sources differ from context 0's");
         }
-        std::vector<uint32_t> ts(nframes + 1);
-        for(int f = 0; f <= nframes; f++)
-            ts[f] = uint32_t(f) * uint32_t(b->tilesPerFrame);
+        // the march starts the frames of the largest sub-volumes first: the rays that are left at its
+        // end are then the short ones
+        std::vector<uint32_t> order(nframes);
+        for(int f = 0; f < nframes; f++)
+            order[f] = uint32_t(f);
+        auto voxels = [&](uint32_t f)
+        {
+            const isaac_hip_ctx* c = b->ctx[f / uint32_t(nviews)];
+            return c->local[0] * c->local[1] * c->local[2];
+        };
+        std::stable_sort(order.begin(), order.end(), [&](uint32_t x, uint32_t y) { return voxels(x) > voxels(y); });
         BCHK(b, hipMemcpyAsync(b->dF, b->hF.data(), sizeof(FrameParams) * nframes, hipMemcpyHostToDevice, b->stream));
         BCHK(b, hipMemcpyAsync(b->dQ, b->hQ.data(), sizeof(PostParams) * nframes, hipMemcpyHostToDevice, b->stream));
         BCHK(b, hipMemcpyAsync(b->dP, b->hP.data(), sizeof(ParticleParams) * nframes, hipMemcpyHostToDevice, b->stream));
-        BCHK(b, hipMemcpyAsync(b->dTileStart, ts.data(), sizeof(uint32_t) * (nframes + 1), hipMemcpyHostToDevice, b->stream));
+        BCHK(b, hipMemcpyAsync(b->dOrder, order.data(), sizeof(uint32_t) * nframes, hipMemcpyHostToDevice, b->stream));
         BCHK(b, hipMemcpyAsync(b->dInvScale, b->hInvScale.data(), sizeof(float) * nframes, hipMemcpyHostToDevice, b->stream));
         BCHK(b, hipStreamSynchronize(b->stream));
         if(nframes != b->nframes || nviews != b->nviews)

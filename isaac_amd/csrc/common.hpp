@@ -160,6 +160,7 @@ namespace isaac_hip
         int32_t nsrc;
         int32_t dtype; // ISAAC_HIP_F32 / F16 / BF16
         int32_t nbx, nby, nbz;
+        int32_t off32; // every source's bricks span < 4 GiB: 32-bit byte offsets
         float invTotalWeight; // 1 / sum of volume-source weights (0 if that sum is 0)
         int32_t T;
         const float4* luts; // all sources' transfer functions, T entries each
@@ -178,12 +179,14 @@ namespace isaac_hip
         const struct FrameParams* frames;
         const PostParams* posts;
         const struct ParticleParams* parts;
-        const uint32_t* tileStart; // nframes + 1 prefix sums of 16x16 tiles per frame
+        const uint32_t* order; // frames in the order they are started in
         int32_t nframes;
-        uint32_t ntiles;
-        int32_t chunk; // tiles per pop of the work counter
-        uint32_t* counter; // zeroed before the launch
+        int32_t tilesX, tilesY; // 16x16 tiles of every frame (all of one size)
+        int32_t chunk; // 8x8 quarters of tiles per pop of a work counter
+        uint32_t* counters; // kMarchQueues counters, kMarchQueueStride words apart, zeroed before the launch
     };
+    // work queues of a persistent march, one per XCD
+    constexpr uint32_t kMarchQueues = 8, kMarchQueueStride = 16;
 
     struct ParticleSourceDev
     {

@@ -732,6 +732,10 @@ namespace isaac_hip
                 B.chain = v.desc.persistent ? c->chain[s] : ChainDesc{};
                 B.lutSlot = s;
             }
+            Q.off32 = 1;
+            for(int s = 0; s < nvf; s++)
+                if(c->vols[s].bricked && c->vols[s].brickBytes > 0xffffffffull)
+                    Q.off32 = 0;
             // the enabled sources' transfer functions are staged in LDS (64 KiB per workgroup)
             if(size_t(Q.nsrc) * size_t(T) * sizeof(float4) > 64 * 1024)
                 return fail(c, ISAAC_HIP_ERR_UNSUPPORTED, "brick form: enabled sources x transfer size above 4096 entries");

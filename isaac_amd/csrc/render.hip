@@ -22,92 +22,6 @@ namespace isaac_hip
 #include "dither_tables.inc"
 #undef DITHER_TABLE
 
-    // ------------------------------------------------------------------ functor chain
-    // pow stays out of line: inlined, its ~70 instructions per component and
-    // functor slot made up most of the code of the marches that evaluate the
-    // chain per sample (rarely used, and the call is only taken for it).
-    __device__ __noinline__ float chain_pow(float a, float b)
-    {
-        return powf(a, b);
-    }
-
-    // f2(f1(f0(v,p0),p1),p2).x with the feature dimension propagating
-    // (lib/isaac/isaac_functor_chain.hpp:96-108, lib/isaac/isaac_functors.hpp:42-183).
-    __device__ inline float apply_chain(const ChainDesc& c, float v0, float v1, float v2, float v3, int n)
-    {
-        float v[4] = {v0, v1, v2, v3};
-#pragma unroll
-        for(int k = 0; k < kMaxFunctors; k++)
-        {
-            const int op = c.op[k];
-            if(op == OP_ADD)
-            {
-#pragma unroll
-                for(int i = 0; i < 4; i++)
-                    if(i < n)
-                        v[i] = v[i] + c.p[k][i];
-            }
-            else if(op == OP_MUL)
-            {
-#pragma unroll
-                for(int i = 0; i < 4; i++)
-                    if(i < n)
-                        v[i] = v[i] * c.p[k][i];
-            }
-            else if(op == OP_LENGTH)
-            {
-                float d;
-                if(n == 1)
-                    d = v[0] * v[0];
-                else if(n == 2)
-                    d = v[0] * v[0] + v[1] * v[1];
-                else if(n == 3)
-                    d = v[0] * v[0] + v[1] * v[1] + v[2] * v[2];
-                else
-                    d = (v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]);
-                v[0] = sqrtf(d);
-                n = 1;
-            }
-            else if(op == OP_POW)
-            {
-#pragma unroll
-                for(int i = 0; i < 4; i++)
-                    if(i < n)
-                        v[i] = chain_pow(v[i], c.p[k][i]);
-            }
-            else if(op == OP_SUM)
-            {
-                float s = 0.0f;
-#pragma unroll
-                for(int i = 0; i < 4; i++)
-                    if(i < n)
-                        s = s + v[i];
-                v[0] = s;
-                n = 1;
-            }
-        }
-        return v[0];
-    }
-
-    // x / d for a divisor fixed per launch, with r = RN(1/d) computed once on the
-    // host: x*r plus one fma residual correction (Markstein's correction), three
-    // instructions instead of the correctly rounded division sequence.  Equal to the
-    // IEEE quotient for finite operands away from overflow and underflow
-    // (tests/cpp/divq_check.c: 0 of 2e8 seeded quotients differ, a quarter of them
-    // next to rounding boundaries; for d = 255 every x in [0, 256],
-    // tests/cpp/div255_check.c).
-    __device__ inline float div_by(float x, float d, float r)
-    {
-        const float q0 = x * r;
-        const float e = __builtin_fmaf(-q0, d, x);
-        return __builtin_fmaf(e, r, q0);
-    }
-
-    __device__ inline int tf_index(float v, int T)
-    {
-        return tf_index_of(v * float(T), T);
-    }
-
     // ------------------------------------------------------------------ classification
     __device__ inline uint32_t dither_b4(int mode, int x, int y, int z, float r, float g, float b, float a)
     {
@@ -466,713 +380,6 @@ namespace isaac_hip
         shade_body(F, xcd_tile(F, blockIdx.x));
     }
 
-    // ------------------------------------------------------------------ precision form
-    // Field bricks (FP32 / FP16 / BF16 + FP32 scale) rendered with
-    // post-classification: interpolate the raw field, then functor chain and
-    // transfer function per sample (the semantics of the reference's legacy
-    // renderer, lib/isaac/isaac_volume_kernel.hpp:101-168), blended across
-    // sources as the classification pass does (lib/isaac/isaac_common_kernel.hpp:574-612)
-    // but without the RGBA8 quantisation.  The ray setup (pixelToRay + clipRay)
-    // runs in binary64; interpolation and compositing accumulate in binary32.
-
-    struct RayD
-    {
-        double dir[3], start[3];
-        double startDepth, endDepth;
-        bool isClipped;
-        double clipN[3];
-    };
-
-    __device__ inline bool ray_setup_d(const FrameParams& F, const PostParams& Q, int px, int py, RayD& r)
-    {
-        const double vx = double(px) / double(F.fbW) * 2.0 - 1.0;
-        const double vy = double(py) / double(F.fbH) * 2.0 - 1.0;
-        double s[4], e[4];
-        for(int k = 0; k < 4; k++)
-        {
-            const double s0 = Q.invd[0 * 4 + k] * vx + Q.invd[1 * 4 + k] * vy;
-            s[k] = s0 + (Q.invd[3 * 4 + k] - Q.invd[2 * 4 + k]);
-            e[k] = s0 + (Q.invd[3 * 4 + k] + Q.invd[2 * 4 + k]);
-        }
-        double d[3], len2 = 0.0;
-        for(int k = 0; k < 3; k++)
-        {
-            r.start[k] = s[k] / s[3] * Q.maxSized;
-            d[k] = e[k] / e[3] * Q.maxSized - r.start[k];
-            len2 += d[k] * d[k];
-        }
-        const double il = 1.0 / sqrt(len2);
-        double bmin[3], bmax[3];
-        for(int k = 0; k < 3; k++)
-        {
-            r.dir[k] = d[k] * il;
-            r.start[k] += double(F.off[k]);
-            bmin[k] = (double(F.bbMin[k]) - r.start[k]) / r.dir[k];
-            bmax[k] = (double(F.bbMax[k]) - r.start[k]) / r.dir[k];
-            if(bmax[k] < bmin[k])
-            {
-                const double t = bmax[k];
-                bmax[k] = bmin[k];
-                bmin[k] = t;
-            }
-            r.clipN[k] = 0.0;
-        }
-        r.isClipped = false;
-        r.startDepth = fmax(bmin[0], fmax(bmin[1], bmin[2]));
-        r.endDepth = fmin(bmax[0], fmin(bmax[1], bmax[2]));
-        for(int k = 0; k < 3; k++)
-        {
-            const double sgn = (r.dir[k] > 0.0) ? 1.0 : ((r.dir[k] < 0.0) ? -1.0 : 0.0);
-            if(bmin[k] == r.startDepth && ((F.outerLow[k] && sgn + 1.0 != 0.0) || (F.outerHigh[k] && sgn - 1.0 != 0.0)))
-            {
-                r.isClipped = true;
-                r.clipN[k] = sgn;
-            }
-        }
-        for(int i = 0; i < F.nclip; i++)
-        {
-            double dn = 0.0, pn = 0.0, sn = 0.0;
-            for(int k = 0; k < 3; k++)
-            {
-                dn += r.dir[k] * double(F.cnorm[i][k]);
-                pn += Q.cposd[i][k] * double(F.cnorm[i][k]);
-                sn += r.start[k] * double(F.cnorm[i][k]);
-            }
-            const double t = (pn - sn) / dn;
-            if(dn > 0.0)
-            {
-                if(r.endDepth < t)
-                    return false;
-                if(r.startDepth <= t)
-                {
-                    for(int k = 0; k < 3; k++)
-                        r.clipN[k] = double(F.cnorm[i][k]);
-                    r.isClipped = true;
-                    r.startDepth = t;
-                }
-            }
-            else
-            {
-                if(r.startDepth > t)
-                    return false;
-                if(r.endDepth > t)
-                    r.endDepth = t;
-            }
-        }
-        r.startDepth = fmax(r.startDepth, double(kZNear));
-        return !(r.startDepth > r.endDepth || isinf(r.startDepth) || isinf(r.endDepth));
-    }
-
-    __device__ inline float half_lo(uint32_t v)
-    {
-        return __half2float(__ushort_as_half((unsigned short) (v & 0xffffu)));
-    }
-    __device__ inline float half_hi(uint32_t v)
-    {
-        return __half2float(__ushort_as_half((unsigned short) (v >> 16)));
-    }
-
-    // Tap geometry of one sample position, shared by every source (all sources
-    // of a rank have the local box's brick grid).  Sampler LINEAR|NEAREST with
-    // CLAMP addressing (lib/isaac/isaac_texture.hpp:182-259): the taps of a sample
-    // all come from the brick holding its clamped (x0, y0, z0) tap; where x1 = x0
-    // (clamped at the edge) the second element of each pair gets weight 0.
-    struct BrickTaps
-    {
-        uint32_t brick; // brick index
-        uint32_t i00, i10, i01, i11; // pair index in a component block of rows (y0,z0) (y1,z0) (y0,z1) (y1,z1)
-        // trilinear weights of the corners (x, y, z) = 000 001 010 011 100 101 110 111,
-        // shared by every component of every source at this position; where both x
-        // taps are texel x0 (CLAMP at the x edge) the x1 corners weigh 0
-        float w[8];
-    };
-
-    template<bool LINEAR>
-    __device__ inline BrickTaps brick_taps(const PostParams& Q, int X, int Y, int Z, float px, float py, float pz)
-    {
-        BrickTaps t;
-        if(!LINEAR)
-        {
-            const uint32_t x = iclamp(int(px), 0, X - 1), y = iclamp(int(py), 0, Y - 1), z = iclamp(int(pz), 0, Z - 1);
-            t.brick = ((z >> 3) * uint32_t(Q.nby) + (y >> 3)) * uint32_t(Q.nbx) + (x >> 3);
-            t.i00 = ((z & 7) * 9 + (y & 7)) * 8 + (x & 7);
-            t.i10 = t.i01 = t.i11 = t.i00;
-            return t;
-        }
-        const float cx = px - 0.5f, cy = py - 0.5f, cz = pz - 0.5f;
-        const float flx = floorf(cx), fly = floorf(cy), flz = floorf(cz);
-        const int bx = int(flx), by = int(fly), bz = int(flz);
-        const uint32_t x0 = iclamp(bx, 0, X - 1), x1 = iclamp(bx + 1, 0, X - 1);
-        const uint32_t y0 = iclamp(by, 0, Y - 1), y1 = iclamp(by + 1, 0, Y - 1);
-        const uint32_t z0 = iclamp(bz, 0, Z - 1), z1 = iclamp(bz + 1, 0, Z - 1);
-        const uint32_t Bx = x0 >> 3, By = y0 >> 3, Bz = z0 >> 3;
-        const uint32_t lx = x0 - (Bx << 3);
-        const uint32_t ly0 = y0 - (By << 3), ly1 = y1 - (By << 3);
-        const uint32_t lz0 = z0 - (Bz << 3), lz1 = z1 - (Bz << 3);
-        t.brick = (Bz * uint32_t(Q.nby) + By) * uint32_t(Q.nbx) + Bx;
-        t.i00 = lx + (lz0 * 9 + ly0) * 8;
-        t.i10 = lx + (lz0 * 9 + ly1) * 8;
-        t.i01 = lx + (lz1 * 9 + ly0) * 8;
-        t.i11 = lx + (lz1 * 9 + ly1) * 8;
-        const float fx = x1 == x0 ? 0.0f : cx - flx, fy = cy - fly, fz = cz - flz;
-        const float ox = 1.0f - fx, oy = 1.0f - fy, oz = 1.0f - fz;
-        const float w00 = oy * oz, w01 = oy * fz, w10 = fy * oz, w11 = fy * fz;
-        t.w[0] = ox * w00;
-        t.w[1] = ox * w01;
-        t.w[2] = ox * w10;
-        t.w[3] = ox * w11;
-        t.w[4] = fx * w00;
-        t.w[5] = fx * w01;
-        t.w[6] = fx * w10;
-        t.w[7] = fx * w11;
-        return t;
-    }
-
-    // the DIM pairs of one pair row (all components of a source side by side):
-    // lo[c] = v_c[x], hi[c] = v_c[x+1], still divided by the brick scale.  One
-    // struct load per row, which the compiler emits as one wide global load.
-    template<int N>
-    struct Words
-    {
-        uint32_t w[N];
-    };
-
-    // 32-bit words of one pair row: 2 per component in FP32, 1 (two 16-bit halves) otherwise
-    template<int DT, int DIM>
-    constexpr int row_words()
-    {
-        return DT == kDtF32 ? 2 * DIM : DIM;
-    }
-
-    // The raw words of one source's sample: its 1 (NEAREST) or 4 (LINEAR) pair
-    // rows and its brick scales, sized for 4 components.  Fetching is split
-    // from interpolation so that the rows of every source of a sample are
-    // requested before the first of them is used.
-    template<int DT>
-    struct SlotRaw
-    {
-        uint32_t r[4][row_words<DT, 4>()];
-        uint32_t sc[4];
-    };
-
-    template<int DT, bool LINEAR, int DIM>
-    __device__ inline void slot_fetch_dim(const BrickSource& S, const BrickTaps& t, SlotRaw<DT>& R)
-    {
-        constexpr int W = row_words<DT, DIM>();
-        const Words<W>* rows = reinterpret_cast<const Words<W>*>(S.data) + t.brick * uint32_t(kBrickPairs);
-        const uint32_t idx[4] = {t.i00, t.i10, t.i01, t.i11};
-#pragma unroll
-        for(int k = 0; k < (LINEAR ? 4 : 1); k++)
-        {
-            const Words<W> a = rows[idx[k]];
-#pragma unroll
-            for(int w = 0; w < W; w++)
-                R.r[k][w] = a.w[w];
-        }
-        const Words<DIM> sc = reinterpret_cast<const Words<DIM>*>(S.scale)[t.brick];
-#pragma unroll
-        for(int c = 0; c < DIM; c++)
-            R.sc[c] = sc.w[c];
-    }
-
-    template<int DT, bool LINEAR>
-    __device__ __attribute__((always_inline)) inline void slot_fetch(const BrickSource& S, const BrickTaps& t, SlotRaw<DT>& R)
-    {
-        switch(S.dim)
-        {
-        case 1: slot_fetch_dim<DT, LINEAR, 1>(S, t, R); break;
-        case 2: slot_fetch_dim<DT, LINEAR, 2>(S, t, R); break;
-        case 3: slot_fetch_dim<DT, LINEAR, 3>(S, t, R); break;
-        default: slot_fetch_dim<DT, LINEAR, 4>(S, t, R); break;
-        }
-    }
-
-    // lo[c] = v_c[x], hi[c] = v_c[x+1] of one fetched row (still divided by the brick scale)
-    template<int DT, int DIM>
-    __device__ inline void decode_row(const uint32_t* w, float lo[DIM], float hi[DIM])
-    {
-#pragma unroll
-        for(int c = 0; c < DIM; c++)
-        {
-            if constexpr(DT == kDtF32)
-            {
-                lo[c] = __uint_as_float(w[2 * c]);
-                hi[c] = __uint_as_float(w[2 * c + 1]);
-            }
-            else if constexpr(DT == kDtF16)
-            {
-                lo[c] = half_lo(w[c]);
-                hi[c] = half_hi(w[c]);
-            }
-            else
-            {
-                lo[c] = __uint_as_float(w[c] << 16);
-                hi[c] = __uint_as_float(w[c] & 0xffff0000u);
-            }
-        }
-    }
-
-    // raw sample of every component of one source with DIM components (v[c], c < DIM)
-    template<int DT, bool LINEAR, int DIM>
-    __device__ inline void slot_interp(const SlotRaw<DT>& R, const BrickTaps& t, float v[4])
-    {
-        if(!LINEAR)
-        {
-            float a[DIM], b[DIM];
-            decode_row<DT, DIM>(R.r[0], a, b);
-#pragma unroll
-            for(int c = 0; c < DIM; c++)
-                v[c] = a[c] * __uint_as_float(R.sc[c]);
-            return;
-        }
-        float d000[DIM], d100[DIM], d010[DIM], d110[DIM], d001[DIM], d101[DIM], d011[DIM], d111[DIM];
-        decode_row<DT, DIM>(R.r[0], d000, d100);
-        decode_row<DT, DIM>(R.r[1], d010, d110);
-        decode_row<DT, DIM>(R.r[2], d001, d101);
-        decode_row<DT, DIM>(R.r[3], d011, d111);
-        // sum of the corners times their weights (one multiply and seven fmas per
-        // component), then the brick scale; equal to the nested lerps in exact arithmetic
-#pragma unroll
-        for(int c = 0; c < DIM; c++)
-        {
-            float a = d000[c] * t.w[0];
-            a = __builtin_fmaf(d001[c], t.w[1], a);
-            a = __builtin_fmaf(d010[c], t.w[2], a);
-            a = __builtin_fmaf(d011[c], t.w[3], a);
-            a = __builtin_fmaf(d100[c], t.w[4], a);
-            a = __builtin_fmaf(d101[c], t.w[5], a);
-            a = __builtin_fmaf(d110[c], t.w[6], a);
-            a = __builtin_fmaf(d111[c], t.w[7], a);
-            v[c] = a * __uint_as_float(R.sc[c]);
-        }
-    }
-
-    // the functor-chain value of one source's sample, dispatched on its component
-    // count (fetch and interpolation in the same case: one source at a time)
-    template<int DT, bool LINEAR, int DIM>
-    __device__ inline void slot_sample(const BrickSource& S, const BrickTaps& t, float v[4])
-    {
-        SlotRaw<DT> R;
-        slot_fetch_dim<DT, LINEAR, DIM>(S, t, R);
-        slot_interp<DT, LINEAR, DIM>(R, t, v);
-    }
-
-    template<int DT, bool LINEAR>
-    __device__ __attribute__((always_inline)) inline float brick_value(const BrickSource& S, const BrickTaps& t)
-    {
-        float v[4] = {0.f, 0.f, 0.f, 0.f};
-        switch(S.dim)
-        {
-        case 1: slot_sample<DT, LINEAR, 1>(S, t, v); break;
-        case 2: slot_sample<DT, LINEAR, 2>(S, t, v); break;
-        case 3: slot_sample<DT, LINEAR, 3>(S, t, v); break;
-        default: slot_sample<DT, LINEAR, 4>(S, t, v); break;
-        }
-        // one chain per source slot, with the component count as a value
-        return apply_chain(S.chain, v[0], v[1], v[2], v[3], S.dim);
-    }
-
-    // Source signature: the component counts of the enabled sources in slot
-    // order, as base-5 digits (slot 0 lowest), 0 = resolved at run time.  A
-    // march compiled for one signature fetches the rows of all its sources
-    // before interpolating any of them, so their latencies overlap.
-    constexpr bool sig_natural(int sig)
-    {
-        return sig >= kSigNatural;
-    }
-
-    constexpr int sig_count(int sig)
-    {
-        int n = 0;
-        for(sig %= kSigNatural; sig > 0; sig /= 5)
-            n++;
-        return n;
-    }
-
-    constexpr int sig_dim(int sig, int slot)
-    {
-        sig %= kSigNatural;
-        for(int i = 0; i < slot; i++)
-            sig /= 5;
-        return sig % 5;
-    }
-
-    // the natural chain's value of a D-component sample: the value itself, or the length
-    // with apply_chain's association ((v0 v0 + v1 v1) + v2 v2)
-    template<int D>
-    __device__ inline float natural_value(const float (&v)[4])
-    {
-        if constexpr(D == 1)
-            return v[0];
-        else if constexpr(D == 2)
-            return sqrtf(v[0] * v[0] + v[1] * v[1]);
-        else if constexpr(D == 3)
-            return sqrtf(v[0] * v[0] + v[1] * v[1] + v[2] * v[2]);
-        else
-            return sqrtf((v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]));
-    }
-
-    template<int DT, bool LINEAR, int SIG, int S>
-    __device__ __attribute__((always_inline)) inline void sig_fetch(const PostParams& Q, const BrickTaps& t, SlotRaw<DT>* R)
-    {
-        if constexpr(S < sig_count(SIG))
-        {
-            slot_fetch_dim<DT, LINEAR, sig_dim(SIG, S)>(Q.src[S], t, R[S]);
-            sig_fetch<DT, LINEAR, SIG, S + 1>(Q, t, R);
-        }
-    }
-
-    struct PostSample
-    {
-        float r, g, b, a; // premultiplied, normalised volume colour
-        float ir, ig, ib, ia; // iso colour and alpha (alpha / threshold * 0.5, maximum over sources)
-    };
-
-    // one source's classified sample into the running sums (weights in slot order)
-    __device__ __attribute__((always_inline)) inline void post_accumulate(PostSample& o, const BrickSource& S, const float4 col)
-    {
-        if(S.weight > 0.0f)
-        {
-            const float a = col.w * S.weight;
-            o.r = o.r + col.x * a;
-            o.g = o.g + col.y * a;
-            o.b = o.b + col.z * a;
-            o.a = o.a + a;
-        }
-        if(S.iso > 0.0f)
-        {
-            const float a = col.w * S.isoScale;
-            if(o.ia < a)
-            {
-                o.ir = col.x;
-                o.ig = col.y;
-                o.ib = col.z;
-                o.ia = a;
-            }
-        }
-    }
-
-    template<int DT, bool LINEAR, int SIG, int S>
-    __device__ __attribute__((always_inline)) inline void sig_classify(
-        const PostParams& Q, const float4* lut, const BrickTaps& t, const SlotRaw<DT>* R, PostSample& o)
-    {
-        if constexpr(S < sig_count(SIG))
-        {
-            constexpr int D = sig_dim(SIG, S);
-            float v[4] = {0.f, 0.f, 0.f, 0.f};
-            slot_interp<DT, LINEAR, D>(R[S], t, v);
-            const float tv = sig_natural(SIG) ? natural_value<D>(v) : apply_chain(Q.src[S].chain, v[0], v[1], v[2], v[3], D);
-            post_accumulate(o, Q.src[S], lut[S * Q.T + tf_index(tv, Q.T)]);
-            sig_classify<DT, LINEAR, SIG, S + 1>(Q, lut, t, R, o);
-        }
-    }
-
-    template<int DT, bool LINEAR, int SIG>
-    __device__ __attribute__((always_inline)) inline PostSample post_classify(const PostParams& Q, const float4* lut, int X, int Y, int Z, float px, float py, float pz)
-    {
-        const BrickTaps t = brick_taps<LINEAR>(Q, X, Y, Z, px, py, pz);
-        PostSample o{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-        if constexpr(SIG != 0)
-        {
-            SlotRaw<DT> R[sig_count(SIG)];
-            sig_fetch<DT, LINEAR, SIG, 0>(Q, t, R);
-            sig_classify<DT, LINEAR, SIG, 0>(Q, lut, t, R, o);
-        }
-        else
-        {
-            // unrolled over the source slots so every parameter-block index is constant
-#pragma unroll
-            for(int s = 0; s < kMaxBrickSources; s++)
-            {
-                if(s >= Q.nsrc)
-                    break;
-                const BrickSource& S = Q.src[s];
-                const float tv = brick_value<DT, LINEAR>(S, t);
-                post_accumulate(o, S, lut[s * Q.T + tf_index(tv, Q.T)]);
-            }
-        }
-        // invTotalWeight = 1 / (sum of volume-source weights), 0 when that sum is 0
-        o.r = o.r * Q.invTotalWeight;
-        o.g = o.g * Q.invTotalWeight;
-        o.b = o.b * Q.invTotalWeight;
-        o.a = o.a * Q.invTotalWeight;
-        return o;
-    }
-
-    // Post-classification march over field bricks.  Same pass structure as
-    // march_kernel (clear, particle DDA, one traversal serving iso and volume,
-    // G-buffer + premultiplied volume colour out); sample positions
-    // startU + stepVec*i with startSteps / end steps taken from the binary64 ray.
-    // the enabled sources' transfer functions, staged in LDS in source order
-    __device__ inline void stage_luts(float4* lds_lut, const PostParams& Q)
-    {
-#pragma unroll
-        for(int j = 0; j < kMaxBrickSources; j++)
-        {
-            if(j >= Q.nsrc)
-                break;
-            const float4* src = Q.luts + size_t(Q.src[j].lutSlot) * Q.T;
-            for(int i = threadIdx.x; i < Q.T; i += blockDim.x)
-                lds_lut[j * Q.T + i] = src[i];
-        }
-    }
-
-    template<int DT, bool LINEAR, bool COUNT, int SIG = 0>
-    __device__ __attribute__((always_inline)) inline void brick_march_body(
-        const FrameParams& F,
-        const PostParams& Q,
-        const ParticleParams& PP,
-        const float4* lut,
-        uint32_t tile)
-    {
-        int px, py;
-        const bool valid = tile_pixel_at(F, tile, px, py);
-        unsigned long long nVol = 0, nIso = 0, nIsoHits = 0, nVolRays = 0, nIsoRays = 0;
-        unsigned long long nCells = 0, nTests = 0, nPartRays = 0, nSteps = 0;
-        if(valid)
-        {
-            const size_t p = size_t(py) * size_t(F.W) + size_t(px);
-            uint32_t color = F.bgClear;
-            F3 normal = f3(0.f, 0.f, 0.f);
-            float depth = FLT_MAX;
-            float4 vcol = make_float4(0.f, 0.f, 0.f, -1.f);
-            RayD rd;
-            const bool inside = ray_setup_d(F, Q, px, py, rd);
-            Ray ray;
-            ray.dir = f3(float(rd.dir[0]), float(rd.dir[1]), float(rd.dir[2]));
-            ray.start = f3(float(rd.start[0]), float(rd.start[1]), float(rd.start[2]));
-            ray.startDepth = float(rd.startDepth);
-            ray.endDepth = float(rd.endDepth);
-            ray.isClipped = rd.isClipped;
-            ray.clipN = f3(float(rd.clipN[0]), float(rd.clipN[1]), float(rd.clipN[2]));
-            if(inside && PP.nsrc > 0)
-            {
-                nPartRays++;
-                particle_dda<COUNT>(PP, ray, color, depth, normal, nCells, nTests);
-            }
-            const int mode = F.renderMode;
-            const bool depthZeroed = mode == 2 || (mode >= 4 && mode <= 8);
-            if(inside)
-            {
-                const double endD = fmin(rd.endDepth, double(depth));
-                bool isoOn = F.isoEnabled && endD > rd.startDepth;
-                bool volBlend = F.volumeEnabled && !depthZeroed && endD > rd.startDepth;
-                if(isoOn || volBlend)
-                {
-                    const F3 sc = f3(F.scale[0], F.scale[1], F.scale[2]);
-                    const double ex = rd.dir[0] / double(sc.x), ey = rd.dir[1] / double(sc.y), ez = rd.dir[2] / double(sc.z);
-                    const double stepUd = double(F.step)
-                        * (sqrt(rd.dir[0] * rd.dir[0] + rd.dir[1] * rd.dir[1] + rd.dir[2] * rd.dir[2]) / sqrt(ex * ex + ey * ey + ez * ez));
-                    const float stepU = float(stepUd);
-                    const float factor = stepU / F.minSize * 2.0f * F.totalWeightAll;
-                    const int startSteps = int(ceil(rd.startDepth / stepUd));
-                    const int endIso = int(floor(endD / stepUd));
-                    int endVol = endIso;
-                    const F3 stepVec = divv(muls(ray.dir, stepU), sc);
-                    const F3 startU = divv(ray.start, sc);
-                    if(isoOn)
-                        nIsoRays++;
-                    float cr = 0.f, cg = 0.f, cb = 0.f, ca = 0.f;
-                    float oldValue = 0.0f;
-                    // traversal state as step bounds, not flags (no lane masks carried by the
-                    // loop): the iso test runs while i <= isoEnd, the volume while i <= volEnd,
-                    // either set below every step to switch it off; hitStep is the hit's step
-                    const int off = -0x7fffffff;
-                    int isoEnd = isoOn ? endIso : off;
-                    int volEnd = volBlend ? endVol : off;
-                    int hitStep = -1;
-                    for(int i = startSteps;; i++)
-                    {
-                        if(i > (isoEnd > volEnd ? isoEnd : volEnd))
-                            break;
-                        if(COUNT)
-                            nSteps++;
-                        const float fi = float(i);
-                        const PostSample sm = post_classify<DT, LINEAR, SIG>(
-                            Q, lut, F.X, F.Y, F.Z, startU.x + stepVec.x * fi, startU.y + stepVec.y * fi, startU.z + stepVec.z * fi);
-                        if(i <= isoEnd)
-                        {
-                            const float value = gmin(sm.ia, 1.0f);
-                            if(COUNT)
-                                nIso++;
-                            const float tmp = oldValue;
-                            oldValue = value;
-                            if(value >= 0.5f)
-                            {
-                                const bool first = ray.isClipped && i == startSteps;
-                                depth = first ? ray.startDepth : fi * stepU + stepU * (0.5f - tmp) / (value - tmp);
-                                hitStep = i;
-                                isoEnd = off;
-                                if(COUNT)
-                                    nIsoHits++;
-                                // the volume pass ends at min(clip end, iso depth)
-                                const double ve = fmin(rd.endDepth, double(depth));
-                                if(!(ve > rd.startDepth))
-                                    volEnd = off;
-                                else if(volEnd != off)
-                                    volEnd = int(floor(ve / stepUd));
-                            }
-                        }
-                        if(i <= volEnd)
-                        {
-                            if(COUNT)
-                                nVol++;
-                            const float w = 1.0f - ca;
-                            cr = cr + w * (sm.r * factor);
-                            cg = cg + w * (sm.g * factor);
-                            cb = cb + w * (sm.b * factor);
-                            ca = ca + w * (sm.a * factor);
-                            if(ca > 0.99f)
-                                volEnd = off;
-                        }
-                    }
-                    const bool isoHit = hitStep >= 0;
-                    const bool isoFirst = isoHit && ray.isClipped && hitStep == startSteps;
-                    // a hit at or before the ray's start leaves no volume segment to blend
-                    if(isoHit && !(fmin(rd.endDepth, double(depth)) > rd.startDepth))
-                        volBlend = false;
-                    if(isoHit)
-                    {
-                        const F3 pu = divv(add(ray.start, muls(ray.dir, depth)), sc);
-                        // hit colour, then the six central-difference samples of the iso value
-                        // (one loop, so the per-sample classification is inlined once)
-                        float hr = 0.f, hg = 0.f, hb = 0.f;
-                        F3 g = f3(0.f, 0.f, 0.f);
-#pragma unroll 1
-                        for(int d = -1; d < 6; d++)
-                        {
-                            const float sx = d == 0 ? 1.0f : (d == 1 ? -1.0f : 0.0f);
-                            const float sy = d == 2 ? 1.0f : (d == 3 ? -1.0f : 0.0f);
-                            const float sz = d == 4 ? 1.0f : (d == 5 ? -1.0f : 0.0f);
-                            const PostSample h = post_classify<DT, LINEAR, SIG>(Q, lut, F.X, F.Y, F.Z, pu.x + sx, pu.y + sy, pu.z + sz);
-                            const float v = gmin(h.ia, 1.0f);
-                            if(d < 0)
-                            {
-                                hr = h.ir;
-                                hg = h.ig;
-                                hb = h.ib;
-                            }
-                            else if(d == 0)
-                                g.x = v;
-                            else if(d == 1)
-                                g.x = g.x - v;
-                            else if(d == 2)
-                                g.y = v;
-                            else if(d == 3)
-                                g.y = g.y - v;
-                            else if(d == 4)
-                                g.z = v;
-                            else
-                                g.z = g.z - v;
-                        }
-                        float gl = len3(g);
-                        if(isoFirst || gl == 0.0f)
-                        {
-                            g = ray.clipN;
-                            gl = 1.0f;
-                        }
-                        normal = f3(-g.x / gl, -g.y / gl, -g.z / gl);
-                        color = to_byte4(hr, hg, hb, 1.0f);
-                    }
-                    if(volBlend)
-                    {
-                        nVolRays++;
-                        vcol = make_float4(cr, cg, cb, ca);
-                    }
-                }
-            }
-            F.color[p] = color;
-            F.depth[p] = depth;
-            F.normal[3 * p + 0] = normal.x;
-            F.normal[3 * p + 1] = normal.y;
-            F.normal[3 * p + 2] = normal.z;
-            F.volColor[p] = vcol;
-            if(!F.aoEnabled)
-                F.ao[p] = 0.0f;
-        }
-        if(COUNT)
-        {
-            block_count_add(F.counters + 0, nVol);
-            block_count_add(F.counters + 1, nIso);
-            block_count_add(F.counters + 2, nIsoHits);
-            block_count_add(F.counters + 3, nCells);
-            block_count_add(F.counters + 4, nTests);
-            block_count_add(F.counters + 5, nVolRays);
-            block_count_add(F.counters + 6, nIsoRays);
-            block_count_add(F.counters + 7, nPartRays);
-            block_count_add(F.counters + 8, nSteps);
-            // the wave runs the traversal loop as long as its longest lane
-            int wm = int(nSteps);
-            for(int off = 32; off > 0; off >>= 1)
-                wm = max(wm, __shfl_xor(wm, off, 64));
-            block_count_add(F.counters + 9, (threadIdx.x & 63u) == 0 ? (unsigned long long) wm : 0ull);
-        }
-    }
-
-    template<int DT, bool LINEAR, bool COUNT>
-    __global__ __launch_bounds__(256) void brick_march_kernel(const FrameParams F, const PostParams Q, const ParticleParams PP)
-    {
-        extern __shared__ float4 lds_lut[];
-        stage_luts(lds_lut, Q);
-        __syncthreads();
-        brick_march_body<DT, LINEAR, COUNT>(F, Q, PP, lds_lut, march_tile(F));
-    }
-
-    // trilinear march compiled for one source signature (see sig_count)
-    template<int DT, int SIG>
-    __global__ __launch_bounds__(256) void brick_march_sig_kernel(const FrameParams F, const PostParams Q, const ParticleParams PP)
-    {
-        extern __shared__ float4 lds_lut[];
-        stage_luts(lds_lut, Q);
-        __syncthreads();
-        brick_march_body<DT, true, false, SIG>(F, Q, PP, lds_lut, march_tile(F));
-    }
-
-    // ------------------------------------------------------------------ batched form
-    // One persistent launch over many frames (sub-volume x view): workgroups pop
-    // chunks of 16x16 tiles from a global counter until the work is exhausted
-    // (every workgroup reaches the exit when the counter passes the last chunk).
-    // Frames share the transfer functions (staged once per workgroup).
-    template<int DT, bool LINEAR, int SIG = 0>
-    __global__ __launch_bounds__(256) void batch_march_kernel(const BatchParams B)
-    {
-        extern __shared__ float4 lds_lut[];
-        __shared__ uint32_t s_work;
-        stage_luts(lds_lut, B.posts[0]);
-        for(;;)
-        {
-            __syncthreads();
-            if(threadIdx.x == 0)
-                s_work = atomicAdd(B.counter, 1u);
-            __syncthreads();
-            // uniform across the workgroup: keep the work index in a scalar register so
-            // the frame's parameter blocks are read with scalar loads
-            const uint32_t t0 = uint32_t(__builtin_amdgcn_readfirstlane(int(s_work))) * uint32_t(B.chunk);
-            if(t0 >= B.ntiles)
-                break;
-            const uint32_t t1 = min(t0 + uint32_t(B.chunk), B.ntiles);
-            // frame of tile t0: largest i with tileStart[i] <= t0
-            int lo = 0, hi = B.nframes - 1;
-            while(lo < hi)
-            {
-                const int mid = (lo + hi + 1) >> 1;
-                if(B.tileStart[mid] <= t0)
-                    lo = mid;
-                else
-                    hi = mid - 1;
-            }
-            int item = __builtin_amdgcn_readfirstlane(lo);
-            for(uint32_t t = t0; t < t1; t++)
-            {
-                while(t >= B.tileStart[item + 1])
-                    item++;
-                item = __builtin_amdgcn_readfirstlane(item);
-                brick_march_body<DT, LINEAR, false, SIG>(B.frames[item], B.posts[item], B.parts[item], lds_lut, t - B.tileStart[item]);
-            }
-        }
-    }
-
-    // per-frame passes of the batch: grid (tiles of the largest frame, frames)
     __global__ __launch_bounds__(256) void batch_ssao_kernel(const FrameParams* frames)
     {
         const FrameParams& F = frames[blockIdx.y];
@@ -1327,141 +534,6 @@ namespace isaac_hip
         if(dtype == kDtF16)
             return launch_brick_build<kDtF16>(src, stride, dim, X, Y, Z, nbx, nby, nbricks, scale, out, s);
         return launch_brick_build<kDtBf16>(src, stride, dim, X, Y, Z, nbx, nby, nbricks, scale, out, s);
-    }
-
-    static_assert(sizeof(FrameParams) + sizeof(PostParams) + sizeof(ParticleParams) <= 4096, "kernel argument block");
-
-    // a source's chain is its natural one: no operations for a scalar source, one
-    // `length` (then nothing) for a vector source
-    bool natural_chain(const ChainDesc& c, int dim)
-    {
-        for(int k = 0; k < kMaxFunctors; k++)
-        {
-            const int want = (k == 0 && dim > 1) ? OP_LENGTH : OP_IDEM;
-            if(c.op[k] != want)
-                return false;
-        }
-        return true;
-    }
-
-    bool natural_chains(const PostParams& Q)
-    {
-        for(int i = 0; i < Q.nsrc; i++)
-            if(!natural_chain(Q.src[i].chain, Q.src[i].dim))
-                return false;
-        return true;
-    }
-
-    int post_signature(const PostParams& Q)
-    {
-        int sig = 0;
-        for(int i = Q.nsrc - 1; i >= 0; i--)
-            sig = sig * 5 + Q.src[i].dim;
-        return Q.nsrc > 0 ? sig : -1;
-    }
-
-    hipError_t launch_brick_march(const FrameParams& F, const PostParams& Q, const ParticleParams& PP, bool counting, hipStream_t s)
-    {
-        const unsigned nb = march_grid(F);
-        if(nb == 0)
-            return hipSuccess;
-        const dim3 grid(nb), block(256);
-        const size_t lds = size_t(Q.nsrc) * Q.T * sizeof(float4);
-        if(F.linear && !counting)
-        {
-            // signatures with a compiled march: density (1), vector (3), and pairs of them
-            const int sig = post_signature(Q);
-            const int v = Q.dtype * 8 + (sig == 1 ? 0 : sig == 3 ? 1 : sig == 6 ? 2 : sig == 8 ? 3 : sig == 16 ? 4 : 7);
-            const bool natural = natural_chains(Q);
-            switch(v)
-            {
-#define ISAAC_SIG_CASE(dt, k, sg)                                                                                       \
-    case dt * 8 + k:                                                                                                    \
-        if(natural)                                                                                                     \
-            hipLaunchKernelGGL((brick_march_sig_kernel<dt, sg + kSigNatural>), grid, block, lds, s, F, Q, PP);          \
-        else                                                                                                            \
-            hipLaunchKernelGGL((brick_march_sig_kernel<dt, sg>), grid, block, lds, s, F, Q, PP);                        \
-        return hipGetLastError();
-                ISAAC_SIG_CASE(0, 0, 1)
-                ISAAC_SIG_CASE(0, 1, 3)
-                ISAAC_SIG_CASE(0, 2, 6)
-                ISAAC_SIG_CASE(0, 3, 8)
-                ISAAC_SIG_CASE(0, 4, 16)
-                ISAAC_SIG_CASE(1, 0, 1)
-                ISAAC_SIG_CASE(1, 1, 3)
-                ISAAC_SIG_CASE(1, 2, 6)
-                ISAAC_SIG_CASE(1, 3, 8)
-                ISAAC_SIG_CASE(1, 4, 16)
-                ISAAC_SIG_CASE(2, 0, 1)
-                ISAAC_SIG_CASE(2, 1, 3)
-                ISAAC_SIG_CASE(2, 2, 6)
-                ISAAC_SIG_CASE(2, 3, 8)
-                ISAAC_SIG_CASE(2, 4, 16)
-#undef ISAAC_SIG_CASE
-            default: break;
-            }
-        }
-        const int v = (Q.dtype * 4) | (F.linear ? 2 : 0) | (counting ? 1 : 0);
-        switch(v)
-        {
-        case 0: hipLaunchKernelGGL((brick_march_kernel<0, false, false>), grid, block, lds, s, F, Q, PP); break;
-        case 1: hipLaunchKernelGGL((brick_march_kernel<0, false, true>), grid, block, lds, s, F, Q, PP); break;
-        case 2: hipLaunchKernelGGL((brick_march_kernel<0, true, false>), grid, block, lds, s, F, Q, PP); break;
-        case 3: hipLaunchKernelGGL((brick_march_kernel<0, true, true>), grid, block, lds, s, F, Q, PP); break;
-        case 4: hipLaunchKernelGGL((brick_march_kernel<1, false, false>), grid, block, lds, s, F, Q, PP); break;
-        case 5: hipLaunchKernelGGL((brick_march_kernel<1, false, true>), grid, block, lds, s, F, Q, PP); break;
-        case 6: hipLaunchKernelGGL((brick_march_kernel<1, true, false>), grid, block, lds, s, F, Q, PP); break;
-        case 7: hipLaunchKernelGGL((brick_march_kernel<1, true, true>), grid, block, lds, s, F, Q, PP); break;
-        case 8: hipLaunchKernelGGL((brick_march_kernel<2, false, false>), grid, block, lds, s, F, Q, PP); break;
-        case 9: hipLaunchKernelGGL((brick_march_kernel<2, false, true>), grid, block, lds, s, F, Q, PP); break;
-        case 10: hipLaunchKernelGGL((brick_march_kernel<2, true, false>), grid, block, lds, s, F, Q, PP); break;
-        default: hipLaunchKernelGGL((brick_march_kernel<2, true, true>), grid, block, lds, s, F, Q, PP); break;
-        }
-        return hipGetLastError();
-    }
-
-    hipError_t launch_batch_march(const BatchParams& B, int dtype, bool linear, int sig, size_t lds, int grid, hipStream_t s)
-    {
-        if(B.nframes <= 0 || grid <= 0)
-            return hipSuccess;
-        const bool natural = sig_natural(sig);
-        sig %= kSigNatural;
-        if(linear && (sig == 1 || sig == 3 || sig == 16))
-        {
-            const int k = dtype * 3 + (sig == 1 ? 0 : sig == 3 ? 1 : 2);
-            switch(k)
-            {
-#define ISAAC_SIG_CASE(dt, j, sg)                                                                                       \
-    case dt * 3 + j:                                                                                                    \
-        if(natural)                                                                                                     \
-            hipLaunchKernelGGL((batch_march_kernel<dt, true, sg + kSigNatural>), dim3(grid), dim3(256), lds, s, B);     \
-        else                                                                                                            \
-            hipLaunchKernelGGL((batch_march_kernel<dt, true, sg>), dim3(grid), dim3(256), lds, s, B);                   \
-        return hipGetLastError();
-                ISAAC_SIG_CASE(0, 0, 1)
-                ISAAC_SIG_CASE(0, 1, 3)
-                ISAAC_SIG_CASE(0, 2, 16)
-                ISAAC_SIG_CASE(1, 0, 1)
-                ISAAC_SIG_CASE(1, 1, 3)
-                ISAAC_SIG_CASE(1, 2, 16)
-                ISAAC_SIG_CASE(2, 0, 1)
-                ISAAC_SIG_CASE(2, 1, 3)
-                ISAAC_SIG_CASE(2, 2, 16)
-#undef ISAAC_SIG_CASE
-            default: break;
-            }
-        }
-        const int v = dtype * 2 + (linear ? 1 : 0);
-        switch(v)
-        {
-        case 0: hipLaunchKernelGGL((batch_march_kernel<0, false>), dim3(grid), dim3(256), lds, s, B); break;
-        case 1: hipLaunchKernelGGL((batch_march_kernel<0, true>), dim3(grid), dim3(256), lds, s, B); break;
-        case 2: hipLaunchKernelGGL((batch_march_kernel<1, false>), dim3(grid), dim3(256), lds, s, B); break;
-        case 3: hipLaunchKernelGGL((batch_march_kernel<1, true>), dim3(grid), dim3(256), lds, s, B); break;
-        case 4: hipLaunchKernelGGL((batch_march_kernel<2, false>), dim3(grid), dim3(256), lds, s, B); break;
-        default: hipLaunchKernelGGL((batch_march_kernel<2, true>), dim3(grid), dim3(256), lds, s, B); break;
-        }
-        return hipGetLastError();
     }
 
     hipError_t launch_batch_ssao(const FrameParams* frames, int nframes, int maxTiles, hipStream_t s)

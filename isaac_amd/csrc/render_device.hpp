@@ -1,5 +1,5 @@
 // Device functions shared by the render kernels: ray setup, pixel tiles of the
-// workgroups, the particle walk, byte scaling.
+// workgroups, the particle walk, byte scaling, functor chains, source signatures.
 #pragma once
 
 #include "kernels.hpp"
@@ -382,5 +382,158 @@ namespace isaac_hip
             return nb;
         const unsigned ns = ((unsigned(F.tilesX) + S - 1u) / S) * ((unsigned(F.tilesY) + S - 1u) / S);
         return (ns + 7u) / 8u * 8u * S * S;
+    }
+
+    // ------------------------------------------------------------------ functor chain
+    // pow stays out of line: inlined, its ~70 instructions per component and
+    // functor slot made up most of the code of the marches that evaluate the
+    // chain per sample (rarely used, and the call is only taken for it).
+    static __device__ __noinline__ float chain_pow(float a, float b)
+    {
+        return powf(a, b);
+    }
+
+    // f2(f1(f0(v,p0),p1),p2).x with the feature dimension propagating
+    // (lib/isaac/isaac_functor_chain.hpp:96-108, lib/isaac/isaac_functors.hpp:42-183).
+    __device__ inline float apply_chain(const ChainDesc& c, float v0, float v1, float v2, float v3, int n)
+    {
+        float v[4] = {v0, v1, v2, v3};
+#pragma unroll
+        for(int k = 0; k < kMaxFunctors; k++)
+        {
+            const int op = c.op[k];
+            if(op == OP_ADD)
+            {
+#pragma unroll
+                for(int i = 0; i < 4; i++)
+                    if(i < n)
+                        v[i] = v[i] + c.p[k][i];
+            }
+            else if(op == OP_MUL)
+            {
+#pragma unroll
+                for(int i = 0; i < 4; i++)
+                    if(i < n)
+                        v[i] = v[i] * c.p[k][i];
+            }
+            else if(op == OP_LENGTH)
+            {
+                float d;
+                if(n == 1)
+                    d = v[0] * v[0];
+                else if(n == 2)
+                    d = v[0] * v[0] + v[1] * v[1];
+                else if(n == 3)
+                    d = v[0] * v[0] + v[1] * v[1] + v[2] * v[2];
+                else
+                    d = (v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]);
+                v[0] = sqrtf(d);
+                n = 1;
+            }
+            else if(op == OP_POW)
+            {
+#pragma unroll
+                for(int i = 0; i < 4; i++)
+                    if(i < n)
+                        v[i] = chain_pow(v[i], c.p[k][i]);
+            }
+            else if(op == OP_SUM)
+            {
+                float s = 0.0f;
+#pragma unroll
+                for(int i = 0; i < 4; i++)
+                    if(i < n)
+                        s = s + v[i];
+                v[0] = s;
+                n = 1;
+            }
+        }
+        return v[0];
+    }
+
+    // x / d for a divisor fixed per launch, with r = RN(1/d) computed once on the
+    // host: x*r plus one fma residual correction (Markstein's correction), three
+    // instructions instead of the correctly rounded division sequence.  Equal to the
+    // IEEE quotient for finite operands away from overflow and underflow
+    // (tests/cpp/divq_check.c: 0 of 2e8 seeded quotients differ, a quarter of them
+    // next to rounding boundaries; for d = 255 every x in [0, 256],
+    // tests/cpp/div255_check.c).
+    __device__ inline float div_by(float x, float d, float r)
+    {
+        const float q0 = x * r;
+        const float e = __builtin_fmaf(-q0, d, x);
+        return __builtin_fmaf(e, r, q0);
+    }
+
+    __device__ inline int tf_index(float v, int T)
+    {
+        return tf_index_of(v * float(T), T);
+    }
+
+    // a source's chain is its natural one: no operations for a scalar source, one
+    // `length` (then nothing) for a vector source
+    inline bool natural_chain(const ChainDesc& c, int dim)
+    {
+        for(int k = 0; k < kMaxFunctors; k++)
+        {
+            const int want = (k == 0 && dim > 1) ? OP_LENGTH : OP_IDEM;
+            if(c.op[k] != want)
+                return false;
+        }
+        return true;
+    }
+
+    // ------------------------------------------------------------------ source signatures
+    // Source signature: the component counts of the enabled sources in slot
+    // order, as base-5 digits (slot 0 lowest), 0 = resolved at run time.  A
+    // march compiled for one signature fetches the rows of all its sources
+    // before interpolating any of them, so their latencies overlap.
+    constexpr bool sig_natural(int sig)
+    {
+        return sig >= kSigNatural;
+    }
+
+    constexpr int sig_count(int sig)
+    {
+        int n = 0;
+        for(sig %= kSigNatural; sig > 0; sig /= 5)
+            n++;
+        return n;
+    }
+
+    constexpr int sig_dim(int sig, int slot)
+    {
+        sig %= kSigNatural;
+        for(int i = 0; i < slot; i++)
+            sig /= 5;
+        return sig % 5;
+    }
+
+    // tf_index(sqrtf(s), T) for s >= 0 (or NaN): v_sqrt_f32 is within one ulp of the square root, so the
+    // value whose integer part is the index is within y * 2^-21 of the one that the correctly rounded
+    // root gives, and the integer parts agree unless an integer lies that near; only then (about one
+    // value in 1000 at T = 1024) the root is rounded correctly, which takes some 15 instructions
+    __device__ inline int tf_index_sqrt(float s, int T)
+    {
+        const float y = __builtin_amdgcn_sqrtf(s) * float(T) + 0x1.fffffep-2f;
+        // (a branch of the whole wave: per lane the compiler would compute both)
+        if(__builtin_amdgcn_ballot_w64(!(fabsf(y - rintf(y)) > y * 0x1p-20f)) != 0) // (NaN and infinity too)
+            return tf_index(sqrtf(s), T);
+        return (int) __builtin_amdgcn_fmed3f(y, 0.0f, float(T - 1));
+    }
+
+    // the transfer index of a D-component sample's natural chain: of the value itself, or of the
+    // length with apply_chain's association ((v0 v0 + v1 v1) + v2 v2)
+    template<int D>
+    __device__ inline int natural_index(const float (&v)[4], int T)
+    {
+        if constexpr(D == 1)
+            return tf_index(v[0], T);
+        else if constexpr(D == 2)
+            return tf_index_sqrt(v[0] * v[0] + v[1] * v[1], T);
+        else if constexpr(D == 3)
+            return tf_index_sqrt(v[0] * v[0] + v[1] * v[1] + v[2] * v[2], T);
+        else
+            return tf_index_sqrt((v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]), T);
     }
 } // namespace isaac_hip

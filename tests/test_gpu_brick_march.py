@@ -1,0 +1,71 @@
+"""The brick form's march against its counting variant, which clamps the taps at every
+step, at volume sizes about a brick (8 voxels) and its apron, and the batch's work
+queues at frame sizes that leave tiles and super-tiles over."""
+import dataclasses
+
+import numpy as np
+import pytest
+
+from isaac_amd import scenes
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", autouse=True)
+def gpu():
+    torch = pytest.importorskip("torch")
+    if not torch.cuda.is_available():
+        pytest.skip("needs a GPU")
+
+
+def _spec(size, sources, fb=(141, 99), step=0.5, pose=scenes.FILL_POSE):
+    X, Y, Z = size
+    rng = np.random.default_rng(X * 10007 + Y * 101 + Z)
+    dens = (0.7 * scenes.gaussian_mixture((Z, Y, X), 5, 6, (0.1 * max(size), 0.3 * max(size)))
+            + 0.2 * rng.uniform(0.0, 1.0, (Z, Y, X))).astype(np.float32)
+    vec = rng.uniform(-0.6, 0.6, (Z, Y, X, 3)).astype(np.float32)
+    vols = {"density": scenes.VolumeSourceSpec("density", dens, "idem", list(scenes.DENSITY_TF), 2.0, 0.4),
+            "vector": scenes.VolumeSourceSpec("vector", vec, "length", list(scenes.VECTOR_TF), 2.0, 0.0),
+            "scaled": scenes.VolumeSourceSpec("scaled", vec, "length | mul(0.8)", list(scenes.VECTOR_TF), 1.0, 0.0)}
+    return scenes.SceneSpec("bricks", tuple(size), tuple(size), (1, 1, 1), framebuffer=fb, volumes=[vols[s] for s in sources],
+                            step=step, interpolation=True, camera=pose)
+
+
+@pytest.mark.parametrize("sources", [("density",), ("vector",), ("density", "vector"), ("scaled", "density")])
+@pytest.mark.parametrize("size", [(1, 1, 1), (8, 9, 7), (17, 16, 24), (41, 8, 33)])
+def test_brick_march_equals_counting_march(size, sources):
+    from isaac_amd import visualization as V
+
+    vis = V.from_scene(_spec(size, sources))
+    for dtype in (vis.F32, vis.F16, vis.BF16):
+        vis.set_render_form(vis.FORM_BRICKS, dtype)
+        for step in (0.5, 0.11, 2.5):
+            vis.step = step
+            vis.update_buffers()
+            img = vis.draw()
+            g = [a.copy() for a in vis.gbuffer()]
+            vis.set_counting(True)
+            assert np.array_equal(vis.draw(), img), (dtype, step)
+            for a, b in zip(vis.gbuffer(), g):
+                assert np.array_equal(a, b), (dtype, step)
+            vis.set_counting(False)
+    vis.close()
+
+
+@pytest.mark.parametrize("fb", [(16, 16), (65, 63), (333, 201), (700, 30)])
+def test_batch_frames_of_any_size(fb):
+    from isaac_amd import batch as B
+
+    vises, _ = B.make_subvolumes(0, count=3, seed=4, fb=fb, dtype=1, sides=[24, 40, 16])
+    projs, mvs = B.views_for(vises, 2, seed=4)
+    ref = np.stack([vises[f // 2].draw(projection=projs[f], modelview_=mvs[f]) for f in range(6)])
+    b = B.Batch(vises, *fb)
+    b.set_views(projs, mvs, bg=vises[0].background_color)
+    for chunk, groups in ((1, 4), (3, 1), (64, 2)):
+        b.set_tuning(B.TUNE_CHUNK, chunk)
+        b.set_tuning(B.TUNE_GROUPS_PER_CU, groups)
+        b.render(B.GRAPH)
+        assert np.array_equal(b.images(), ref), (chunk, groups)
+    b.close()
+    for v in vises:
+        v.close()
