@@ -339,15 +339,18 @@ extern "C"
         b->nviews = nviews;
         // the source signature selects a march compiled for it when every frame shares it
         int sig = post_signature(b->hQ[0]);
-        bool natural = true;
+        bool natural = true, joint = true;
         for(int f = 0; f < nframes; f++)
         {
+            joint = joint && b->hQ[f].joint;
             if(post_signature(b->hQ[f]) != sig)
                 sig = 0;
             natural = natural && natural_chains(b->hQ[f]);
         }
         if(sig > 0 && natural)
             sig += kSigNatural;
+        if(sig > 0 && joint)
+            sig += kSigJoint;
         const size_t lutLds = size_t(b->hQ[0].nsrc) * size_t(b->hQ[0].T) * sizeof(float4);
         // launch arguments the captured graph holds
         if(c0->brickDtype != b->dtype || c0->interpolation != b->linear || sig != b->sig || lutLds != b->lutLds)

@@ -201,17 +201,17 @@ namespace isaac_hip
     __device__ inline void slot_fetch_dim(const BrickSource& S, const BrickTaps& t, SlotRaw<DT>& R)
     {
         constexpr int W = row_words<DT, DIM>();
-        const Words<W>* rows = static_cast<const Words<W>*>(S.data);
+        const uint32_t* rows = static_cast<const uint32_t*>(S.data);
         const uint32_t idx[4] = {t.row, t.row + t.dy, t.row + t.dz, t.row + t.dy + t.dz};
 #pragma unroll
         for(int k = 0; k < (LINEAR ? 4 : 1); k++)
         {
-            const Words<W> a = rows[idx[k]];
+            const Words<W> a = *reinterpret_cast<const Words<W>*>(rows + size_t(idx[k]) * uint32_t(S.stride));
 #pragma unroll
             for(int w = 0; w < W; w++)
                 R.r[k][w] = a.w[w];
         }
-        const Words<DIM> sc = reinterpret_cast<const Words<DIM>*>(S.scale)[t.brick];
+        const Words<DIM> sc = *reinterpret_cast<const Words<DIM>*>(S.scale + size_t(t.brick) * uint32_t(S.scaleStride));
 #pragma unroll
         for(int c = 0; c < DIM; c++)
             R.sc[c] = sc.w[c];
@@ -228,13 +228,16 @@ namespace isaac_hip
     {
         constexpr int W = row_words<DT, DIM>();
         constexpr uint32_t dist[4] = {0u, kPairRowY, kPairRowZ, kPairRowY + kPairRowZ};
-        const GlobalBytes base = (GlobalBytes) S.data + row * uint32_t(4 * W);
+        const uint32_t rowBytes = 4u * uint32_t(S.stride), at = row * rowBytes;
 #pragma unroll
         for(int k = 0; k < 4; k++)
+        {
+            const GlobalBytes base = (GlobalBytes) S.data + dist[k] * rowBytes; // uniform
 #pragma unroll
             for(int w = 0; w < W; w++)
-                R.r[k][w] = ((GlobalWords) (base + dist[k] * uint32_t(4 * W)))[w];
-        const GlobalWords sc = (GlobalWords) ((GlobalBytes) S.scale + brick * uint32_t(4 * DIM));
+                R.r[k][w] = ((GlobalWords) (base + at))[w];
+        }
+        const GlobalWords sc = (GlobalWords) ((GlobalBytes) S.scale + brick * (4u * uint32_t(S.scaleStride)));
 #pragma unroll
         for(int c = 0; c < DIM; c++)
             R.sc[c] = sc[c];
@@ -345,6 +348,32 @@ namespace isaac_hip
         }
     }
 
+    // both sources of joint rows: 4 gathers and one of the scales
+    template<int DT, int D0, int D1>
+    __device__ __attribute__((always_inline)) inline void joint_fetch_interior(const PostParams& Q, uint32_t row, uint32_t brick, SlotRaw<DT>* R)
+    {
+        constexpr uint32_t dist[4] = {0u, kPairRowY, kPairRowZ, kPairRowY + kPairRowZ}, W = D0 + D1;
+        const GlobalBytes base = (GlobalBytes) Q.src[0].data + row * (4u * W);
+#pragma unroll
+        for(int k = 0; k < 4; k++)
+        {
+            const GlobalWords w = (GlobalWords) (base + dist[k] * (4u * W));
+#pragma unroll
+            for(int c = 0; c < D0; c++)
+                R[0].r[k][c] = w[c];
+#pragma unroll
+            for(int c = 0; c < D1; c++)
+                R[1].r[k][c] = w[D0 + c];
+        }
+        const GlobalWords sc = (GlobalWords) ((GlobalBytes) Q.src[0].scale + brick * (4u * W));
+#pragma unroll
+        for(int c = 0; c < D0; c++)
+            R[0].sc[c] = sc[c];
+#pragma unroll
+        for(int c = 0; c < D1; c++)
+            R[1].sc[c] = sc[D0 + c];
+    }
+
     // an interior sample's fetched rows and its fractions
     template<int DT, int SIG>
     struct InteriorSample
@@ -369,7 +398,10 @@ namespace isaac_hip
         // 648 brick + (x & 7) + 8 (y & 7) + 72 (z & 7) with v & 7 = v - 8 (v >> 3)
         const uint32_t row = x + Bx * uint32_t(kBrickPairs - 8) + y * kPairRowY + By * (perY - 8u * kPairRowY) + z * kPairRowZ
             + Bz * (perZ - 8u * kPairRowZ);
-        sig_fetch_interior<DT, SIG, 0>(Q, row, brick, s.R);
+        if constexpr(sig_joint(SIG))
+            joint_fetch_interior<DT, sig_dim(SIG, 0), sig_dim(SIG, 1)>(Q, row, brick, s.R);
+        else
+            sig_fetch_interior<DT, SIG, 0>(Q, row, brick, s.R);
     }
 
     struct PostSample
@@ -780,11 +812,12 @@ namespace isaac_hip
     // of a super-tile share an L2.  A wave pops from its own XCD's queue (workgroup b runs on XCD
     // b % 8) until that is empty and then helps with the others'.  Every wave takes its own work:
     // waves of one workgroup that shared a pop waited for the longest rays of all four.
-    // Bound by the texture address unit (97 % busy: 10 gathers a step, 27 cycles each, as the 8x8 rays
-    // of a wave touch 32 cache lines a gather).  Measured on MI355X, 12 sub-volumes of sides 32..256
-    // x 4 views at 960x540 in FP16: 13.3 -> 9.7 ms for the batch (one counter of 16x16 tiles for all
-    // workgroups, corners clamped at every step, parameter blocks in vector registers before);
-    // pops of 2, 4 and 8 quarters 10.1, 11.5 and 13.5 ms; one queue per CU 9.7 ms.
+    // Bound by the texture address unit, as the 8x8 rays of a wave touch 32 cache lines a gather
+    // (27 cycles each): joint rows of two sources take 5 gathers a step in place of 10.  Measured on
+    // MI355X, 12 sub-volumes of sides 32..256 x 4 views at 960x540 in FP16, for the batch: 13.3 ms
+    // (one counter of 16x16 tiles for all workgroups, corners clamped at every step, parameter blocks
+    // in vector registers), 9.8 ms with these queues and interior steps, 7.9 ms with joint rows.
+    // Before joint rows: pops of 2, 4 and 8 quarters 10.1, 11.5 and 13.5 ms; one queue per CU 9.7 ms.
     struct MarchQueues
     {
         uint32_t sx, sy, perFrame, total; // super-tiles of a frame; units of a queue, per frame and in all
@@ -885,6 +918,18 @@ namespace isaac_hip
             const bool natural = natural_chains(Q);
             switch(v)
             {
+            // joint rows: the pairs of sources that update_buffers joins
+#define ISAAC_SIG_JOINT_CASE(dt, k, sg)                                                                                 \
+    case dt * 8 + k:                                                                                                    \
+        if(Q.joint && natural)                                                                                          \
+            hipLaunchKernelGGL((brick_march_sig_kernel<dt, sg + kSigNatural + kSigJoint>), grid, block, lds, s, F, Q, PP); \
+        else if(Q.joint)                                                                                                \
+            hipLaunchKernelGGL((brick_march_sig_kernel<dt, sg + kSigJoint>), grid, block, lds, s, F, Q, PP);            \
+        else if(natural)                                                                                                \
+            hipLaunchKernelGGL((brick_march_sig_kernel<dt, sg + kSigNatural>), grid, block, lds, s, F, Q, PP);          \
+        else                                                                                                            \
+            hipLaunchKernelGGL((brick_march_sig_kernel<dt, sg>), grid, block, lds, s, F, Q, PP);                        \
+        return hipGetLastError();
 #define ISAAC_SIG_CASE(dt, k, sg)                                                                                       \
     case dt * 8 + k:                                                                                                    \
         if(natural)                                                                                                     \
@@ -899,14 +944,15 @@ namespace isaac_hip
                 ISAAC_SIG_CASE(0, 4, 16)
                 ISAAC_SIG_CASE(1, 0, 1)
                 ISAAC_SIG_CASE(1, 1, 3)
-                ISAAC_SIG_CASE(1, 2, 6)
-                ISAAC_SIG_CASE(1, 3, 8)
-                ISAAC_SIG_CASE(1, 4, 16)
+                ISAAC_SIG_JOINT_CASE(1, 2, 6)
+                ISAAC_SIG_JOINT_CASE(1, 3, 8)
+                ISAAC_SIG_JOINT_CASE(1, 4, 16)
                 ISAAC_SIG_CASE(2, 0, 1)
                 ISAAC_SIG_CASE(2, 1, 3)
-                ISAAC_SIG_CASE(2, 2, 6)
-                ISAAC_SIG_CASE(2, 3, 8)
-                ISAAC_SIG_CASE(2, 4, 16)
+                ISAAC_SIG_JOINT_CASE(2, 2, 6)
+                ISAAC_SIG_JOINT_CASE(2, 3, 8)
+                ISAAC_SIG_JOINT_CASE(2, 4, 16)
+#undef ISAAC_SIG_JOINT_CASE
 #undef ISAAC_SIG_CASE
             default: break;
             }
@@ -934,29 +980,44 @@ namespace isaac_hip
     {
         if(B.nframes <= 0 || grid <= 0)
             return hipSuccess;
-        const bool natural = sig_natural(sig);
+        const bool natural = sig_natural(sig), joint = sig_joint(sig);
         sig %= kSigNatural;
         if(linear && (sig == 1 || sig == 3 || sig == 16))
         {
             const int k = dtype * 3 + (sig == 1 ? 0 : sig == 3 ? 1 : 2);
             switch(k)
             {
+#define ISAAC_BATCH_LAUNCH(dt, sg)                                                                                      \
+    hipLaunchKernelGGL((batch_march_kernel<dt, true, sg>), dim3(grid), dim3(256), lds, s, B.frames, B.posts, B.parts, B.order, B)
+#define ISAAC_SIG_JOINT_CASE(dt, j, sg)                                                                                 \
+    case dt * 3 + j:                                                                                                    \
+        if(joint && natural)                                                                                            \
+            ISAAC_BATCH_LAUNCH(dt, sg + kSigNatural + kSigJoint);                                                       \
+        else if(joint)                                                                                                  \
+            ISAAC_BATCH_LAUNCH(dt, sg + kSigJoint);                                                                     \
+        else if(natural)                                                                                                \
+            ISAAC_BATCH_LAUNCH(dt, sg + kSigNatural);                                                                   \
+        else                                                                                                            \
+            ISAAC_BATCH_LAUNCH(dt, sg);                                                                                 \
+        return hipGetLastError();
 #define ISAAC_SIG_CASE(dt, j, sg)                                                                                       \
     case dt * 3 + j:                                                                                                    \
         if(natural)                                                                                                     \
-            hipLaunchKernelGGL((batch_march_kernel<dt, true, sg + kSigNatural>), dim3(grid), dim3(256), lds, s, B.frames, B.posts, B.parts, B.order, B);     \
+            ISAAC_BATCH_LAUNCH(dt, sg + kSigNatural);                                                                   \
         else                                                                                                            \
-            hipLaunchKernelGGL((batch_march_kernel<dt, true, sg>), dim3(grid), dim3(256), lds, s, B.frames, B.posts, B.parts, B.order, B);                   \
+            ISAAC_BATCH_LAUNCH(dt, sg);                                                                                 \
         return hipGetLastError();
                 ISAAC_SIG_CASE(0, 0, 1)
                 ISAAC_SIG_CASE(0, 1, 3)
                 ISAAC_SIG_CASE(0, 2, 16)
                 ISAAC_SIG_CASE(1, 0, 1)
                 ISAAC_SIG_CASE(1, 1, 3)
-                ISAAC_SIG_CASE(1, 2, 16)
+                ISAAC_SIG_JOINT_CASE(1, 2, 16)
                 ISAAC_SIG_CASE(2, 0, 1)
                 ISAAC_SIG_CASE(2, 1, 3)
-                ISAAC_SIG_CASE(2, 2, 16)
+                ISAAC_SIG_JOINT_CASE(2, 2, 16)
+#undef ISAAC_SIG_JOINT_CASE
+#undef ISAAC_BATCH_LAUNCH
 #undef ISAAC_SIG_CASE
             default: break;
             }

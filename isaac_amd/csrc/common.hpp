@@ -23,6 +23,7 @@ namespace isaac_hip
     // its natural one (none for a scalar source, one `length` for a vector source),
     // evaluated inline in the interpreter's operation order instead of interpreted
     constexpr int kSigNatural = 1000;
+    constexpr int kSigJoint = 2 * kSigNatural; // added where the sources share joint rows
     // The march tests iso alphas only in iso cells that the classification marked: cells of 8^3
     // base texels.  (4^3 cells would double the steps of the walk through them, 16^3 ones would
     // double the steps tested in front of every surface.)
@@ -137,6 +138,10 @@ namespace isaac_hip
     // any sample come from one brick with 4 aligned pair loads per component.  Pairs
     // are float2 (F32) or two 16-bit values (F16, BF16) holding v / scale, with one
     // FP32 scale per brick and component.
+    //
+    // Two enabled sources of 1 and 1, 1 and 3 or 3 and 1 components in a 16-bit form share
+    // joint rows, the components of both side by side: their samples lie at the same
+    // place, and a gather instruction costs the same whether it fetches 4 bytes or 16.
     constexpr int kBrick = 8;
     constexpr int kBrickPairs = 8 * 9 * 9;
     constexpr int kMaxBrickSources = 4;
@@ -144,9 +149,10 @@ namespace isaac_hip
 
     struct BrickSource
     {
-        const void* data; // [brick][648 pair rows][component]
-        const float* scale; // [brick][component]
+        const void* data; // [brick][648 pair rows] rows of `stride` words, component at its first
+        const float* scale; // [brick] rows of scaleStride
         int32_t dim;
+        int32_t stride, scaleStride;
         int32_t active; // weight + iso > 0
         float weight;
         float iso;
@@ -161,6 +167,7 @@ namespace isaac_hip
         int32_t dtype; // ISAAC_HIP_F32 / F16 / BF16
         int32_t nbx, nby, nbz;
         int32_t off32; // every source's bricks span < 4 GiB: 32-bit byte offsets
+        int32_t joint; // src[0] and src[1] are all components of the joint rows
         float invTotalWeight; // 1 / sum of volume-source weights (0 if that sum is 0)
         int32_t T;
         const float4* luts; // all sources' transfer functions, T entries each

@@ -26,6 +26,8 @@ namespace isaac_hip
         int64_t nbricks = 0;
         int brickDim = 0;
         bool bricked = false; // bricks hold the source as of the last update_buffers
+        int jointAt = -1; // they are joint rows, from this component on
+        bool ownBricks = false; // brick and brickScale hold them (too)
         uint8_t* adv[2] = {nullptr, nullptr}; // field source: advection textures (current, history)
         int advCur = 0;
         size_t advVox = 0;
@@ -118,6 +120,14 @@ struct isaac_hip_ctx
     int builtTexLayout = -1; // tuneTexLayout at the last combined-form update_buffers
     int form = ISAAC_HIP_FORM_COMBINED;
     int brickDtype = ISAAC_HIP_F32;
+    // joint rows of two sources (common.hpp): jointDim components, 0 if the last
+    // update_buffers made none.  ownBricksWanted: get_bricks was asked for a source's own
+    // arrays, which are kept up from then on
+    void* joint = nullptr;
+    float* jointScale = nullptr;
+    size_t jointBytes = 0, jointScaleCount = 0;
+    int jointDim = 0;
+    bool ownBricksWanted = false;
     int builtForm = -1; // form prepared by the last update_buffers
     bool floatOut = false;
     float4* outFloat = nullptr;

@@ -441,10 +441,38 @@ namespace
         return 0;
     }
 
+    int64_t brick_count(const isaac_hip_ctx* c)
+    {
+        return ((c->local[0] + 7) / 8) * ((c->local[1] + 7) / 8) * ((c->local[2] + 7) / 8);
+    }
+
+    void free_bricks(isaac_hip_ctx* c, VolSlot& v)
+    {
+        if(!v.brick && !v.brickScale)
+            return;
+        (void) hipFree(v.brick);
+        (void) hipFree(v.brickScale);
+        v.brick = nullptr;
+        v.brickScale = nullptr;
+        v.brickBytes = v.scaleCount = 0;
+        c->generation++;
+    }
+
+    void free_joint(isaac_hip_ctx* c)
+    {
+        if(!c->joint && !c->jointScale)
+            return;
+        (void) hipFree(c->joint);
+        (void) hipFree(c->jointScale);
+        c->joint = nullptr;
+        c->jointScale = nullptr;
+        c->jointBytes = c->jointScaleCount = 0;
+        c->generation++;
+    }
+
     int ensure_bricks(isaac_hip_ctx* c, VolSlot& v, int dim)
     {
-        const int64_t nbx = (c->local[0] + 7) / 8, nby = (c->local[1] + 7) / 8, nbz = (c->local[2] + 7) / 8;
-        const int64_t nb = nbx * nby * nbz;
+        const int64_t nb = brick_count(c);
         const size_t pairBytes = c->brickDtype == ISAAC_HIP_F32 ? 8 : 4;
         const size_t bytes = size_t(nb) * size_t(dim) * size_t(kBrickPairs) * pairBytes;
         const size_t ns = size_t(nb) * size_t(dim);
@@ -452,20 +480,37 @@ namespace
             return fail(c, ISAAC_HIP_ERR_UNSUPPORTED, "brick form: more than 2^32 pairs per source (32-bit pair index)");
         if(v.brick && v.brickBytes == bytes && v.scaleCount == ns)
             return 0;
-        if(v.brick)
-            (void) hipFree(v.brick);
-        if(v.brickScale)
-            (void) hipFree(v.brickScale);
-        v.brick = nullptr;
-        v.brickScale = nullptr;
-        v.brickBytes = v.scaleCount = 0;
+        free_bricks(c, v);
         c->generation++;
         HIPCHK(c, hipMalloc(&v.brick, std::max<size_t>(bytes, 8)));
         HIPCHK(c, hipMalloc(&v.brickScale, std::max<size_t>(ns, 1) * 4));
         v.brickBytes = bytes;
         v.scaleCount = ns;
-        v.nbricks = nb;
-        v.brickDim = dim;
+        return 0;
+    }
+
+    int ensure_joint(isaac_hip_ctx* c, int dim)
+    {
+        const size_t ns = size_t(brick_count(c)) * size_t(dim), bytes = ns * size_t(kBrickPairs) * 4;
+        if(c->joint && c->jointBytes == bytes && c->jointScaleCount == ns)
+            return 0;
+        free_joint(c);
+        c->generation++;
+        HIPCHK(c, hipMalloc(&c->joint, std::max<size_t>(bytes, 8)));
+        HIPCHK(c, hipMalloc(&c->jointScale, std::max<size_t>(ns, 1) * 4));
+        c->jointBytes = bytes;
+        c->jointScaleCount = ns;
+        return 0;
+    }
+
+    // a source's own arrays from its joint rows
+    int split_joint(isaac_hip_ctx* c, VolSlot& v)
+    {
+        if(int rc = ensure_bricks(c, v, v.brickDim))
+            return rc;
+        HIPCHK(c, launch_brick_split(c->joint, c->jointScale, c->jointDim, v.jointAt, v.brickDim, v.nbricks, v.brick, v.brickScale,
+                                     c->stream));
+        v.ownBricks = true;
         return 0;
     }
 
@@ -714,6 +759,7 @@ namespace isaac_hip
             for(int s = 0; s < nvf; s++)
                 tw += c->weight[s];
             Q.invTotalWeight = tw != 0.0f ? 1.0f / tw : 0.0f;
+            int jointDims = 0;
             for(int s = 0; s < nvf; s++)
             {
                 const VolSlot& v = c->vols[s];
@@ -722,9 +768,13 @@ namespace isaac_hip
                 if(!v.bricked)
                     return fail(c, ISAAC_HIP_ERR_STATE, "source " + std::to_string(s) + " enabled after update_buffers; call it again");
                 BrickSource& B = Q.src[Q.nsrc++];
-                B.data = v.brick;
-                B.scale = v.brickScale;
+                const bool joint = v.jointAt >= 0;
+                B.data = joint ? static_cast<const uint32_t*>(c->joint) + v.jointAt : v.brick;
+                B.scale = joint ? c->jointScale + v.jointAt : v.brickScale;
                 B.dim = v.brickDim;
+                B.stride = joint ? c->jointDim : (c->brickDtype == ISAAC_HIP_F32 ? 2 : 1) * v.brickDim;
+                B.scaleStride = joint ? c->jointDim : v.brickDim;
+                jointDims += joint ? v.brickDim : 0;
                 B.active = 1;
                 B.weight = c->weight[s];
                 B.iso = c->iso[s];
@@ -734,8 +784,10 @@ namespace isaac_hip
             }
             Q.off32 = 1;
             for(int s = 0; s < nvf; s++)
-                if(c->vols[s].bricked && c->vols[s].brickBytes > 0xffffffffull)
+                if(c->vols[s].bricked && (c->vols[s].jointAt >= 0 ? c->jointBytes : c->vols[s].brickBytes) > 0xffffffffull)
                     Q.off32 = 0;
+            // (either of the two may have been switched off since)
+            Q.joint = c->jointDim > 0 && jointDims == c->jointDim ? 1 : 0;
             // the enabled sources' transfer functions are staged in LDS (64 KiB per workgroup)
             if(size_t(Q.nsrc) * size_t(T) * sizeof(float4) > 64 * 1024)
                 return fail(c, ISAAC_HIP_ERR_UNSUPPORTED, "brick form: enabled sources x transfer size above 4096 entries");
@@ -971,14 +1023,12 @@ extern "C"
         {
             if(v.npTex)
                 (void) hipFree(v.npTex);
-            if(v.brick)
-                (void) hipFree(v.brick);
-            if(v.brickScale)
-                (void) hipFree(v.brickScale);
+            free_bricks(c, v);
             for(uint8_t* a : v.adv)
                 if(a)
                     (void) hipFree(a);
         }
+        free_joint(c);
         for(auto& p : c->parts)
             free_part(p);
         aonet_destroy(c);
@@ -1405,43 +1455,81 @@ extern "C"
         {
             // brick form: re-lay every enabled volume/field source (the raw
             // source when persistent, its functor-applied texture otherwise)
+            BrickBuildSource src[kMaxBrickSources];
+            VolSlot* slots[kMaxBrickSources];
             int active = 0;
             for(int s = 0; s < nvf; s++)
             {
                 VolSlot& v = c->vols[s];
-                v.bricked = false;
+                v.bricked = v.ownBricks = false;
+                v.jointAt = -1;
+            }
+            c->jointDim = 0;
+            for(int s = 0; s < nvf; s++)
+            {
+                VolSlot& v = c->vols[s];
                 if(!v.set || c->weight[s] + c->iso[s] <= 0.0f)
                     continue;
                 if(s >= c->nv)
                     return fail(c, ISAAC_HIP_ERR_UNSUPPORTED, "brick form: field sources (advection) render in the combined form");
-                if(++active > kMaxBrickSources)
+                if(active == kMaxBrickSources)
                     return fail(c, ISAAC_HIP_ERR_UNSUPPORTED, "brick form: at most 4 enabled volume/field sources");
-                const float* src;
-                int64_t st[3];
-                int dim;
+                BrickBuildSource& B = src[active];
+                slots[active++] = &v;
                 if(v.desc.persistent)
                 {
-                    src = (const float*) v.desc.data;
-                    dim = v.desc.feature_dim;
+                    B.src = (const float*) v.desc.data;
+                    B.dim = v.desc.feature_dim;
                     for(int k = 0; k < 3; k++)
-                        st[k] = v.desc.stride[k];
+                        B.stride[k] = v.desc.stride[k];
                 }
                 else
                 {
                     const int64_t g = v.desc.guard_size;
                     const int64_t gX = c->local[0] + 2 * g, gY = c->local[1] + 2 * g;
-                    src = v.npTex + (g + g * gX + g * gX * gY);
-                    dim = 1;
-                    st[0] = 1;
-                    st[1] = gX;
-                    st[2] = gX * gY;
+                    B.src = v.npTex + (g + g * gX + g * gX * gY);
+                    B.dim = 1;
+                    B.stride[0] = 1;
+                    B.stride[1] = gX;
+                    B.stride[2] = gX * gY;
                 }
-                int rc = ensure_bricks(c, v, dim);
-                if(rc)
+                v.nbricks = brick_count(c);
+                v.brickDim = B.dim;
+            }
+            const int X = int(c->local[0]), Y = int(c->local[1]), Z = int(c->local[2]);
+            // joint rows: 2 or 4 words, so that a row is one aligned load, and < 4 GiB, so that
+            // the march's 32-bit offsets reach them
+            const int dims = active == 2 ? src[0].dim + src[1].dim : 0;
+            const bool joint = c->brickDtype != ISAAC_HIP_F32 && (dims == 2 || (dims == 4 && src[0].dim != 2))
+                && uint64_t(brick_count(c)) * kBrickPairs * uint64_t(dims) * 4 <= 0xffffffffull;
+            if(joint)
+            {
+                if(int rc = ensure_joint(c, dims))
                     return rc;
-                HIPCHK(c, launch_bricks(src, st, dim, int(c->local[0]), int(c->local[1]), int(c->local[2]), c->brickDtype,
-                                        v.brickScale, v.brick, c->stream));
-                v.bricked = true;
+                HIPCHK(c, launch_bricks(src, 2, X, Y, Z, c->brickDtype, c->jointScale, c->joint, c->stream));
+                c->jointDim = dims;
+                for(int i = 0; i < 2; i++)
+                {
+                    slots[i]->jointAt = i ? src[0].dim : 0;
+                    slots[i]->bricked = true;
+                }
+            }
+            else
+                free_joint(c);
+            for(int i = 0; i < active; i++)
+            {
+                VolSlot& v = *slots[i];
+                if(!joint)
+                {
+                    if(int rc = ensure_bricks(c, v, v.brickDim))
+                        return rc;
+                    HIPCHK(c, launch_bricks(src + i, 1, X, Y, Z, c->brickDtype, v.brickScale, v.brick, c->stream));
+                    v.bricked = v.ownBricks = true;
+                }
+                else if(!c->ownBricksWanted)
+                    free_bricks(c, v);
+                else if(int rc = split_joint(c, v))
+                    return rc;
             }
             // the particle records after the GPU-heavy brick build, so the host enqueues
             // their short launches while the build runs
@@ -1774,6 +1862,16 @@ extern "C"
         if(!c || source < 0 || source >= c->nv + c->nf)
             return ISAAC_HIP_ERR_ARG;
         const VolSlot& v = c->vols[source];
+        if(v.bricked && !v.ownBricks)
+        {
+            // from joint rows on the first request, kept up by update_buffers afterwards
+            isaac_hip_ctx* m = const_cast<isaac_hip_ctx*>(c);
+            HIPCHK(m, hipSetDevice(c->device));
+            m->ownBricksWanted = true;
+            if(int rc = split_joint(m, m->vols[source]))
+                return rc;
+            HIPCHK(m, hipStreamSynchronize(c->stream));
+        }
         if(pairs)
             *pairs = v.bricked ? v.brick : nullptr;
         if(scales)

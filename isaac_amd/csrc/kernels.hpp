@@ -28,19 +28,22 @@ namespace isaac_hip
     hipError_t launch_shade(const FrameParams& F, hipStream_t s);
 
     // ---- precision form: field bricks and the post-classification march
-    // src: local voxel (0,0,0) of an AoS float source (dim components, element strides);
-    // scale: nbricks*dim floats; out: nbricks*dim*648 pairs (float2 or 2 x 16 bit)
+    // a source of the brick build: local voxel (0,0,0) of an AoS float source (dim
+    // components, element strides)
+    struct BrickBuildSource
+    {
+        const float* src;
+        int64_t stride[3];
+        int32_t dim;
+    };
+    // the bricks of one source, or the joint rows of two (16-bit forms; 1 and 1, 1 and 3 or 3
+    // and 1 components): scale: nbricks*dim floats; out: nbricks*648*dim pairs (float2 or 2 x
+    // 16 bit), dim the sum over the sources
     hipError_t launch_bricks(
-        const float* src,
-        const int64_t stride[3],
-        int dim,
-        int X,
-        int Y,
-        int Z,
-        int dtype,
-        float* scale,
-        void* out,
-        hipStream_t s);
+        const BrickBuildSource* sources, int nsources, int X, int Y, int Z, int dtype, float* scale, void* out, hipStream_t s);
+    // components at..at+dim-1 of joint rows of jointDim components as a source's own bricks
+    hipError_t launch_brick_split(
+        const void* joint, const float* jointScale, int jointDim, int at, int dim, int64_t nbricks, void* out, float* scale, hipStream_t s);
     // batched form: the persistent march over all frames (grid = persistent workgroups),
     // then SSAO and shading over a (maxTiles, nframes) grid
     hipError_t launch_batch_march(const BatchParams& B, int dtype, bool linear, int sig, size_t lds, int grid, hipStream_t s);

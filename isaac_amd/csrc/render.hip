@@ -392,150 +392,6 @@ namespace isaac_hip
         shade_body(frames[blockIdx.y], blockIdx.x);
     }
 
-
-    // per brick and component: scale = max |v| over the 9^3 region (1 if all zero)
-    __device__ inline uint32_t to_bf16_rne(float f)
-    {
-        const uint32_t u = __float_as_uint(f);
-        if((u & 0x7f800000u) == 0x7f800000u)
-            return (u >> 16) | ((u & 0xffffu) ? 0x40u : 0u); // inf / nan
-        return (u + 0x7fffu + ((u >> 16) & 1u)) >> 16;
-    }
-
-    // One workgroup per brick: the brick's 9^3 region (x, y, z clamped to the local
-    // box) of all DIM components is read once into LDS; wave c < DIM reduces the
-    // max |v| of component c (the brick scale: 1 when the region is all zero or the
-    // form is FP32); then every thread writes pairs (v[x], v[x+1]) of the region,
-    // divided by the scale and rounded for 16-bit forms.  Output element
-    // (brick*648 + pair)*DIM + c, pair = (lz*9 + ly)*8 + lx.
-    template<int DT, int DIM>
-    __global__ __launch_bounds__(256) void brick_build_kernel(
-        const float* src,
-        int64_t sx,
-        int64_t sy,
-        int64_t sz,
-        int X,
-        int Y,
-        int Z,
-        int nbx,
-        int nby,
-        float* scale,
-        void* out)
-    {
-        __shared__ float reg[729 * DIM];
-        __shared__ float sc[DIM], rc[DIM];
-        __shared__ int64_t rowOff[81]; // element offset of region row (ly, lz), x = 0
-        const int64_t brick = blockIdx.x;
-        const int Bx = int(brick % nbx), By = int((brick / nbx) % nby), Bz = int(brick / (int64_t(nbx) * nby));
-        if(threadIdx.x < 81)
-        {
-            const int lz = int(threadIdx.x) / 9, ly = int(threadIdx.x) - lz * 9;
-            const int y = min(By * 8 + ly, Y - 1), z = min(Bz * 8 + lz, Z - 1);
-            rowOff[threadIdx.x] = (int64_t(y) * sy + int64_t(z) * sz) * DIM;
-        }
-        __syncthreads();
-        const int x0 = Bx * 8, xLast = X - 1 - x0; // last local x inside the box
-        const int64_t sxD = sx * DIM;
-        for(int i = threadIdx.x; i < 729 * DIM; i += 256)
-        {
-            const int vox = i / DIM, c = i - vox * DIM;
-            const int row = vox / 9, lx = vox - row * 9;
-            const int x = x0 + min(lx, xLast);
-            reg[i] = src[rowOff[row] + int64_t(x) * sxD + c];
-        }
-        __syncthreads();
-        const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-        if(wave < DIM)
-        {
-            float m = 0.0f;
-            if(DT != kDtF32)
-                for(int vox = lane; vox < 729; vox += 64)
-                    m = fmaxf(m, fabsf(reg[vox * DIM + wave]));
-            for(int off = 32; off > 0; off >>= 1)
-                m = fmaxf(m, __shfl_xor(m, off));
-            const float s = m > 0.0f ? m : 1.0f;
-            if(lane == 0)
-            {
-                sc[wave] = s;
-                // RN(1/s) for the quotients, 0 where s is outside [2^-60, 2^60] (there
-                // the quotients take the IEEE division)
-                rc[wave] = (s >= 0x1p-60f && s <= 0x1p+60f) ? 1.0f / s : 0.0f;
-                scale[brick * DIM + wave] = s;
-            }
-        }
-        __syncthreads();
-        for(int e = threadIdx.x; e < kBrickPairs * DIM; e += 256)
-        {
-            const int pair = e / DIM, c = e - pair * DIM;
-            const int vox0 = (pair >> 3) * 9 + (pair & 7);
-            const float v0 = reg[vox0 * DIM + c], v1 = reg[(vox0 + 1) * DIM + c];
-            const int64_t i = brick * (kBrickPairs * DIM) + e;
-            if(DT == kDtF32)
-                reinterpret_cast<float2*>(out)[i] = make_float2(v0, v1);
-            else
-            {
-                // v / s as x*r plus one fma residual step (div_by), with v's sign (the
-                // residual step turns -0 into +0): the IEEE quotient for |v| <= s with s in
-                // [2^-60, 2^60]; for BF16, whose range keeps tiny quotients, only where
-                // |v| >= 2^-60 (the residual stays normal)
-                const float s = sc[c], r = rc[c];
-                auto quot = [&](float v) {
-                    const bool fast = r != 0.0f && (DT == kDtF16 || fabsf(v) >= 0x1p-60f);
-                    return fast ? copysignf(div_by(v, s, r), v) : v / s;
-                };
-                const float q0 = quot(v0), q1 = quot(v1);
-                uint32_t w;
-                if(DT == kDtF16)
-                    w = uint32_t(__half_as_ushort(__float2half_rn(q0))) | (uint32_t(__half_as_ushort(__float2half_rn(q1))) << 16);
-                else
-                    w = to_bf16_rne(q0) | (to_bf16_rne(q1) << 16);
-                reinterpret_cast<uint32_t*>(out)[i] = w;
-            }
-        }
-    }
-
-    template<int DT>
-    hipError_t launch_brick_build(
-        const float* src, const int64_t stride[3], int dim, int X, int Y, int Z, int nbx, int nby, int64_t nbricks, float* scale,
-        void* out, hipStream_t s)
-    {
-        const dim3 grid = dim3(static_cast<unsigned>(nbricks)), block = dim3(256);
-        switch(dim)
-        {
-        case 1: hipLaunchKernelGGL((brick_build_kernel<DT, 1>), grid, block, 0, s, src, stride[0], stride[1], stride[2], X, Y, Z, nbx, nby, scale, out); break;
-        case 2: hipLaunchKernelGGL((brick_build_kernel<DT, 2>), grid, block, 0, s, src, stride[0], stride[1], stride[2], X, Y, Z, nbx, nby, scale, out); break;
-        case 3: hipLaunchKernelGGL((brick_build_kernel<DT, 3>), grid, block, 0, s, src, stride[0], stride[1], stride[2], X, Y, Z, nbx, nby, scale, out); break;
-        case 4: hipLaunchKernelGGL((brick_build_kernel<DT, 4>), grid, block, 0, s, src, stride[0], stride[1], stride[2], X, Y, Z, nbx, nby, scale, out); break;
-        default: return hipErrorInvalidValue;
-        }
-        return hipGetLastError();
-    }
-
-    hipError_t launch_bricks(
-        const float* src,
-        const int64_t stride[3],
-        int dim,
-        int X,
-        int Y,
-        int Z,
-        int dtype,
-        float* scale,
-        void* out,
-        hipStream_t s)
-    {
-        const int nbx = (X + 7) / 8, nby = (Y + 7) / 8, nbz = (Z + 7) / 8;
-        const int64_t nbricks = int64_t(nbx) * nby * nbz;
-        if(nbricks == 0)
-            return hipSuccess;
-        if(nbricks > int64_t(0x7fffffff))
-            return hipErrorInvalidValue;
-        if(dtype == kDtF32)
-            return launch_brick_build<kDtF32>(src, stride, dim, X, Y, Z, nbx, nby, nbricks, scale, out, s);
-        if(dtype == kDtF16)
-            return launch_brick_build<kDtF16>(src, stride, dim, X, Y, Z, nbx, nby, nbricks, scale, out, s);
-        return launch_brick_build<kDtBf16>(src, stride, dim, X, Y, Z, nbx, nby, nbricks, scale, out, s);
-    }
-
     hipError_t launch_batch_ssao(const FrameParams* frames, int nframes, int maxTiles, hipStream_t s)
     {
         if(nframes <= 0 || maxTiles <= 0)

@@ -490,7 +490,12 @@ namespace isaac_hip
     // before interpolating any of them, so their latencies overlap.
     constexpr bool sig_natural(int sig)
     {
-        return sig >= kSigNatural;
+        return sig % kSigJoint >= kSigNatural;
+    }
+
+    constexpr bool sig_joint(int sig)
+    {
+        return sig >= kSigJoint;
     }
 
     constexpr int sig_count(int sig)

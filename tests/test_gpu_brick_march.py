@@ -26,6 +26,7 @@ def _spec(size, sources, fb=(141, 99), step=0.5, pose=scenes.FILL_POSE):
     vec = rng.uniform(-0.6, 0.6, (Z, Y, X, 3)).astype(np.float32)
     vols = {"density": scenes.VolumeSourceSpec("density", dens, "idem", list(scenes.DENSITY_TF), 2.0, 0.4),
             "vector": scenes.VolumeSourceSpec("vector", vec, "length", list(scenes.VECTOR_TF), 2.0, 0.0),
+            "soft": scenes.VolumeSourceSpec("soft", np.ascontiguousarray(1.0 - dens), "idem", list(scenes.DENSITY_TF), 1.5, 0.0),
             "scaled": scenes.VolumeSourceSpec("scaled", vec, "length | mul(0.8)", list(scenes.VECTOR_TF), 1.0, 0.0)}
     return scenes.SceneSpec("bricks", tuple(size), tuple(size), (1, 1, 1), framebuffer=fb, volumes=[vols[s] for s in sources],
                             step=step, interpolation=True, camera=pose)
@@ -69,3 +70,52 @@ def test_batch_frames_of_any_size(fb):
     b.close()
     for v in vises:
         v.close()
+
+
+@pytest.mark.parametrize("dtype", ["F16", "BF16"])
+@pytest.mark.parametrize("sources", [("density", "vector"), ("scaled", "density"), ("density", "soft")])
+@pytest.mark.parametrize("size", [(1, 1, 1), (8, 9, 7), (17, 16, 24), (41, 8, 33)])
+def test_joint_rows_equal_rows_of_one_source(size, sources, dtype):
+    """Two sources in joint rows against the same two in rows of their own (update_buffers
+    with a third source enabled keeps every source apart; it is switched off after it), one
+    of two joined sources against the same in its own rows, and the arrays that bricks()
+    gives for a joined source before and after another update against those of its own."""
+    from isaac_amd import visualization as V
+
+    spec = _spec(size, sources + ("vector",))
+    spec.volumes[2] = dataclasses.replace(spec.volumes[2], name="third")
+    vis = V.from_scene(spec)
+    vis.set_render_form(vis.FORM_BRICKS, getattr(vis, dtype))
+    weights, iso = list(vis.source_weight), list(vis.iso_threshold)
+
+    def enable(slots):
+        vis.source_weight = [w if i in slots else 0.0 for i, w in enumerate(weights)]
+        vis.iso_threshold = [t if i in slots else 0.0 for i, t in enumerate(iso)]
+
+    def frame():
+        img = vis.draw()
+        return [img] + [a.copy() for a in vis.gbuffer()]
+
+    def same(a, b):
+        return all(np.array_equal(x, y) for x, y in zip(a, b))
+
+    enable((0, 1, 2))
+    vis.update_buffers()
+    own = [vis.bricks(i) for i in (0, 1)]
+    want = {}
+    for slots in ((0, 1), (0,), (1,)):
+        enable(slots)
+        want[slots] = frame()
+    enable((0, 1))
+    vis.update_buffers()
+    for slots in want:
+        enable(slots)
+        assert same(frame(), want[slots]), slots
+    enable((0, 1))
+    for again in range(3):
+        for i in (0, 1):
+            pairs, scales = vis.bricks(i)
+            assert np.array_equal(pairs, own[i][0]) and np.array_equal(scales, own[i][1]), (again, i)
+        vis.update_buffers()
+        assert same(frame(), want[(0, 1)])
+    vis.close()
