@@ -236,36 +236,6 @@ def measure(vis, poses, out, steps, warmup, instrumented=None):
     return wall, total_samples, avg_us, avg_counts, counts
 
 
-def tex_layout_study(vis, poses, frames=6):
-    """March time and classification time (which holds the brick copy, or the binary16
-    copy's stores) of each texture layout at the tuned schedule, per pose; medians over
-    `frames` updated frames."""
-    import numpy as np
-
-    keep = vis.tex_layout
-    res = {}
-    for layout in (0, 8, 16):
-        vis.set_tuning(vis.TUNE_TEX_LAYOUT, layout)
-        vis.update_buffers()
-        per = {}
-        for name, p in zip(("default", "fill"), poses):
-            set_pose_of(vis, p)
-            vis.update_buffers()
-            vis.draw(out=False)
-            m, c = [], []
-            for _ in range(frames):
-                vis.update_buffers()
-                vis.draw(out=False)
-                t = vis.timings()
-                m.append(t["march_us"])
-                c.append(t["optimization_buffer_us"])
-            per[name] = {"march_us": float(np.median(m)), "classify_us": float(np.median(c))}
-        res[f"layout={layout}"] = per
-    vis.set_tuning(vis.TUNE_TEX_LAYOUT, keep)
-    vis.update_buffers()
-    return res
-
-
 def learned_ao(vis, poses, out, args):
     """Train the occlusion network on the GPU from plain-SSAO triples of 16 scenes of
     this workload's style and size with other seeds (fields, particles, clipping
@@ -597,7 +567,6 @@ def main() -> int:
 
         vis.update_buffers()
         tuning = autotune.tune_march(vis, poses)
-        tuning["tex_layout_study"] = tex_layout_study(vis, poses)
     instrumented = {}
     wall, total_samples, avg_us, avg_counts, counts = measure(vis, poses, out, args.steps, args.warmup, instrumented)
     ms_per_step = wall / args.steps * 1e3
