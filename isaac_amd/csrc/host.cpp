@@ -470,10 +470,8 @@ namespace
         c->generation++;
     }
 
-    int ensure_bricks(isaac_hip_ctx* c, VolSlot& v, int dim)
+    int ensure_bricks(isaac_hip_ctx* c, VolSlot& v, int64_t nb, int dim, size_t pairBytes)
     {
-        const int64_t nb = brick_count(c);
-        const size_t pairBytes = c->brickDtype == ISAAC_HIP_F32 ? 8 : 4;
         const size_t bytes = size_t(nb) * size_t(dim) * size_t(kBrickPairs) * pairBytes;
         const size_t ns = size_t(nb) * size_t(dim);
         if(uint64_t(ns) * uint64_t(kBrickPairs) >= (uint64_t(1) << 32))
@@ -503,10 +501,11 @@ namespace
         return 0;
     }
 
-    // a source's own arrays from its joint rows
+    // a source's own arrays from its joint rows, of the size and type the rows were built in (the
+    // context's local size and brick type may have changed since)
     int split_joint(isaac_hip_ctx* c, VolSlot& v)
     {
-        if(int rc = ensure_bricks(c, v, v.brickDim))
+        if(int rc = ensure_bricks(c, v, v.nbricks, v.brickDim, 4))
             return rc;
         HIPCHK(c, launch_brick_split(c->joint, c->jointScale, c->jointDim, v.jointAt, v.brickDim, v.nbricks, v.brick, v.brickScale,
                                      c->stream));
@@ -1521,7 +1520,7 @@ extern "C"
                 VolSlot& v = *slots[i];
                 if(!joint)
                 {
-                    if(int rc = ensure_bricks(c, v, v.brickDim))
+                    if(int rc = ensure_bricks(c, v, v.nbricks, v.brickDim, c->brickDtype == ISAAC_HIP_F32 ? 8 : 4))
                         return rc;
                     HIPCHK(c, launch_bricks(src + i, 1, X, Y, Z, c->brickDtype, v.brickScale, v.brick, c->stream));
                     v.bricked = v.ownBricks = true;

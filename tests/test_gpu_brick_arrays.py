@@ -1,0 +1,60 @@
+"""The per-source brick arrays of isaac_hip_get_bricks and the layouts behind them (rows of
+one source, joint rows of two): what calls between a request, an update and a render may
+change, and what they leave alone."""
+import numpy as np
+import pytest
+
+from isaac_amd import scenes
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", autouse=True)
+def gpu():
+    torch = pytest.importorskip("torch")
+    if not torch.cuda.is_available():
+        pytest.skip("needs a GPU")
+
+
+def _vis(size=(24, 17, 19), count=2, dtype="F16", fb=(64, 48)):
+    """`count` sources (density, vector, soft), all enabled, in the brick form and updated."""
+    from isaac_amd import visualization as V
+
+    X, Y, Z = size
+    rng = np.random.default_rng(X * 10007 + Y * 101 + Z)
+    dens = scenes.gaussian_mixture((Z, Y, X), 5, 6, (0.1 * max(size), 0.3 * max(size))).astype(np.float32)
+    vols = [scenes.VolumeSourceSpec("density", dens, "idem", list(scenes.DENSITY_TF), 2.0, 0.4),
+            scenes.VolumeSourceSpec("vector", rng.uniform(-0.6, 0.6, (Z, Y, X, 3)).astype(np.float32), "length",
+                                    list(scenes.VECTOR_TF), 2.0, 0.0),
+            scenes.VolumeSourceSpec("soft", np.ascontiguousarray(1.0 - dens), "idem", list(scenes.DENSITY_TF), 1.5, 0.0)]
+    vis = V.from_scene(scenes.SceneSpec("arrays", tuple(size), tuple(size), (1, 1, 1), framebuffer=fb, volumes=vols[:count],
+                                        step=0.5, interpolation=True, camera=scenes.FILL_POSE))
+    vis.set_render_form(vis.FORM_BRICKS, getattr(vis, dtype))
+    vis.update_buffers()
+    return vis
+
+
+def _own(vis):
+    """What bricks() gives for both sources of an equal context without joint rows."""
+    ref = _vis(vis.local_size, 3)
+    out = [ref.bricks(i) for i in (0, 1)]
+    ref.close()
+    return out
+
+
+@pytest.mark.parametrize("change", ["smaller", "larger"])
+def test_bricks_of_the_last_update_after_a_size_change(change):
+    """Asked for between a change of the local size and the next update, joint rows are
+    split at the size they were built in."""
+    vis = _vis()
+    want = _own(vis)
+    built = vis.local_size
+    vis.update_local_size((9, 8, 7) if change == "smaller" else (64, 64, 64))
+    for i in (0, 1):
+        pairs, scales = vis.bricks(i)
+        assert np.array_equal(pairs, want[i][0]) and np.array_equal(scales, want[i][1])
+    vis.update_local_size(built)
+    vis.update_buffers()
+    for i in (0, 1):
+        assert np.array_equal(vis.bricks(i)[0], want[i][0])
+    vis.close()
