@@ -266,7 +266,7 @@ extern "C"
                 return bfail(b, ISAAC_HIP_ERR_ARG, "contexts on different devices");
             if(c->form != ISAAC_HIP_FORM_BRICKS || c->builtForm != ISAAC_HIP_FORM_BRICKS || !c->classified)
                 return bfail(b, ISAAC_HIP_ERR_STATE, "context " + std::to_string(i) + ": brick form with update_buffers done");
-            if(c->brickDtype != c0->brickDtype || c->interpolation != c0->interpolation || c->nsrc != c0->nsrc
+            if(c->brickDtype != c0->brickDtype || c->builtDtype != c0->builtDtype || c->interpolation != c0->interpolation || c->nsrc != c0->nsrc
                || c->cfg.transfer_size != c0->cfg.transfer_size || c->aoEnabled != c0->aoEnabled)
                 return bfail(b, ISAAC_HIP_ERR_ARG, "context " + std::to_string(i) + ": render state differs from context 0");
             for(int s = 0; s < c->nsrc; s++)
@@ -353,9 +353,9 @@ extern "C"
             sig += kSigJoint;
         const size_t lutLds = size_t(b->hQ[0].nsrc) * size_t(b->hQ[0].T) * sizeof(float4);
         // launch arguments the captured graph holds
-        if(c0->brickDtype != b->dtype || c0->interpolation != b->linear || sig != b->sig || lutLds != b->lutLds)
+        if(c0->builtDtype != b->dtype || c0->interpolation != b->linear || sig != b->sig || lutLds != b->lutLds)
             b->graphStale = true;
-        b->dtype = c0->brickDtype;
+        b->dtype = c0->builtDtype;
         b->linear = c0->interpolation;
         b->sig = sig;
         b->lutLds = lutLds;

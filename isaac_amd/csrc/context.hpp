@@ -120,6 +120,7 @@ struct isaac_hip_ctx
     int builtTexLayout = -1; // tuneTexLayout at the last combined-form update_buffers
     int form = ISAAC_HIP_FORM_COMBINED;
     int brickDtype = ISAAC_HIP_F32;
+    int builtDtype = ISAAC_HIP_F32; // brickDtype at the last brick-form update_buffers: what frames read
     // joint rows of two sources (common.hpp): jointDim components, 0 if the last
     // update_buffers made none.  ownBricksWanted: get_bricks was asked for a source's own
     // arrays, which are kept up from then on

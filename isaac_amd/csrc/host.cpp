@@ -748,7 +748,7 @@ namespace isaac_hip
             for(int i = 0; i < c->nclip; i++)
                 for(int k = 0; k < 3; k++)
                     Q.cposd[i][k] = double(c->clipPos[i][k]) * double(c->gsScaled[k]) * 0.5 + double(F.off[k]);
-            Q.dtype = c->brickDtype;
+            Q.dtype = c->builtDtype;
             Q.nbx = int32_t((c->local[0] + 7) / 8);
             Q.nby = int32_t((c->local[1] + 7) / 8);
             Q.nbz = int32_t((c->local[2] + 7) / 8);
@@ -771,7 +771,7 @@ namespace isaac_hip
                 B.data = joint ? static_cast<const uint32_t*>(c->joint) + v.jointAt : v.brick;
                 B.scale = joint ? c->jointScale + v.jointAt : v.brickScale;
                 B.dim = v.brickDim;
-                B.stride = joint ? c->jointDim : (c->brickDtype == ISAAC_HIP_F32 ? 2 : 1) * v.brickDim;
+                B.stride = joint ? c->jointDim : (c->builtDtype == ISAAC_HIP_F32 ? 2 : 1) * v.brickDim;
                 B.scaleStride = joint ? c->jointDim : v.brickDim;
                 jointDims += joint ? v.brickDim : 0;
                 B.active = 1;
@@ -1464,6 +1464,7 @@ extern "C"
                 v.jointAt = -1;
             }
             c->jointDim = 0;
+            c->builtDtype = c->brickDtype;
             for(int s = 0; s < nvf; s++)
             {
                 VolSlot& v = c->vols[s];
@@ -1878,7 +1879,7 @@ extern "C"
         if(nbricks)
             *nbricks = v.bricked ? v.nbricks : 0;
         if(pair_bytes)
-            *pair_bytes = c->brickDtype == ISAAC_HIP_F32 ? 8 : 4;
+            *pair_bytes = (v.bricked ? c->builtDtype : c->brickDtype) == ISAAC_HIP_F32 ? 8 : 4;
         return 0;
     }
 

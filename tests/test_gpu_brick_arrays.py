@@ -58,3 +58,31 @@ def test_bricks_of_the_last_update_after_a_size_change(change):
     for i in (0, 1):
         assert np.array_equal(vis.bricks(i)[0], want[i][0])
     vis.close()
+
+
+@pytest.mark.parametrize("count", [1, 2])
+@pytest.mark.parametrize("built,asked", [("F16", "F32"), ("F32", "F16"), ("F16", "BF16"), ("BF16", "F32")])
+def test_brick_type_takes_effect_at_the_next_update(count, built, asked):
+    """Frames, batches and bricks() between a change of the brick type and the next update
+    read the bricks in the type they were built in."""
+    from isaac_amd import batch as B
+
+    vis, other = _vis(count=count, dtype=built), _vis(count=count, dtype=asked)
+    want, after = vis.draw(), other.draw()
+    arrays = [vis.bricks(i) for i in range(count)]
+    b = B.Batch([vis], 64, 48)
+    projs, mvs = B.views_for([vis], 1, seed=2)
+    ref = vis.draw(projection=projs[0], modelview_=mvs[0])
+    vis.set_render_form(vis.FORM_BRICKS, getattr(vis, asked))
+    assert np.array_equal(vis.draw(), want)
+    for i in range(count):
+        for x, y in zip(vis.bricks(i), arrays[i]):
+            assert x.dtype == y.dtype and np.array_equal(x, y)
+    b.set_views(projs, mvs, bg=vis.background_color)
+    b.render(B.GRAPH)
+    assert np.array_equal(b.images()[0], ref)
+    vis.update_buffers()
+    assert np.array_equal(vis.draw(), after)
+    b.close()
+    vis.close()
+    other.close()
