@@ -446,16 +446,15 @@ namespace
         return ((c->local[0] + 7) / 8) * ((c->local[1] + 7) / 8) * ((c->local[2] + 7) / 8);
     }
 
-    void free_bricks(isaac_hip_ctx* c, VolSlot& v)
+    // (A source's own arrays are what frames read only where update_buffers says so, which then
+    // counts the generation: a copy made for isaac_hip_get_bricks is in no frame's parameters.)
+    void free_bricks(VolSlot& v)
     {
-        if(!v.brick && !v.brickScale)
-            return;
         (void) hipFree(v.brick);
         (void) hipFree(v.brickScale);
         v.brick = nullptr;
         v.brickScale = nullptr;
         v.brickBytes = v.scaleCount = 0;
-        c->generation++;
     }
 
     void free_joint(isaac_hip_ctx* c)
@@ -478,8 +477,7 @@ namespace
             return fail(c, ISAAC_HIP_ERR_UNSUPPORTED, "brick form: more than 2^32 pairs per source (32-bit pair index)");
         if(v.brick && v.brickBytes == bytes && v.scaleCount == ns)
             return 0;
-        free_bricks(c, v);
-        c->generation++;
+        free_bricks(v);
         HIPCHK(c, hipMalloc(&v.brick, std::max<size_t>(bytes, 8)));
         HIPCHK(c, hipMalloc(&v.brickScale, std::max<size_t>(ns, 1) * 4));
         v.brickBytes = bytes;
@@ -1022,7 +1020,7 @@ extern "C"
         {
             if(v.npTex)
                 (void) hipFree(v.npTex);
-            free_bricks(c, v);
+            free_bricks(v);
             for(uint8_t* a : v.adv)
                 if(a)
                     (void) hipFree(a);
@@ -1463,6 +1461,7 @@ extern "C"
                 v.bricked = v.ownBricks = false;
                 v.jointAt = -1;
             }
+            const int wasJoint = c->jointDim;
             c->jointDim = 0;
             c->builtDtype = c->brickDtype;
             for(int s = 0; s < nvf; s++)
@@ -1516,18 +1515,23 @@ extern "C"
             }
             else
                 free_joint(c);
+            if(c->jointDim != wasJoint)
+                c->generation++;
             for(int i = 0; i < active; i++)
             {
                 VolSlot& v = *slots[i];
                 if(!joint)
                 {
+                    const void* const was = v.brick;
                     if(int rc = ensure_bricks(c, v, v.nbricks, v.brickDim, c->brickDtype == ISAAC_HIP_F32 ? 8 : 4))
                         return rc;
+                    if(v.brick != was)
+                        c->generation++;
                     HIPCHK(c, launch_bricks(src + i, 1, X, Y, Z, c->brickDtype, v.brickScale, v.brick, c->stream));
                     v.bricked = v.ownBricks = true;
                 }
                 else if(!c->ownBricksWanted)
-                    free_bricks(c, v);
+                    free_bricks(v);
                 else if(int rc = split_joint(c, v))
                     return rc;
             }

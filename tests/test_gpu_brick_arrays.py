@@ -86,3 +86,27 @@ def test_brick_type_takes_effect_at_the_next_update(count, built, asked):
     b.close()
     vis.close()
     other.close()
+
+
+@pytest.mark.parametrize("resized", [False, True])
+def test_bricks_between_batch_renders(resized):
+    """Asking for arrays changes nothing that a batch reads: its next render is accepted and
+    gives the same frames, also where the caller's arrays are made anew at another size."""
+    from isaac_amd import batch as B
+
+    vis = _vis()
+    if resized:
+        vis.bricks(0)
+        vis.update_local_size((9, 8, 7))
+        vis.update_buffers()
+    b = B.Batch([vis], 64, 48)
+    projs, mvs = B.views_for([vis], 2, seed=2)
+    b.set_views(projs, mvs, bg=vis.background_color)
+    b.render(B.GRAPH)
+    want = b.images()
+    for i in (0, 1, 0):
+        vis.bricks(i)
+        b.render(B.GRAPH)
+        assert np.array_equal(b.images(), want), i
+    b.close()
+    vis.close()
