@@ -291,7 +291,13 @@ extern "C"
      * x fastest; pair row (lz*9 + ly)*8 + lx holds (v[x], v[x+1]) at voxel
      * (8bx+lx, 8by+ly, 8bz+lz), coordinates clamped into the local box), each pair
      * *pair_bytes (8 or 4) bytes; *scales = nbricks * feature_dim floats.  Valid after
-     * update_buffers in BRICKS form. */
+     * update_buffers in BRICKS form.  Where the march reads two sources in joint rows, the
+     * first request of a source's pointers allocates its arrays, fills them from the last
+     * update's rows and waits for the stream.  Pointers given out stay valid, and follow every
+     * update that has the source enabled, until an update at another local size, brick type
+     * or component count; keeping them up costs each update with joint rows one more pass over
+     * the source's bricks.  (nbricks and pair_bytes alone, with null pointers, cost nothing.)
+     * Not to be called while another thread uses the context. */
     int isaac_hip_get_bricks(
         const isaac_hip_ctx* ctx,
         int source,

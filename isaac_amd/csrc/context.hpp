@@ -28,6 +28,7 @@ namespace isaac_hip
         bool bricked = false; // bricks hold the source as of the last update_buffers
         int jointAt = -1; // they are joint rows, from this component on
         bool ownBricks = false; // brick and brickScale hold them (too)
+        bool ownWanted = false; // get_bricks gave brick and brickScale out: kept, and kept up to date
         uint8_t* adv[2] = {nullptr, nullptr}; // field source: advection textures (current, history)
         int advCur = 0;
         size_t advVox = 0;
@@ -122,13 +123,11 @@ struct isaac_hip_ctx
     int brickDtype = ISAAC_HIP_F32;
     int builtDtype = ISAAC_HIP_F32; // brickDtype at the last brick-form update_buffers: what frames read
     // joint rows of two sources (common.hpp): jointDim components, 0 if the last
-    // update_buffers made none.  ownBricksWanted: get_bricks was asked for a source's own
-    // arrays, which are kept up from then on
+    // update_buffers made none
     void* joint = nullptr;
     float* jointScale = nullptr;
     size_t jointBytes = 0, jointScaleCount = 0;
     int jointDim = 0;
-    bool ownBricksWanted = false;
     int builtForm = -1; // form prepared by the last update_buffers
     bool floatOut = false;
     float4* outFloat = nullptr;

@@ -1530,7 +1530,7 @@ extern "C"
                     HIPCHK(c, launch_bricks(src + i, 1, X, Y, Z, c->brickDtype, v.brickScale, v.brick, c->stream));
                     v.bricked = v.ownBricks = true;
                 }
-                else if(!c->ownBricksWanted)
+                else if(!v.ownWanted)
                     free_bricks(v);
                 else if(int rc = split_joint(c, v))
                     return rc;
@@ -1865,16 +1865,19 @@ extern "C"
     {
         if(!c || source < 0 || source >= c->nv + c->nf)
             return ISAAC_HIP_ERR_ARG;
-        const VolSlot& v = c->vols[source];
-        if(v.bricked && !v.ownBricks)
+        isaac_hip_ctx* m = const_cast<isaac_hip_ctx*>(c);
+        VolSlot& v = m->vols[source];
+        if(v.bricked && (pairs || scales))
         {
             // from joint rows on the first request, kept up by update_buffers afterwards
-            isaac_hip_ctx* m = const_cast<isaac_hip_ctx*>(c);
-            HIPCHK(m, hipSetDevice(c->device));
-            m->ownBricksWanted = true;
-            if(int rc = split_joint(m, m->vols[source]))
-                return rc;
-            HIPCHK(m, hipStreamSynchronize(c->stream));
+            if(!v.ownBricks)
+            {
+                HIPCHK(m, hipSetDevice(c->device));
+                if(int rc = split_joint(m, v))
+                    return rc;
+                HIPCHK(m, hipStreamSynchronize(c->stream));
+            }
+            v.ownWanted = true;
         }
         if(pairs)
             *pairs = v.bricked ? v.brick : nullptr;

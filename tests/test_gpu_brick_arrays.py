@@ -110,3 +110,62 @@ def test_bricks_between_batch_renders(resized):
         assert np.array_equal(b.images(), want), i
     b.close()
     vis.close()
+
+
+def _pointers(vis, source):
+    import ctypes
+
+    from isaac_amd._lib import check, lib
+
+    pairs, scales, n, size = ctypes.c_void_p(), ctypes.c_void_p(), ctypes.c_int64(), ctypes.c_int32()
+    check(lib().isaac_hip_get_bricks(vis._ctx, source, ctypes.byref(pairs), ctypes.byref(scales), ctypes.byref(n),
+                                     ctypes.byref(size)), vis._ctx, "get_bricks")
+    return pairs.value, scales.value
+
+
+def _enable(vis, slots):
+    """The sources' weights and thresholds with all but `slots` switched off."""
+    if not hasattr(vis, "all_on"):
+        vis.all_on = (list(vis.source_weight), list(vis.iso_threshold))
+    vis.source_weight = [w if i in slots else 0.0 for i, w in enumerate(vis.all_on[0])]
+    vis.iso_threshold = [t if i in slots else 0.0 for i, t in enumerate(vis.all_on[1])]
+
+
+def _read(vis, pointers, like):
+    vis.synchronize()
+    out = [np.empty_like(a) for a in like]
+    for a, p in zip(out, pointers):
+        vis._d2h(a, p)
+    return out
+
+
+@pytest.mark.parametrize("asked", [(0,), (1,), (0, 1)])
+def test_pointers_stay_while_sources_come_and_go(asked):
+    """Pointers taken while three sources lie in rows of their own are valid, and hold the
+    last update's bricks, when two of them share rows, when one is left and when all are on
+    again; nothing is asked for again in between."""
+    import torch
+
+    vis = _vis(count=3)
+    like = {i: vis.bricks(i) for i in asked}
+    held = {i: _pointers(vis, i) for i in asked}
+    grow = 1.0
+    for slots in ((0, 1), (0,), (0, 1), (1,), (0, 1, 2), (0, 1)):
+        _enable(vis, slots)
+        grow *= 0.75  # other contents each time
+        for s in (0, 1):
+            vis.volume_sources[s].tensor.mul_(0.75)
+        torch.cuda.synchronize()
+        vis.update_buffers()
+        vis.draw(out=False)
+        for i in asked:
+            if i not in slots:
+                continue
+            pairs, scales = _read(vis, held[i], like[i])
+            # a scale is the largest |value| of its brick and component; the pairs are quotients by
+            # it, at most 1, which the rounded products move by one step of binary16 at most
+            assert np.allclose(scales, like[i][1] * grow, rtol=1e-5), slots
+            assert np.abs(pairs.view(np.float16).astype(np.float32) - like[i][0].view(np.float16).astype(np.float32)).max() <= 2.0 ** -11
+    for i in asked:
+        assert _pointers(vis, i) == held[i]
+    vis.close()
