@@ -122,12 +122,15 @@ struct isaac_hip_ctx
     int form = ISAAC_HIP_FORM_COMBINED;
     int brickDtype = ISAAC_HIP_F32;
     int builtDtype = ISAAC_HIP_F32; // brickDtype at the last brick-form update_buffers: what frames read
-    // joint rows of two sources (common.hpp): jointDim components, 0 if the last
-    // update_buffers made none
+    // joint rows of two sources (common.hpp): jointDim components in jointBytes, 0 if the last
+    // update_buffers made none; the buffers hold jointCap components of jointBricks bricks.  They
+    // and the sources' own arrays stay while the other layout is in use (a source switched off
+    // and on again), at most twice the bricks' memory; given up where an allocation fails
     void* joint = nullptr;
     float* jointScale = nullptr;
-    size_t jointBytes = 0, jointScaleCount = 0;
-    int jointDim = 0;
+    size_t jointBytes = 0;
+    int64_t jointBricks = 0;
+    int jointDim = 0, jointCap = 0;
     int builtForm = -1; // form prepared by the last update_buffers
     bool floatOut = false;
     float4* outFloat = nullptr;

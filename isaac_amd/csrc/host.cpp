@@ -465,11 +465,37 @@ namespace
         (void) hipFree(c->jointScale);
         c->joint = nullptr;
         c->jointScale = nullptr;
-        c->jointBytes = c->jointScaleCount = 0;
+        c->jointBytes = 0;
+        c->jointBricks = 0;
+        c->jointCap = 0;
         c->generation++;
     }
 
-    int ensure_bricks(isaac_hip_ctx* c, VolSlot& v, int64_t nb, int dim, size_t pairBytes)
+    // What an array is allocated for, and so which arrays go where memory is short: those of the
+    // layout that the update does not build, except what get_bricks gave out
+    enum class BrickUse
+    {
+        Own,
+        Joint,
+        Copy // of joint rows in use: nothing goes
+    };
+
+    hipError_t brick_malloc(isaac_hip_ctx* c, void** p, size_t bytes, BrickUse use)
+    {
+        const hipError_t e = hipMalloc(p, bytes);
+        if(e != hipErrorOutOfMemory || use == BrickUse::Copy)
+            return e;
+        (void) hipGetLastError();
+        if(use == BrickUse::Own)
+            free_joint(c);
+        else
+            for(VolSlot& v : c->vols)
+                if(!v.ownWanted)
+                    free_bricks(v);
+        return hipMalloc(p, bytes);
+    }
+
+    int ensure_bricks(isaac_hip_ctx* c, VolSlot& v, int64_t nb, int dim, size_t pairBytes, BrickUse use)
     {
         const size_t bytes = size_t(nb) * size_t(dim) * size_t(kBrickPairs) * pairBytes;
         const size_t ns = size_t(nb) * size_t(dim);
@@ -478,8 +504,8 @@ namespace
         if(v.brick && v.brickBytes == bytes && v.scaleCount == ns)
             return 0;
         free_bricks(v);
-        HIPCHK(c, hipMalloc(&v.brick, std::max<size_t>(bytes, 8)));
-        HIPCHK(c, hipMalloc(&v.brickScale, std::max<size_t>(ns, 1) * 4));
+        HIPCHK(c, brick_malloc(c, &v.brick, std::max<size_t>(bytes, 8), use));
+        HIPCHK(c, brick_malloc(c, reinterpret_cast<void**>(&v.brickScale), std::max<size_t>(ns, 1) * 4, use));
         v.brickBytes = bytes;
         v.scaleCount = ns;
         return 0;
@@ -487,15 +513,18 @@ namespace
 
     int ensure_joint(isaac_hip_ctx* c, int dim)
     {
-        const size_t ns = size_t(brick_count(c)) * size_t(dim), bytes = ns * size_t(kBrickPairs) * 4;
-        if(c->joint && c->jointBytes == bytes && c->jointScaleCount == ns)
-            return 0;
-        free_joint(c);
-        c->generation++;
-        HIPCHK(c, hipMalloc(&c->joint, std::max<size_t>(bytes, 8)));
-        HIPCHK(c, hipMalloc(&c->jointScale, std::max<size_t>(ns, 1) * 4));
+        const int64_t nb = brick_count(c);
+        const size_t ns = size_t(nb) * size_t(dim), bytes = ns * size_t(kBrickPairs) * 4;
+        if(c->jointCap < dim || c->jointBricks != nb)
+        {
+            free_joint(c);
+            c->generation++;
+            HIPCHK(c, brick_malloc(c, &c->joint, std::max<size_t>(bytes, 8), BrickUse::Joint));
+            HIPCHK(c, brick_malloc(c, reinterpret_cast<void**>(&c->jointScale), std::max<size_t>(ns, 1) * 4, BrickUse::Joint));
+            c->jointBricks = nb;
+            c->jointCap = dim;
+        }
         c->jointBytes = bytes;
-        c->jointScaleCount = ns;
         return 0;
     }
 
@@ -503,7 +532,7 @@ namespace
     // context's local size and brick type may have changed since)
     int split_joint(isaac_hip_ctx* c, VolSlot& v)
     {
-        if(int rc = ensure_bricks(c, v, v.nbricks, v.brickDim, 4))
+        if(int rc = ensure_bricks(c, v, v.nbricks, v.brickDim, 4, BrickUse::Copy))
             return rc;
         HIPCHK(c, launch_brick_split(c->joint, c->jointScale, c->jointDim, v.jointAt, v.brickDim, v.nbricks, v.brick, v.brickScale,
                                      c->stream));
@@ -1513,8 +1542,8 @@ extern "C"
                     slots[i]->bricked = true;
                 }
             }
-            else
-                free_joint(c);
+            else if(c->brickDtype == ISAAC_HIP_F32)
+                free_joint(c); // (no combination of sources uses it)
             if(c->jointDim != wasJoint)
                 c->generation++;
             for(int i = 0; i < active; i++)
@@ -1523,17 +1552,18 @@ extern "C"
                 if(!joint)
                 {
                     const void* const was = v.brick;
-                    if(int rc = ensure_bricks(c, v, v.nbricks, v.brickDim, c->brickDtype == ISAAC_HIP_F32 ? 8 : 4))
+                    if(int rc = ensure_bricks(c, v, v.nbricks, v.brickDim, c->brickDtype == ISAAC_HIP_F32 ? 8 : 4, BrickUse::Own))
                         return rc;
                     if(v.brick != was)
                         c->generation++;
                     HIPCHK(c, launch_bricks(src + i, 1, X, Y, Z, c->brickDtype, v.brickScale, v.brick, c->stream));
                     v.bricked = v.ownBricks = true;
                 }
-                else if(!v.ownWanted)
-                    free_bricks(v);
-                else if(int rc = split_joint(c, v))
-                    return rc;
+                else if(v.ownWanted)
+                {
+                    if(int rc = split_joint(c, v))
+                        return rc;
+                }
             }
             // the particle records after the GPU-heavy brick build, so the host enqueues
             // their short launches while the build runs

@@ -169,3 +169,25 @@ def test_pointers_stay_while_sources_come_and_go(asked):
     for i in asked:
         assert _pointers(vis, i) == held[i]
     vis.close()
+
+
+def test_switching_a_source_on_and_off_allocates_nothing():
+    """Each layout keeps its arrays: once every combination was there, updates neither
+    allocate nor free, and the frames are those of the first time."""
+    import torch
+
+    vis = _vis(size=(64, 64, 64), count=3)
+    cycle = ((0, 1), (0,), (1,), (0, 2), (0, 1, 2))
+    frames, free = {}, set()
+    for turn in range(3):
+        for slots in cycle:
+            _enable(vis, slots)
+            vis.update_buffers()
+            img = vis.draw()
+            if turn == 0:
+                frames[slots] = img
+                continue
+            assert np.array_equal(img, frames[slots]), slots
+            free.add(torch.cuda.mem_get_info()[0])
+    assert len(free) == 1, free
+    vis.close()
