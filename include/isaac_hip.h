@@ -491,7 +491,11 @@ extern "C"
         const void** ao);
     /* device pointer of the combined textures (lib/isaac.hpp:646-647): one texel per
      * local voxel, x fastest; each texel is *texel_bytes (8) bytes: the combined volume
-     * RGBA8 followed by the combined iso RGBA8 */
+     * RGBA8 followed by the combined iso RGBA8.  The march reads the two as textures of their
+     * own: the first request allocates the side-by-side texels, fills them and waits for the
+     * stream; they follow every update from then on (one more pass of 16 bytes a voxel) and
+     * stay where they are until the local size changes.  Not to be called while another thread
+     * uses the context. */
     int isaac_hip_get_combined_textures(const isaac_hip_ctx* ctx, const void** texels, int32_t* texel_bytes);
     /* device pointers of field source field_idx's current advection texture (local
      * voxels, x fastest, one byte each) and of the noise texture (floats), and the

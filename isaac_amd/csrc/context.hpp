@@ -215,6 +215,7 @@ namespace isaac_hip
 
     inline int hip_fail(isaac_hip_ctx* c, hipError_t e, const char* what)
     {
+        (void) hipGetLastError(); // reported here: not to be found again behind the next launch
         return fail(c, ISAAC_HIP_ERR_DEVICE, std::string(what) + ": " + hipGetErrorString(e));
     }
 

@@ -351,6 +351,8 @@ namespace
         c->texVol = c->texIso = nullptr;
         c->texBoth = nullptr;
         c->isoCells = nullptr;
+        c->texVox = 0;
+        c->classified = false;
         c->generation++;
         // one allocation for both textures and the iso cells, each on a 256-byte boundary.  One
         // texel of padding: the march reads texels x and x+1 with one 8-byte load, also at the
@@ -370,7 +372,6 @@ namespace
             HIPCHK(c, hipMemsetAsync(c->texBoth, 0, nvox * sizeof(uint2), c->stream));
         }
         c->texVox = nvox;
-        c->classified = false;
         return 0;
     }
 
@@ -1577,6 +1578,8 @@ extern "C"
             return 0;
         }
         // classification (lib/isaac.hpp:1916-1947)
+        if(!c->texVox)
+            return fail(c, ISAAC_HIP_ERR_STATE, "no textures: the last change of the local size failed");
         ClassifyParams P{};
         P.X = int32_t(c->local[0]);
         P.Y = int32_t(c->local[1]);
@@ -1987,7 +1990,7 @@ extern "C"
             return 0;
         // built by the first request, and by every update after it
         isaac_hip_ctx* m = const_cast<isaac_hip_ctx*>(c);
-        if(!m->texBoth)
+        if(!m->texBoth && m->texVox) // (no textures after a change of the local size that failed)
         {
             HIPCHK(m, hipSetDevice(m->device));
             HIPCHK(m, hipMalloc(&m->texBoth, m->texVox * sizeof(uint2)));

@@ -93,3 +93,31 @@ def test_iso_cell_marks_do_not_outlive_their_update():
             assert np.array_equal(_counting_equal(vis), with_iso)
     assert not np.array_equal(_counting_equal(vis), with_iso)
     vis.close()
+
+
+def test_local_size_that_does_not_fit():
+    """A local size whose textures cannot be allocated: an error, then nothing to draw, classify
+    or ask for, until a size that fits."""
+    import ctypes
+
+    from isaac_amd import visualization as V
+    from isaac_amd._lib import IsaacHipError, lib
+
+    vis = V.from_scene(_spec((24, 20, 16)))
+    vis.update_buffers()
+    want = vis.draw()
+    vis.combined_textures()
+    with pytest.raises(IsaacHipError):
+        vis.update_local_size((1 << 20, 1 << 13, 1 << 12))  # 2^45 voxels: 256 TiB
+    for call in (vis.draw, vis.update_buffers):
+        with pytest.raises(IsaacHipError):
+            call()
+    ptr, size = ctypes.c_void_p(1), ctypes.c_int32()
+    assert lib().isaac_hip_get_combined_textures(vis._ctx, ctypes.byref(ptr), ctypes.byref(size)) == 0
+    assert not ptr.value and size.value == 8
+    vis.update_local_size((24, 20, 16))
+    vis.update_buffers()
+    assert np.array_equal(vis.draw(), want)
+    vol, iso = vis.combined_textures()
+    assert vol.any() and iso.any()
+    vis.close()
