@@ -56,6 +56,34 @@ def test_march_equals_counting_march(size, linear):
         vis.close()
 
 
+@pytest.mark.parametrize("linear", [True, False])
+@pytest.mark.parametrize("data", ["full", "noise", "dots", "slabs"])
+def test_rays_that_start_in_marked_cells(data, linear):
+    """Data with a surface everywhere: all above the threshold, noise about it, single voxels
+    above it 5 apart (marked throughout, hardly a hit), and slabs of 24 voxels above and below
+    it (rays start in one, two, three and more marked cells in a row)."""
+    from isaac_amd import visualization as V
+
+    X, Y, Z = 65, 50, 71
+    z, y, x = np.meshgrid(np.arange(Z), np.arange(Y), np.arange(X), indexing="ij")
+    dens = {"full": np.full((Z, Y, X), 0.9), "noise": np.random.default_rng(3).uniform(0.0, 1.0, (Z, Y, X)),
+            "dots": np.where((x % 5 == 2) & (y % 5 == 2) & (z % 5 == 2), 0.55, 0.0),
+            "slabs": np.where((x + y) // 24 % 2 == 0, 0.8, 0.1)}[data].astype(np.float32)
+    spec = _spec((X, Y, Z), linear, pose=scenes.FILL_POSE)
+    spec.volumes[0] = dataclasses.replace(spec.volumes[0], data=dens)
+    vis = V.from_scene(spec)
+    hits = 0
+    for step in (0.5, 2.5):
+        vis.step = step
+        for iso in (0.5, 0.05):
+            vis.iso_threshold = [iso]
+            vis.update_buffers()
+            _counting_equal(vis)
+            hits += int((vis.gbuffer()[1] < 3e38).sum())
+    assert hits > (0 if data == "dots" else 1000)  # (a trilinear sum about a single voxel hardly reaches the threshold)
+    vis.close()
+
+
 def test_iso_threshold_changed_between_updates():
     """A threshold set after a classification without one finds no surface until the next
     update, as the iso texels are 0 then; the texels a caller asked for follow every update."""
