@@ -53,6 +53,26 @@ def test_brick_march_equals_counting_march(size, sources):
     vis.close()
 
 
+@pytest.mark.parametrize("linear", [True, False])
+@pytest.mark.parametrize("dtype", ["F32", "F16", "BF16"])
+def test_three_sources_against_the_oracle(oracle_lib, dtype, linear):
+    """Three sources (no signature of their own: every one through the general fetch) at a size
+    that leaves partial bricks on each axis, within 2/255 of the oracle on 99.9 % of the pixels
+    (colours of 8 bits whose sums round in another order)."""
+    from isaac_amd import visualization as V
+    from oracle import oracle
+
+    spec = dataclasses.replace(_spec((17, 21, 30), ("density", "vector", "soft")), interpolation=linear)
+    vis = V.from_scene(spec)
+    vis.set_render_form(vis.FORM_BRICKS, getattr(vis, dtype))
+    vis.update_buffers()
+    img = vis.draw()
+    ora = oracle.render_post(spec, 32, getattr(vis, dtype))
+    assert (img[..., 3] > 0).mean() > 0.1
+    assert (np.abs(img.astype(np.int32) - ora.rgba.astype(np.int32)).max(axis=2) <= 2).mean() >= 0.999
+    vis.close()
+
+
 @pytest.mark.parametrize("fb", [(16, 16), (65, 63), (333, 201), (700, 30)])
 def test_batch_frames_of_any_size(fb):
     from isaac_amd import batch as B
