@@ -15,8 +15,10 @@ The timed frames record HIP events around the march only (its time for the
 roofline); the per-kernel breakdown comes from the same frames run just before
 with events between all kernels (ms_per_step_all_timing_events).
 
-Metric: trilinear samples per second (volume + iso march samples actually
-executed, after early ray termination), with frames/s alongside.  The same run
+Metric: trilinear samples per second (the volume + iso samples of the reference's
+march of these rays, after early ray termination, as the counting march takes them;
+the timed march leaves out iso samples in cells without a voxel above the threshold:
+volume_samples_per_s has the samples it takes all of), with frames/s alongside.  The same run
 also times the brick render forms (FP32 / FP16 / BF16 field bricks,
 post-classification) on the same workload and reports them under "forms".
 """
@@ -68,10 +70,11 @@ def kernel_bytes(counts, spec, n_vox, n_particles, n_visible, form="combined"):
     if form == "combined":
         # 16 B of sources in, two RGBA8 texels out per voxel
         out["classify"] = n_vox * (src_bytes + 8)
-        # fused march: 8 RGBA8 taps per volume sample and per iso sample, 7 iso samples at a hit;
-        # G-buffer writes colour 4 + normal 12 + depth 4 + volume colour 16
-        out["march"] = (32 * (counts["vol_samples"] + counts["iso_samples"]) + 7 * 32 * counts["iso_hits"]
-                        + particles + 36 * npx)
+        # fused march: 8 RGBA8 taps per volume sample, 7 iso samples at a hit; G-buffer writes colour 4
+        # + normal 12 + depth 4 + volume colour 16.  The iso samples of the counting march (one a step)
+        # are not taken by the timed one except between the iso cells that its rays meet, which nothing
+        # counts: they are left out, so this is what the march moves at least
+        out["march"] = 32 * counts["vol_samples"] + 7 * 32 * counts["iso_hits"] + particles + 36 * npx
     else:
         vb = VALUE_BYTES[FORMS[form][1]]
         # brick build: sources in; 648 pairs of 2 values per 512 voxels and component out, + scales
@@ -506,13 +509,8 @@ def main() -> int:
     ap.add_argument("--form-steps", type=int, default=10)
     ap.add_argument("--no-cpu-baseline", action="store_true")
     ap.add_argument("--cpu-threads", type=int, default=0)
-    ap.add_argument("--prefetch", type=int, default=0, help="march kernel: fetch step i+1 before compositing step i")
-    ap.add_argument("--march-waves", type=int, default=0, help="march occupancy target (0, 6, 8)")
-    ap.add_argument("--march-threads", type=int, default=256, help="march workgroup: 256 (4 waves) or 64 (one wave)")
-    ap.add_argument("--tex-layout", type=int, default=0,
-                    help="texture the march reads: 0 linear, 8 bricks of 8^3, 16 binary16 copy of the volume RGBA")
-    ap.add_argument("--no-tune", action="store_true",
-                    help="keep --prefetch / --march-waves / --march-threads instead of autotuning")
+    ap.add_argument("--march-threads", type=int, default=64, help="march workgroup: 64 (one wave) or 256 (4 waves)")
+    ap.add_argument("--no-tune", action="store_true", help="keep --march-threads instead of autotuning")
     ap.add_argument("--no-learned-ao", action="store_true", help="skip training / timing the learned occlusion pass")
     ap.add_argument("--ao-train-steps", type=int, default=1250, help="16 crops each: 20,000 triples")
     ap.add_argument("--no-batch", action="store_true", help="skip the batched sub-volumes x views workload")
@@ -550,15 +548,12 @@ def main() -> int:
     spec = scenes.prod_scene(n=n)
     poses = [scenes.DEFAULT_POSE, scenes.FILL_POSE]
     vis = V.from_scene(spec, 0)
-    vis.set_tuning(vis.TUNE_MARCH_PREFETCH, args.prefetch)
     out = torch.empty((spec.framebuffer[1], spec.framebuffer[0], 4), dtype=torch.uint8, device="cuda")
     n_vox = n ** 3
     n_particles = int(spec.particles[0].pos.shape[0])
     n_visible = int(np.count_nonzero(spec.particles[0].attr[:, 0] >= 0.995))
 
-    vis.set_tuning(vis.TUNE_MARCH_WAVES, args.march_waves)
     vis.set_tuning(vis.TUNE_MARCH_THREADS, args.march_threads)
-    vis.set_tuning(vis.TUNE_TEX_LAYOUT, args.tex_layout)
     form, dt = FORMS[args.form]
     vis.set_render_form(form, dt)
     tuning = None
@@ -608,6 +603,7 @@ def main() -> int:
             "form": args.form,
         },
         "fps": args.steps / wall,
+        "volume_samples_per_s": avg_counts["vol_samples"] * args.steps / wall,
         "fps_host_output": args.steps / wall_h,
         "ms_per_step_host_output": wall_h / args.steps * 1e3,
         # the same frames with timing events between all kernels (per-kernel breakdown below)
