@@ -107,19 +107,25 @@ def test_iso_threshold_changed_between_updates():
     vis.close()
 
 
-def test_iso_cell_marks_do_not_outlive_their_update():
-    """300 updates (the marks' numbers wrap at 255), a surface in every 70th."""
+def test_surfaces_around_the_wrap_of_the_marks():
+    """The marks of the iso cells carry their update's number, 1..255 in turn, and are cleared
+    when it wraps: the surface of every update about two wraps, another one each time, is
+    the counting march's, which does not read the marks.  (A mark that outlived its update would
+    only have steps tested in vain; a lost one would lose the surface.)"""
     from isaac_amd import visualization as V
 
     vis = V.from_scene(dataclasses.replace(_spec((24, 20, 16)), clipping=[]))
-    vis.update_buffers()
-    with_iso = vis.draw()
-    for k in range(300):
-        vis.iso_threshold = [0.4 if k % 70 == 69 else 0.0]
+    plain, frames = None, []
+    for k in range(1, 516):  # update k has number (k - 1) % 255 + 1
+        near = min(k % 255, 255 - k % 255) <= 4
+        vis.iso_threshold = [(0.4, 0.2, 0.6)[k % 3] if near else 0.0]
         vis.update_buffers()
-        if k % 70 == 69:
-            assert np.array_equal(_counting_equal(vis), with_iso)
-    assert not np.array_equal(_counting_equal(vis), with_iso)
+        if near:
+            frames.append(_counting_equal(vis))
+        elif plain is None:
+            plain = vis.draw()
+    assert len(frames) > 20 and all(not np.array_equal(f, plain) for f in frames)
+    assert np.array_equal(frames[-1], frames[-4]) and not np.array_equal(frames[-1], frames[-2])
     vis.close()
 
 
