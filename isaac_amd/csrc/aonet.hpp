@@ -45,7 +45,7 @@ namespace isaac_hip
     // network's (cin, cout, ca) shapes: (8,16,0) (16,16,0) (16,32,0) (32,32,0)
     // (32,64,0) (64,64,0) (128,64,64) (96,32,64) (48,16,32); weights [cout][kp] with
     // kp = 9*cin rounded up to a multiple of 32 (zero columns).  The fused pool and
-    // head outputs equal launch_pool2 / launch_head_infer applied to the activation.
+    // head outputs are formed from the activation as it is stored (binary16).
     hipError_t launch_conv_fwd(const ConvArgs& a, int cout, size_t max_lds, hipStream_t s);
 
     // Where the gradient of a layer's output comes from

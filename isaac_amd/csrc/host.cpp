@@ -1527,7 +1527,9 @@ extern "C"
             }
             const int X = int(c->local[0]), Y = int(c->local[1]), Z = int(c->local[2]);
             // joint rows: 2 or 4 words, so that a row is one aligned load, and < 4 GiB, so that
-            // the march's 32-bit offsets reach them
+            // the march's 32-bit offsets reach them.  March of 128^3 in FP16 at 960x540, joint against
+            // rows of their own, trilinear / nearest: 1 + 3 components 388 / 527 against 421 / 545 us,
+            // 3 + 1 387 / 523 against 417 / 539, 1 + 1 294 / 465 against 341 / 482
             const int dims = active == 2 ? src[0].dim + src[1].dim : 0;
             const bool joint = c->brickDtype != ISAAC_HIP_F32 && (dims == 2 || (dims == 4 && src[0].dim != 2))
                 && uint64_t(brick_count(c)) * kBrickPairs * uint64_t(dims) * 4 <= 0xffffffffull;

@@ -132,9 +132,8 @@ namespace isaac_hip
     };
 
     // ------------------------------------------------------------------ pixel tiling
-    // workgroup -> 16x16 tile, XCD-banded; returns false for threads outside the viewport
-    // pixel of this thread in 16x16 tile `b` of the viewport (row-major tiles)
-    // pixel of this lane in 16x16 tile b, whose 8x8 quarter `wave` (0..3) its wave renders
+    // pixel of this lane in 16x16 tile b of the viewport (row-major tiles), whose 8x8 quarter
+    // `wave` (0..3) its wave renders; false outside the viewport
     __device__ inline bool tile_pixel_at(const FrameParams& F, uint32_t b, uint32_t wave, int& px, int& py)
     {
         const uint32_t tx = b % uint32_t(F.tilesX), ty = b / uint32_t(F.tilesX);
@@ -197,11 +196,6 @@ namespace isaac_hip
     {
         const uint32_t b = march_block(F);
         return F.tileOrder != 0 ? supertile_tile(F, b) : xcd_tile(F, b);
-    }
-
-    __device__ inline bool tile_pixel(const FrameParams& F, int& px, int& py)
-    {
-        return tile_pixel_at(F, xcd_tile(F, blockIdx.x), px, py);
     }
 
     __device__ inline void block_count_add(unsigned long long* dst, unsigned long long v)
