@@ -314,18 +314,22 @@ namespace isaac_hip
     // A ray that starts in kIsoLead marked cells in a row is in data whose surface is everywhere
     // (noise about the threshold, a box opaque from its face on), and has most likely met it before
     // the walk would end: it is not walked on, every step is tested.  Measured on MI355X at 960x540,
-    // march of 192^3 voxels all above the threshold, trilinear / nearest: 40 / 38 us walked to the end,
-    // 25 / 20 us this way (the test at every step that the walk replaced: 24 / 17.5); uniform noise about
-    // the threshold 110 / 57 -> 106 / 37 (107 / 36).  Stopping at any marked cells in a row, not only at
-    // the ray's start, tests the steps of rays along a surface too: 256^3 production frame 370 -> 423 us.
-    constexpr int kIsoLead = 3;
+    // march of 192^3 voxels all above the threshold, trilinear / nearest: 38 / 36 us walked to the end,
+    // 31 / 27 us this way (the test at every step that the walk replaced: 24 / 17); uniform noise about
+    // the threshold, nearest: 53 -> 44 us (36).  Fewer cells gain more there (8: 28 / 23 and 41 us, 3: 25 / 20
+    // and 38 us), but rays that run along a surface from a clipping plane start in as many: of eleven 256^3
+    // production frames one goes from 604 to 657 us with 8, others from 3 on, none with 12 or 16; anywhere
+    // along the ray 4 in a row take all of them from 610 to 659 us.  The count is kept where a cell is
+    // marked only: every instruction on the path of the others, or a loop of its own for the first
+    // cells, costs frames with a surface 1-3 %.
+    constexpr int kIsoLead = 16;
     __device__ inline void iso_steps(const FrameParams& F, const StepLine& L, int first, int last, int& from, int& to)
     {
         const F3 inv = f3(1.0f / L.v.x, 1.0f / L.v.y, 1.0f / L.v.z);
         const float lastF = float(last);
         from = 0x7fffffff;
-        to = -0x7fffffff;
-        int lead = 0; // marked cells in a row from the ray's start
+        to = first - 1;
+        int lead = 0; // marked cells in a row from the ray's start (below 0 behind a gap)
         for(float k = float(first); k <= lastF;)
         {
             const F3 p = L.at(k);
@@ -344,19 +348,16 @@ namespace isaac_hip
             };
             const float t = fminf(fminf(exit(cx, L.c.x, L.v.x, inv.x, F.X), exit(cy, L.c.y, L.v.y, inv.y, F.Y)),
                                   exit(cz, L.c.z, L.v.z, inv.z, F.Z));
-            const float end = floorf(fmaxf(fminf(t, lastF), k));
+            float end = floorf(fmaxf(fminf(t, lastF), k));
             if(mark == F.isoEpoch)
             {
-                from = min(from, int(k));
-                to = int(end);
-                if(++lead == kIsoLead)
-                {
-                    to = last;
-                    break;
-                }
+                const int start = int(k);
+                lead = start == to + 1 ? lead + 1 : -0x40000000;
+                if(lead == kIsoLead)
+                    end = lastF;
+                from = min(from, start);
+                to = int(end); // (last where end is lastF: both are below 2^23)
             }
-            else
-                lead = -0x40000000;
             k = end + 1.0f;
         }
     }
@@ -511,11 +512,11 @@ namespace isaac_hip
                                     nSteps++;
                                 const Place pl = place(i);
                                 const Weights W = corner_weights(pl.fx, pl.fy, pl.fz);
-                                // both textures' texels are requested before the first is looked at (nearest
-                                // march of 181x127x203 voxels at 1283x719 181 -> 168 us, without the request ahead that
-                                // the interior steps have)
+                                // (nearest, which has no request ahead: both textures' texels are requested before the
+                                // first is looked at, march of 181x127x203 voxels at 1283x719 176 -> 168 us; the trilinear
+                                // march, whose interior steps have one, holds 8 more VGPRs for nothing)
                                 uint32_t tv[8];
-                                if(i <= volEnd)
+                                if(!LINEAR && i <= volEnd)
                                     fetch_place<LINEAR, OFF32>(F.vol, pl, tv);
                                 if(i >= isoFrom && i <= isoEnd)
                                 {
@@ -527,6 +528,8 @@ namespace isaac_hip
                                 {
                                     if(COUNT)
                                         nVol++;
+                                    if(LINEAR)
+                                        fetch_place<LINEAR, OFF32>(F.vol, pl, tv);
                                     composite(acc, vol_sums<LINEAR>(tv, W), vscale);
                                     if(acc.a > 0.99f)
                                         volEnd = off;
@@ -686,7 +689,7 @@ namespace isaac_hip
 
     // Workgroups of one wave by default (march_block), which any SIMD with a free slot takes: with
     // four waves a workgroup waits for four slots of one CU while its rays' lengths differ.  At
-    // 96 VGPRs (5 waves per SIMD); held to 80 or 64 registers for 6 or 8 waves it spills and is slower.
+    // 88 VGPRs (5 waves per SIMD); held to 80 or 64 registers for 6 or 8 waves it spills and is slower.
     // Measured on MI355X, before (8-byte texels with both textures, byte conversions, an iso sum test
     // every step, four-wave workgroups) and after: 256^3 with iso-surface and 2 M particles at
     // 1920x1080 530 -> 365 us (volume in the middle of the frame) and 866 -> 735 us (filling it);

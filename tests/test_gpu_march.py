@@ -61,10 +61,10 @@ def test_march_equals_counting_march(size, linear):
 def test_rays_that_start_in_marked_cells(data, linear):
     """Data with a surface everywhere: all above the threshold, noise about it, single voxels
     above it 5 apart (marked throughout, hardly a hit), and slabs of 24 voxels above and below
-    it (rays start in one, two, three and more marked cells in a row)."""
+    it (rays start in fewer marked cells in a row), along a box of 16 iso cells and more."""
     from isaac_amd import visualization as V
 
-    X, Y, Z = 65, 50, 71
+    X, Y, Z = 150, 52, 141
     z, y, x = np.meshgrid(np.arange(Z), np.arange(Y), np.arange(X), indexing="ij")
     dens = {"full": np.full((Z, Y, X), 0.9), "noise": np.random.default_rng(3).uniform(0.0, 1.0, (Z, Y, X)),
             "dots": np.where((x % 5 == 2) & (y % 5 == 2) & (z % 5 == 2), 0.55, 0.0),
