@@ -311,18 +311,19 @@ namespace isaac_hip
     // the march, when all lanes of a wave walk together: lanes leave cells at different steps, so a
     // walk from cell to cell inside the march would make each lane wait for all the others' walks.
     //
-    // A ray that starts in kIsoLead marked cells in a row is in data whose surface is everywhere
+    // A ray that starts in LEAD marked cells in a row is in data whose surface is everywhere
     // (noise about the threshold, a box opaque from its face on), and has most likely met it before
     // the walk would end: it is not walked on, every step is tested.  Measured on MI355X at 960x540,
     // march of 192^3 voxels all above the threshold, trilinear / nearest: 38 / 36 us walked to the end,
-    // 31 / 27 us this way (the test at every step that the walk replaced: 24 / 17); uniform noise about
-    // the threshold, nearest: 53 -> 44 us (36).  Fewer cells gain more there (8: 28 / 23 and 41 us, 3: 25 / 20
-    // and 38 us), but rays that run along a surface from a clipping plane start in as many: of eleven 256^3
-    // production frames one goes from 604 to 657 us with 8, others from 3 on, none with 12 or 16; anywhere
-    // along the ray 4 in a row take all of them from 610 to 659 us.  The count is kept where a cell is
-    // marked only: every instruction on the path of the others, or a loop of its own for the first
-    // cells, costs frames with a surface 1-3 %.
-    constexpr int kIsoLead = 16;
+    // 31 / 20 us with 16 and 3 cells (the test at every step that the walk replaced: 24 / 17); uniform noise
+    // about the threshold 112 / 53 -> 108 / 38 us (101 / 36).  Fewer cells would gain the trilinear march
+    // more there (8: 28 us, 3: 25 us), but rays that run along a surface from a clipping plane start in as
+    // many and test in vain: of eleven 256^3 production frames one goes from 604 to 657 us with 8, others
+    // from 3 on, none with 12 or 16; anywhere along the ray 4 in a row take all of them from 610 to
+    // 659 us.  A test of the nearest march is one load beside another, and takes its frames from 620 to
+    // 622 us at most.  The count is kept where a cell is marked only: every instruction on the path of the
+    // others, or a loop of its own for the first cells, costs frames with a surface 1-3 %.
+    template<int LEAD>
     __device__ inline void iso_steps(const FrameParams& F, const StepLine& L, int first, int last, int& from, int& to)
     {
         const F3 inv = f3(1.0f / L.v.x, 1.0f / L.v.y, 1.0f / L.v.z);
@@ -353,7 +354,7 @@ namespace isaac_hip
             {
                 const int start = int(k);
                 lead = start == to + 1 ? lead + 1 : -0x40000000;
-                if(lead == kIsoLead)
+                if(lead == LEAD)
                     end = lastF;
                 from = min(from, start);
                 to = int(end); // (last where end is lastF: both are below 2^23)
@@ -438,7 +439,7 @@ namespace isaac_hip
                                 isoEnd = endIso;
                             }
                             else
-                                iso_steps(F, L, startSteps, endIso, isoFrom, isoEnd);
+                                iso_steps<LINEAR ? 16 : 3>(F, L, startSteps, endIso, isoFrom, isoEnd);
                         }
                         float oldValue = 0.0f; // (0 before the first step)
                         int oldStep = startSteps - 1;
