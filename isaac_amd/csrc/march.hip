@@ -691,12 +691,13 @@ namespace isaac_hip
     // Workgroups of one wave by default (march_block), which any SIMD with a free slot takes: with
     // four waves a workgroup waits for four slots of one CU while its rays' lengths differ.  At
     // 88 VGPRs (5 waves per SIMD); held to 80 or 64 registers for 6 or 8 waves it spills and is slower.
-    // Measured on MI355X, before (8-byte texels with both textures, byte conversions, an iso sum test
-    // every step, four-wave workgroups) and after: 256^3 with iso-surface and 2 M particles at
-    // 1920x1080 530 -> 365 us (volume in the middle of the frame) and 866 -> 735 us (filling it);
-    // 512^3 at 3840x2160 and step 0.25 4900 -> 3740 us, 436 G samples/s, 354 cycles of a SIMD per
-    // 64 samples of which about 305 issue VALU instructions; 64^3 at 512x512 82 -> 58 us.  Four-wave
-    // workgroups: 370, 805, 3735 and 58 us.  Without the request ahead: 416, 733, 3990 and 73 us.
+    // Measured on MI355X (events around it), before (8-byte texels with both textures, byte conversions,
+    // an iso sum test every step, four-wave workgroups) and after: 256^3 with iso-surface and 2 M particles
+    // at 1920x1080 514 -> 370 us (volume in the middle of the frame) and 810 -> 730 us (filling it, 176 G
+    // samples/s: the waves wait for gathers and the last ones run alone); 512^3 at 3840x2160 and step 0.25
+    // 4730 -> 3700 us, 439 G samples/s, 354 cycles of a SIMD per 64 samples of which about 305 issue VALU
+    // instructions; 64^3 at 512x512 82 -> 58 us.  Four-wave workgroups: 370, 805, 3735 and 58 us.  Without the
+    // request ahead: 416, 733, 3990 and 73 us.
     template<bool LINEAR, bool COUNT, bool OFF32>
     __global__ __launch_bounds__(256) void march_kernel(const FrameParams F, const ParticleParams PP)
     {
