@@ -695,7 +695,7 @@ namespace isaac_hip
     // an iso sum test every step, four-wave workgroups) and after: 256^3 with iso-surface and 2 M particles
     // at 1920x1080 514 -> 370 us (volume in the middle of the frame) and 810 -> 730 us (filling it, 176 G
     // samples/s: the waves wait for gathers and the last ones run alone); 512^3 at 3840x2160 and step 0.25
-    // 4730 -> 3700 us, 439 G samples/s, 354 cycles of a SIMD per 64 samples of which about 305 issue VALU
+    // 4730 -> 3720 us, 436 G samples/s, 354 cycles of a SIMD per 64 samples of which about 305 issue VALU
     // instructions; 64^3 at 512x512 82 -> 58 us.  Four-wave workgroups: 370, 805, 3735 and 58 us.  Without the
     // request ahead: 416, 733, 3990 and 73 us.
     template<bool LINEAR, bool COUNT, bool OFF32>
