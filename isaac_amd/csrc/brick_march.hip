@@ -773,20 +773,21 @@ namespace isaac_hip
         }
         if(COUNT)
         {
-            block_count_add(F.counters + 0, nVol);
-            block_count_add(F.counters + 1, nIso);
-            block_count_add(F.counters + 2, nIsoHits);
-            block_count_add(F.counters + 3, nCells);
-            block_count_add(F.counters + 4, nTests);
-            block_count_add(F.counters + 5, nVolRays);
-            block_count_add(F.counters + 6, nIsoRays);
-            block_count_add(F.counters + 7, nPartRays);
-            block_count_add(F.counters + 8, nSteps);
+            unsigned long long* const cnt = F.counters + blockIdx.x % kCounterSets * kCounterStride;
+            block_count_add(cnt + 0, nVol);
+            block_count_add(cnt + 1, nIso);
+            block_count_add(cnt + 2, nIsoHits);
+            block_count_add(cnt + 3, nCells);
+            block_count_add(cnt + 4, nTests);
+            block_count_add(cnt + 5, nVolRays);
+            block_count_add(cnt + 6, nIsoRays);
+            block_count_add(cnt + 7, nPartRays);
+            block_count_add(cnt + 8, nSteps);
             // the wave runs the traversal loop as long as its longest lane
             int wm = int(nSteps);
             for(int off = 32; off > 0; off >>= 1)
                 wm = max(wm, __shfl_xor(wm, off, 64));
-            block_count_add(F.counters + 9, (threadIdx.x & 63u) == 0 ? (unsigned long long) wm : 0ull);
+            block_count_add(cnt + 9, (threadIdx.x & 63u) == 0 ? (unsigned long long) wm : 0ull);
         }
     }
 

@@ -128,8 +128,11 @@ namespace isaac_hip
         float* ao;
         float4* volColor; // premultiplied volume colour per pixel; w < 0: the volume pass did not blend
         float4* outFloat; // optional: final colour before RGBA8 quantisation (precision studies)
-        unsigned long long* counters;
+        unsigned long long* counters; // kCounterSets sets of kCounterStride, added up when they are read
     };
+    // Workgroup b of a counting march adds to set b % kCounterSets: on one set the adds of all workgroups
+    // meet in ten addresses (128^3 at 960x540 with one-wave workgroups, nearest: 338 us a frame)
+    constexpr uint32_t kCounterSets = 64, kCounterStride = 16;
 
     // ------------------------------------------------------------------ precision form (field bricks)
     // A source re-laid into 8^3 bricks with a one-voxel apron on the + side, stored

@@ -1018,7 +1018,7 @@ extern "C"
            || (e = hipMalloc(&c->color, npx * 4)) != hipSuccess || (e = hipMalloc(&c->depth, npx * 4)) != hipSuccess
            || (e = hipMalloc(&c->normal, npx * 12)) != hipSuccess || (e = hipMalloc(&c->ao, npx * 4)) != hipSuccess
            || (e = hipMalloc(&c->volColor, npx * 16)) != hipSuccess
-           || (e = hipMalloc(&c->counters, 64 * sizeof(unsigned long long))) != hipSuccess)
+           || (e = hipMalloc(&c->counters, kCounterSets * kCounterStride * sizeof(unsigned long long))) != hipSuccess)
         {
             isaac_hip_destroy(c);
             return ISAAC_HIP_ERR_ALLOC;
@@ -1027,7 +1027,7 @@ extern "C"
         (void) hipMemsetAsync(c->depth, 0, npx * 4, c->stream);
         (void) hipMemsetAsync(c->normal, 0, npx * 12, c->stream);
         (void) hipMemsetAsync(c->ao, 0, npx * 4, c->stream);
-        (void) hipMemsetAsync(c->counters, 0, 64 * sizeof(unsigned long long), c->stream);
+        (void) hipMemsetAsync(c->counters, 0, kCounterSets * kCounterStride * sizeof(unsigned long long), c->stream);
         rc = alloc_textures(c);
         if(rc != 0)
         {
@@ -1711,7 +1711,7 @@ extern "C"
                 return rc;
         }
         if(c->counting)
-            HIPCHK(c, launch_fill_u32(reinterpret_cast<uint32_t*>(c->counters), 0u, 2 * ISAAC_HIP_CNT_COUNT, c->stream));
+            HIPCHK(c, launch_fill_u32(reinterpret_cast<uint32_t*>(c->counters), 0u, 2 * kCounterSets * kCounterStride, c->stream));
         HIPCHK(c, mark(c, 4));
         if(c->form == ISAAC_HIP_FORM_BRICKS)
             HIPCHK(c, launch_brick_march(F, Q, PP, c->counting, c->stream));
@@ -1959,11 +1959,16 @@ extern "C"
     {
         if(!c || !out)
             return ISAAC_HIP_ERR_ARG;
-        unsigned long long h[16];
+        static_assert(ISAAC_HIP_CNT_COUNT <= kCounterStride, "counters of a set");
+        unsigned long long h[kCounterSets * kCounterStride];
         HIPCHK(c, hipMemcpyAsync(h, c->counters, sizeof(h), hipMemcpyDeviceToHost, c->stream));
         HIPCHK(c, hipStreamSynchronize(c->stream));
         for(int i = 0; i < ISAAC_HIP_CNT_COUNT; i++)
-            out[i] = h[i];
+        {
+            out[i] = 0;
+            for(uint32_t s = 0; s < kCounterSets; s++)
+                out[i] += h[s * kCounterStride + uint32_t(i)];
+        }
         return 0;
     }
 
